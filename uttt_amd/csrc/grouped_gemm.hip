@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "gemm_pipe.h"
+#include "tile192_host.h"
 
 namespace uttt {
 namespace {
@@ -2084,6 +2085,8 @@ extern "C" size_t uttt_grouped_wgrad_pair_workspace_bytes(int B, int E, int I, i
   if (B <= 0 || E <= 0 || I <= 0 || D <= 0 || N <= 0) return 0;
   const WgTask t0 = wg_task(nullptr, nullptr, nullptr, 2 * I, D);
   const WgTask t1 = wg_task(nullptr, nullptr, nullptr, D, I);
+  const Wg192Plan pl = wg192_plan(B, E, I, D, N);
+  if (pl.use) return pl.bytes;
   size_t off1;
   return wg_part_bytes(t0, t1, B, E, wg_splits(t0, t1, B, E, N), &off1);
 }
@@ -2103,6 +2106,14 @@ extern "C" int uttt_grouped_wgrad_pair(const void* dy0_dy2_tok, const void* k,
                    aligned16(dw0_w2) && aligned16(dw1),
                "grouped_wgrad_pair: tensors must be 16-byte aligned");
   // dW0_W2 [2I][D] = DY^T K;  dW1 [D][I] = V^T Hid
+  const Wg192Plan pl = wg192_plan(B, E, I, D, N);
+  if (pl.use) {
+    UTTT_REQUIRE(pl.bytes == 0 || (workspace && workspace_bytes >= pl.bytes && aligned16(workspace)),
+                 "grouped_wgrad_pair: workspace of %zu bytes needed (got %zu)", pl.bytes,
+                 workspace_bytes);
+    return launch_wg192(pl, dy0_dy2_tok, k, hidden_tok, v, dw0_w2, dw1, group_sizes, B, E, I, D, N,
+                        workspace, as_stream(stream), "grouped_wgrad_pair");
+  }
   const WgTask t0 = wg_task(k, dy0_dy2_tok, dw0_w2, 2 * I, D);
   const WgTask t1 = wg_task(hidden_tok, v, dw1, D, I);
   return launch_wg(t0, t1, group_sizes, B, E, N, wg_splits(t0, t1, B, E, N), workspace,
@@ -2333,6 +2344,10 @@ extern "C" int uttt_grouped_update_bwd(
                                    "grouped_update_bwd(grad_V)"))
     return rc;
   // 7. grad_W0_W2 [2I][D] = grad_x0_x2^T K;  grad_W1 [D][I] = V^T grad_dh
+  const Wg192Plan pl = wg192_plan(B, E, I, D, N);
+  if (pl.use && pl.bytes <= ws.gx)  // the partials over dhg, gy and dx, which nothing reads any more
+    return launch_wg192(pl, gx, k, gdh, v, grad_w0_w2, grad_w1, group_sizes, B, E, I, D, N, wsb, st,
+                        "grouped_update_bwd(weights)");
   const WgTask t0 = wg_task(k, gx, grad_w0_w2, 2 * I, D);
   const WgTask t1 = wg_task(gdh, v, grad_w1, D, I);
   return launch_wg(t0, t1, group_sizes, B, E, N, 1, nullptr, 0, st, "grouped_update_bwd(weights)");

@@ -1,0 +1,242 @@
+// Products of narrow matrices on 192 x 192 tiles (tile192.h): the weight
+// gradients of small experts, their token segments cut into chunks.  Called
+// through the C entries of grouped_gemm.hip, which choose between these and
+// the 256 x 256 tiles.
+#include <algorithm>
+
+#include "tile192.h"
+#include "tile192_host.h"
+
+namespace uttt {
+namespace {
+
+using namespace pipe;
+using namespace t192;
+
+__device__ __forceinline__ void store8_bf16(uint16_t* p, const float (&v)[8]) {
+  uint4 u;
+  u.x = pack_bf16x2(v[0], v[1]);
+  u.y = pack_bf16x2(v[2], v[3]);
+  u.z = pack_bf16x2(v[4], v[5]);
+  u.w = pack_bf16x2(v[6], v[7]);
+  *reinterpret_cast<uint4*>(p) = u;
+}
+
+// ======================================================= weight gradients ==
+// out[b, e][x][y] = sum_{n in seg(b, e)} P[n, y] Q[n, x] (two tasks per
+// launch), the segment of every expert cut into chunks of `chunk` tokens: one
+// workgroup per (chunk, output tile).  An expert with one chunk (an empty one
+// has one of no tokens: zeros) stores its bf16 output; the chunks of a longer
+// one store fp32 partials, part[b * parts_ub + index among the batch's partial
+// chunks], which wg192_reduce_kernel adds in chunk order (the result does not
+// depend on scheduling).  An expert with several chunks has more than `chunk`
+// tokens, so a batch has at most 2 N / chunk partial chunks.
+//
+// Bound by the token rows' stream from memory: 48 experts of 192 x 192 over
+// 196 608 tokens read 377 MB in 98 us (+ 6 us of reduction), against 285-459 us
+// (routing from even to skewed) for one 256 x 256-tile workgroup per output
+// tile, where 144 workgroups run and the longest expert sets the time; 96
+// experts of 384 x 384 over 16 384 tokens 42 us against 70.
+struct Wg192Task {
+  const uint16_t* p;
+  const uint16_t* q;
+  uint16_t* out;
+  int X, Y;
+  int y_tiles, x_tiles;
+};
+
+struct Wg192Args {
+  Wg192Task t[2];
+  const int32_t* gs;
+  float* part;       // [B * parts_ub][n_out] fp32
+  int64_t n_out;     // elements of both outputs of one expert
+  int B, E, N, chunk;
+  int slots, parts_ub;  // upper bounds of one batch's chunks and partial chunks
+};
+
+// Chunk `slot` of a batch: its expert, first token, tokens, and its index
+// among the partial chunks (-1: the expert's only chunk).
+struct ChunkPos {
+  int e, start, size, part;
+};
+
+// The chunks of a segment of g tokens, and those that store partials.
+__device__ __forceinline__ int chunks_of(int g, int chunk) { return max(1, (g + chunk - 1) / chunk); }
+__device__ __forceinline__ int partials_of(int nt) { return nt > 1 ? nt : 0; }
+
+__device__ ChunkPos find_chunk(const int32_t* __restrict__ gs_b, int E, int N, int chunk,
+                               int slot) {
+  const int lane = threadIdx.x & 63;
+  int tok_base = 0, base = 0, pbase = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane;
+    const int graw = e < E ? gs_b[e] : 0;
+    const int g = graw > 0 ? graw : 0;
+    const int tok_incl = wave_incl_scan(g);
+    const int start = min(tok_base + tok_incl - g, N);
+    const int gc = min(g, N - start);
+    const int nt = e < E ? chunks_of(gc, chunk) : 0;
+    const int incl = wave_incl_scan(nt);
+    const int excl = base + incl - nt;
+    const int pincl = wave_incl_scan(partials_of(nt));
+    const uint64_t bal = __ballot(slot >= excl && slot < excl + nt);
+    if (bal != 0ull) {
+      const int src = __ffsll((unsigned long long)bal) - 1;
+      const int i = slot - lane_value(excl, src);
+      const int size = lane_value(gc, src) - i * chunk;
+      const int parts = lane_value(nt, src);
+      return ChunkPos{__builtin_amdgcn_readfirstlane(e0 + src), lane_value(start, src) + i * chunk,
+                      min(size, chunk),
+                      parts > 1 ? pbase + lane_value(pincl, src) - parts + i : -1};
+    }
+    tok_base += lane_value(tok_incl, 63);
+    base += lane_value(incl, 63);
+    pbase += lane_value(pincl, 63);
+  }
+  return ChunkPos{-1, 0, 0, -1};
+}
+
+__global__ __launch_bounds__(kTThreads, 2) void wg192_kernel(Wg192Args a) {
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kTRing * kTStage];
+  const int n0 = a.t[0].y_tiles * a.t[0].x_tiles;
+  const int per = n0 + a.t[1].y_tiles * a.t[1].x_tiles;
+  // the tiles of one chunk run on one XCD: they read the same token rows
+  const int loc = blockIdx.x / kXcds;
+  const int unit = loc / per * kXcds + blockIdx.x % kXcds;
+  const int t = loc % per;
+  if (unit >= a.B * a.slots) return;
+  const int b = unit / a.slots;
+  const ChunkPos cp = find_chunk(a.gs + (int64_t)b * a.E, a.E, a.N, a.chunk, unit - b * a.slots);
+  if (cp.e < 0) return;
+  const bool first = t < n0;
+  const Wg192Task& tk = first ? a.t[0] : a.t[1];
+  const int tl = first ? t : t - n0;
+  const int y0 = tl / tk.x_tiles * kT, x0 = tl % tk.x_tiles * kT;
+  Acc acc;
+  zero_acc(acc);
+  if (cp.size > 0) {
+    const int64_t row = (int64_t)b * a.N + cp.start;
+    const Operand P{tk.p + row * tk.Y, tk.Y, tk.Y, cp.size};
+    const Operand Q{tk.q + row * tk.X, tk.X, tk.X, cp.size};
+    Loader<RMajor> lp, lq;
+    lp.init(P, y0);
+    lq.init(Q, x0);
+    k_loop<RMajor, RMajor>(lp, lq, (cp.size + kTK - 1) / kTK, ring, acc);
+  }
+  const int X = tk.X, Y = tk.Y;
+  const bool partial = cp.part >= 0;
+  uint16_t* out = tk.out + ((int64_t)b * a.E + cp.e) * X * Y;
+  float* part = a.part + ((int64_t)b * a.parts_ub + (partial ? cp.part : 0)) * a.n_out + (first ? 0 : (int64_t)a.t[0].X * a.t[0].Y);
+  staged(
+      acc, reinterpret_cast<float*>(ring), [](auto, auto, int, int) {},
+      [&](auto, auto, int n, int g, const float (&v)[8]) __attribute__((always_inline)) {
+        const int x = x0 + n, y = y0 + 8 * g;
+        if (x >= X || y >= Y) return;
+        const int64_t at = (int64_t)x * Y + y;
+        if (partial) {
+          *reinterpret_cast<float4*>(part + at) = make_float4(v[0], v[1], v[2], v[3]);
+          *reinterpret_cast<float4*>(part + at + 4) = make_float4(v[4], v[5], v[6], v[7]);
+        } else {
+          store8_bf16(out + at, v);
+        }
+      });
+}
+
+// The outputs of the experts with several chunks: bf16 of the partials' sum,
+// added in chunk order.  blockIdx.y = b * E + e.
+__global__ __launch_bounds__(256) void wg192_reduce_kernel(Wg192Args a) {
+  const int b = blockIdx.y / a.E, e = blockIdx.y % a.E;
+  const int lane = threadIdx.x & 63;
+  const int32_t* gs_b = a.gs + (int64_t)b * a.E;
+  int tok_base = 0, slot = 0, parts = 0;
+  for (int e0 = 0; e0 < a.E; e0 += 64) {
+    const int ee = e0 + lane;
+    const int graw = ee < a.E ? gs_b[ee] : 0;
+    const int g = graw > 0 ? graw : 0;
+    const int tok_incl = wave_incl_scan(g);
+    const int start = min(tok_base + tok_incl - g, a.N);
+    const int nt = ee < a.E ? partials_of(chunks_of(min(g, a.N - start), a.chunk)) : 0;
+    const int incl = wave_incl_scan(nt);
+    if (e < e0 + 64) {
+      parts = lane_value(nt, e - e0);
+      slot += lane_value(incl, e - e0) - parts;
+      break;
+    }
+    tok_base += lane_value(tok_incl, 63);
+    slot += lane_value(incl, 63);
+  }
+  if (parts < 2) return;
+  const int64_t n0 = (int64_t)a.t[0].X * a.t[0].Y;
+  const float* src = a.part + ((int64_t)b * a.parts_ub + slot) * a.n_out;
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < a.n_out;
+       i += (int64_t)gridDim.x * 2048) {
+    float v[8] = {};
+#pragma unroll 4
+    for (int s = 0; s < parts; ++s) {
+      const float4 x = *reinterpret_cast<const float4*>(src + s * a.n_out + i);
+      const float4 y = *reinterpret_cast<const float4*>(src + s * a.n_out + i + 4);
+      v[0] += x.x; v[1] += x.y; v[2] += x.z; v[3] += x.w;
+      v[4] += y.x; v[5] += y.y; v[6] += y.z; v[7] += y.w;
+    }
+    uint16_t* o = i < n0 ? a.t[0].out + ((int64_t)b * a.E + e) * n0 + i
+                         : a.t[1].out + ((int64_t)b * a.E + e) * (a.n_out - n0) + i - n0;
+    store8_bf16(o, v);
+  }
+}
+
+int tiles_of(int n) { return (n + kT - 1) / kT; }
+
+}  // namespace
+
+// ------------------------------------------------------------------ host ----
+Wg192Plan wg192_plan(int B, int E, int I, int D, int N) {
+  Wg192Plan p{};
+  // dW0_W2 [2I][D] and dW1 [D][I]
+  p.per = tiles_of(2 * I) * tiles_of(D) + tiles_of(D) * tiles_of(I);
+  const int64_t tiles256 =
+      (int64_t)B * E * (((2 * I + 255) / 256) * ((D + 255) / 256) + ((D + 255) / 256) * ((I + 255) / 256));
+  const bool narrow = I <= 512 && D <= 512;
+  p.use = E > 1 && N > 0 && (narrow || (N <= 256 * (int64_t)E && tiles256 < 2048));
+  int chunk = 4096;
+  if (narrow) {
+    chunk = 512;
+    while (chunk < 4096 && (chunk < 2 * D || (int64_t)chunk * 256 < (int64_t)B * N * p.per)) chunk *= 2;
+  }
+  p.chunk = chunk;
+  p.slots = (N + chunk - 1) / chunk + E;
+  p.parts_ub = N > chunk ? (int)(2 * (int64_t)N / chunk) : 0;
+  p.n_out = (int64_t)3 * I * D;
+  p.bytes = (size_t)B * p.parts_ub * p.n_out * sizeof(float);
+  return p;
+}
+
+int launch_wg192(const Wg192Plan& pl, const void* dy, const void* k, const void* hid,
+                 const void* v, void* dw0_w2, void* dw1, const int32_t* gs, int B, int E, int I,
+                 int D, int N, void* workspace, hipStream_t st, const char* what) {
+  const int64_t units = ((int64_t)B * pl.slots + kXcds - 1) / kXcds * kXcds;
+  UTTT_REQUIRE(units * pl.per <= 0x7fffffffLL, "%s: problem too large for one launch", what);
+  Wg192Args a{};
+  auto task = [](const void* p, const void* q, void* out, int X, int Y) {
+    return Wg192Task{static_cast<const uint16_t*>(p), static_cast<const uint16_t*>(q),
+                     static_cast<uint16_t*>(out), X, Y, tiles_of(Y), tiles_of(X)};
+  };
+  a.t[0] = task(k, dy, dw0_w2, 2 * I, D);
+  a.t[1] = task(hid, v, dw1, D, I);
+  a.gs = gs;
+  a.part = static_cast<float*>(workspace);
+  a.n_out = pl.n_out;
+  a.B = B;
+  a.E = E;
+  a.N = N;
+  a.chunk = pl.chunk;
+  a.slots = pl.slots;
+  a.parts_ub = pl.parts_ub;
+  hipLaunchKernelGGL(wg192_kernel, dim3((unsigned)(units * pl.per)), dim3(kTThreads), 0, st, a);
+  if (int rc = check_launch(what)) return rc;
+  if (pl.parts_ub == 0) return UTTT_OK;  // no expert has a second chunk
+  const unsigned blocks = (unsigned)std::min<int64_t>((pl.n_out / 8 + 255) / 256, 64);
+  hipLaunchKernelGGL(wg192_reduce_kernel, dim3(blocks, (unsigned)(B * E)), dim3(256), 0, st, a);
+  return check_launch(what);
+}
+
+}  // namespace uttt

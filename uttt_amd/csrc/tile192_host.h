@@ -1,0 +1,42 @@
+// Host side of the 192 x 192 tile kernels (tile192.hip).
+#pragma once
+
+#include "common.h"
+
+namespace uttt {
+
+// Chunked weight gradients of the grouped UPDATE on 192 x 192 tiles: `use`
+// where they are the faster ones, a pure function of the sizes (so the
+// workspace query and the launch agree):
+//   - narrow experts (I, D <= 512): the 256 x 256 tiles are half padding and
+//     one expert's few tiles are bound by its longest segment (48 experts of
+//     192 x 192 over 196 608 tokens: 285-459 -> 105 us; 96 of 384 x 384 over
+//     16 384: 70 -> 46, over 196 608: 374 -> 290);
+//   - short segments (at most 256 tokens per expert on average) on grids under
+//     eight rounds of 256-tile workgroups: 16 experts of 768 x 1536 over 3062
+//     tokens 71 -> 57 us; 32 of 1536 x 3072 over 4096 (27 rounds) 420 / 423.
+// Not for one expert per batch (uTTT-Dense heads), where the split-K 256 tiles
+// measure the same or faster (4 x [192 x 384] over 98 304 tokens 79 / 90 us).
+// Longer segments of wide experts keep the 256 tiles (16 of 768 x 1536 over
+// 49 152 tokens: 394 / 521 us).
+// Chunk length: about 256 (chunk, tile) workgroups on an even routing, 512 to
+// 4096 tokens, at least 2 D (a batch's partials then fit in the backward's
+// dead intermediates, 12 N I bytes).
+struct Wg192Plan {
+  bool use;
+  int per;        // output tiles of one expert
+  int chunk;      // tokens per chunk
+  int slots;      // upper bound of the chunks of one batch
+  int parts_ub;   // upper bound of its partial chunks
+  int64_t n_out;  // output elements of one expert
+  size_t bytes;   // fp32 partials
+};
+Wg192Plan wg192_plan(int B, int E, int I, int D, int N);
+
+// dW0_W2 [2I][D] = DY^T K and dW1 [D][I] = V^T Hid of every expert.  I, D
+// multiples of 8, pointers 16-byte aligned; `workspace` holds plan.bytes.
+int launch_wg192(const Wg192Plan& plan, const void* dy, const void* k, const void* hid,
+                 const void* v, void* dw0_w2, void* dw1, const int32_t* gs, int B, int E, int I,
+                 int D, int N, void* workspace, hipStream_t st, const char* what);
+
+}  // namespace uttt
