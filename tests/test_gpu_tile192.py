@@ -1,13 +1,16 @@
 """The 192 x 192-tile products (csrc/tile192.hip): the chunked weight
-gradients at the edges of their chunks, tiles and experts, against fp64.
+gradients at the edges of their chunks, tiles and experts, against fp64, and
+the Newton-Schulz steps.
 
-Bound per element: one bf16 rounding of the result (2^-9 relative, 2^-8 taken)
+Bound of the gradients per element: one bf16 rounding of the result (2^-9 relative, 2^-8 taken)
 plus the fp32 accumulation of n products, n * 2^-24 of the sum of their
 magnitudes, whatever the order.
 """
 import pytest
 import torch
 
+from oracle import write as OW
+from uttt_amd import fast_weight_write as FWW
 from uttt_amd.lact_moe_triton import _grouped as G
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +53,42 @@ def test_chunked_weight_gradients(name):
                 ref = p64.T @ q64
                 bound = 2.0 ** -8 * ref.abs() + n * 2.0 ** -24 * (p64.abs().T @ q64.abs())
                 assert bool(((ours.double() - ref).abs() <= bound).all()), (b, e, n)
+
+
+# (matrices, rows, columns, dtype, offset in elements): partial tiles on both
+# axes, more matrices than XCDs, several tiles per side (mirrored ones), a side
+# below one MFMA block, an input that is not 16-byte aligned
+@pytest.mark.parametrize("n,R,C,dtype,offset", [
+    (5, 200, 264, torch.float32, 0), (9, 384, 384, torch.bfloat16, 0),
+    (2, 776, 392, torch.float32, 0), (3, 8, 1000, torch.bfloat16, 0),
+    (1, 584, 584, torch.float32, 0), (2, 208, 416, torch.float32, 1),
+    (2, 416, 208, torch.bfloat16, 1),
+])
+def test_newton_schulz5_tiles(n, R, C, dtype, offset):
+    """Against the same iteration in fp64: overall no further off than 1.5x the
+    bf16 oracle (both are bf16 realisations of one map), and at most 5e-2 of
+    the rms row (column) norm in every row and column of 200 elements or more.
+    A perturbation grows by up to a = 4 per step along
+    a small singular direction, so two realisations differ by about 1e-2,
+    spread evenly over the rows, and no elementwise bound of a few ulps holds;
+    an element that is wrong by its own size is 1 / sqrt(side) of its row, at
+    least 5e-2 for the sides up to 392."""
+    G = torch.randn(n, R, C, generator=torch.Generator().manual_seed(R + C)).to(dtype)
+    buf = torch.empty(n * R * C + offset, dtype=dtype, device=DEV)
+    dev = buf[offset:].view(n, R, C)
+    dev.copy_(G)
+    ours = FWW.newton_schulz5(dev, 0.75).cpu().double()
+    ref = (OW.newton_schulz5(G) * 0.75).double()
+    X = G.double()
+    X = X.transpose(1, 2) if R > C else X
+    X = X / (X.norm(dim=(1, 2), keepdim=True) + 1e-7)
+    for a, b, c in OW.NS5_COEFFS:
+        A = X @ X.transpose(1, 2)
+        X = a * X + (b * A + c * A @ A) @ X
+    exact = (X.transpose(1, 2) if R > C else X) * 0.75
+    rel = lambda x: ((x - exact).norm() / exact.norm()).item()
+    assert rel(ours) <= 1.5 * rel(ref) + 1e-3
+    for dim in (1, 2):
+        if exact.shape[dim] >= 200:
+            rms = exact.norm(dim=dim).pow(2).mean().sqrt()
+            assert ((ours - exact).norm(dim=dim).max() / rms).item() <= 5e-2

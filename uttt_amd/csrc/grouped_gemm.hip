@@ -44,8 +44,6 @@ struct TnArgs {
                             // gm = 0: plain order (m-tile fastest)
   int B, E, N;
   int two;                  // tile 1 multiplied
-  int sym;                  // symmetric output (one square group per batch, m_step equal to
-                            // the token tile): only tiles on or below the diagonal are computed
   const int32_t* gs;
 };
 
@@ -358,135 +356,6 @@ struct EpiStore {
           store4(ob, ea.ld, c.tt.start + c.tt.n0 + n, col, v[0], v[1], v[2], v[3]);
       });
     }
-  }
-};
-
-// --- epilogue: o = bf16(bf16(alpha * in) + bf16(beta * bf16(acc))) (no `in`:
-// o = bf16(beta * bf16(acc))), stored to `out`, and bf16(gamma * o) to `out2`
-// when given; all token-major [B, N, ld] at the product's position.  The
-// Newton-Schulz steps with the bf16 rounding after every operation that the
-// reference's bf16 tensor arithmetic has: A = X X^T (with c A as out2),
-// B = b A + (c A) A, X' = a X + B X.
-// Through the LDS frame (16-byte accesses along the token rows; the arrays
-// are 16-byte aligned workspace with ld a multiple of 8).
-// SYM: the product is symmetric and only tiles on or below the diagonal run
-// (TnArgs::sym); a tile strictly below the diagonal also stores its
-// transpose, every thread 8 consecutive tokens of one output row (`in` is
-// symmetric too, so the transposed element is read from the transposed
-// position).
-struct EpiLinCombArgs {
-  uint16_t* out;
-  uint16_t* out2;
-  const uint16_t* in;
-  int64_t ld;
-  int col_end;
-  int N;
-  float alpha, beta, gamma;
-};
-
-// 8 consecutive elements at offset `at` of every array; xin = in[at .. at + 7]
-// as loaded (ignored without `in`).
-__device__ __forceinline__ void lincomb8(const EpiLinCombArgs& ea, const float (&v)[8],
-                                         const uint4& xin, int64_t at) {
-  float x[8], o[8];
-  unpack8(xin, x);
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const float p = bf16r(ea.beta * bf16r(v[u]));
-    o[u] = ea.in != nullptr ? bf16r(bf16r(ea.alpha * x[u]) + p) : p;
-  }
-  store8(ea.out + at, o);
-  if (ea.out2 != nullptr) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) o[u] *= ea.gamma;
-    store8(ea.out2 + at, o);
-  }
-}
-
-template <bool SYM = false>
-struct EpiLinComb {
-  static constexpr bool kStaleColumnsUnused = true;
-  using Args = EpiLinCombArgs;
-  template <int NA>
-  __device__ __forceinline__ static void apply(const Args& ea, const f32x16 (&acc0)[NA][kNB],
-                                               const f32x16 (&acc1)[NA][kNB], const TileCtx& c,
-                                               bool two) {
-    const int64_t bo = (int64_t)c.b * ea.N * ea.ld;
-    (void)two;  // past col_end when tile 1 is not multiplied
-    // `in` is read from valid addresses whether or not it is given (out's,
-    // ignored then), all of a quarter's loads before any is used: a load
-    // under a branch, or one used at once, waits for every store in flight
-    const uint16_t* src = ea.in != nullptr ? ea.in : ea.out;
-    const bool mirror = SYM && c.m0 < c.tt.n0;  // uniform: a tile strictly below the diagonal
-    block_barrier();                             // every wave is done reading the stage buffers
-    static_for<4>([&](auto QQ) __attribute__((always_inline)) {
-      constexpr int Q = QQ;
-      // the tile itself: token nl of the quarter, rows 8 g .. 8 g + 7 of each part
-      uint4 xt[kItemsOf<NA>][2];
-#pragma unroll
-      for (int k = 0; k < kItemsOf<NA>; ++k) {
-        const int it = threadIdx.x + kThreadsOf<NA> * k;
-        const int nl = it >> 4, g = it & 15;
-        const bool tok_ok = c.tt.n0 + Q * 64 + nl < c.tt.size;
-        const int64_t tok = c.tt.start + c.tt.n0 + Q * 64 + nl;
-#pragma unroll
-        for (int part = 0; part < 2; ++part) {
-          const int col = c.m0 + part * kTileRows + 8 * g;
-          const int64_t at = tok_ok && col < ea.col_end ? bo + tok * ea.ld + col : bo;
-          xt[k][part] = *reinterpret_cast<const uint4*>(src + at);
-        }
-      }
-      // its transpose: row `col` of the output, 8 consecutive tokens
-      uint4 xm[2 * kItemsOf<NA>];
-      if (mirror) {
-#pragma unroll
-        for (int k = 0; k < 2 * kItemsOf<NA>; ++k) {
-          const int it = threadIdx.x + kThreadsOf<NA> * k;
-          const int r = it & 127, part = (it >> 7) & 1, g8 = it >> 8;
-          const int nq = Q * 64 + 8 * g8;
-          const int col = c.m0 + part * kTileRows + r;
-          const bool ok = c.tt.n0 + nq < c.tt.size && col < ea.col_end;  // multiples of 8
-          const int64_t at = ok ? bo + (int64_t)col * ea.ld + c.tt.start + c.tt.n0 + nq : bo;
-          xm[k] = *reinterpret_cast<const uint4*>(src + at);
-        }
-      }
-      stage_quarter<Q>(acc0, acc1, c);
-      block_barrier();
-#pragma unroll
-      for (int k = 0; k < kItemsOf<NA>; ++k) {
-        const int it = threadIdx.x + kThreadsOf<NA> * k;
-        const int nl = it >> 4, g = it & 15;
-        if (c.tt.n0 + Q * 64 + nl >= c.tt.size) continue;
-        const int64_t tok = c.tt.start + c.tt.n0 + Q * 64 + nl;
-#pragma unroll
-        for (int part = 0; part < 2; ++part) {
-          const int col = c.m0 + part * kTileRows + 8 * g;
-          if (col >= ea.col_end) continue;  // col_end is a multiple of 8
-          float v[8];
-          staged8(part == 0 ? c.lds0 : c.lds1, nl, g, v);
-          lincomb8(ea, v, xt[k][part], bo + tok * ea.ld + col);
-        }
-      }
-      if (mirror) {
-#pragma unroll
-        for (int k = 0; k < 2 * kItemsOf<NA>; ++k) {
-          const int it = threadIdx.x + kThreadsOf<NA> * k;
-          const int r = it & 127, part = (it >> 7) & 1, g8 = it >> 8;
-          const int nq = Q * 64 + 8 * g8;
-          const int col = c.m0 + part * kTileRows + r;
-          if (c.tt.n0 + nq >= c.tt.size || col >= ea.col_end) continue;
-          const float* lds = part == 0 ? c.lds0 : c.lds1;
-          float v[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            const int nl = 8 * g8 + u;
-            v[u] = lds[nl * 128 + (((r >> 2) ^ (nl & 31)) << 2) + (r & 3)];
-          }
-          lincomb8(ea, v, xm[k], bo + (int64_t)col * ea.ld + c.tt.start + c.tt.n0 + nq);
-        }
-      }
-      block_barrier();
-    });
   }
 };
 
@@ -851,7 +720,7 @@ __global__ __launch_bounds__(kThreadsOf<NA>) void tn_kernel(TnArgs a, typename E
   if (mt >= a.m_tiles || ntg >= a.B * a.n_tiles_ub) return;  // padding of the super-tile grid
   const int b = ntg / a.n_tiles_ub, nt = ntg % a.n_tiles_ub;
   const TokenTile tt = find_token_tile<kBRows>(a.gs + (int64_t)b * a.E, a.E, a.N, nt);
-  if (tt.e < 0 || (a.sym && mt * a.m_step > tt.n0)) return;
+  if (tt.e < 0) return;
   const int m0 = mt * a.m_step;
 
   const int64_t ag = ((int64_t)b * a.E + tt.e) * a.a_group;
@@ -1448,12 +1317,15 @@ __global__ __launch_bounds__(256) void transpose16_kernel(const uint16_t* __rest
 // ============================================ Newton-Schulz orthogonalisation ==
 // Per matrix G [R, C] (BE of them): X = bf16(G) as [m, n] = [min, max] (G
 // transposed when R > C), X /= bf16(bf16(||X||_F) + 1e-7), five steps of
-// A = X X^T, B = b A + (c A) A, X = a X + B X, then bf16(X * scale) back in
-// G's orientation.  Reference: zeropower_via_newtonschulz5,
+// A = X X^T, B = b A + (c A) A, X = a X + B X (tile192.hip), then
+// bf16(X * scale) back in G's orientation (the last step's epilogue).
+// Reference: zeropower_via_newtonschulz5,
 // uttt_llm/flame/custom_models/uttt_moe/ttt_operation.py:19-46.
 constexpr int kNsParts = 64;   // partial sums of squares per matrix
 
-// part[be, p] = sum of bf16(g)^2 over the p-th of kNsParts equal slices of matrix be.
+// part[be, p] = sum of bf16(g)^2 over the p-th of kNsParts equal slices of
+// matrix be.  Bound by its loads' latency: eight of a thread's go out before
+// the first is added (in order).
 template <class TT>
 __global__ __launch_bounds__(256) void ns_sumsq_kernel(const typename TT::S* __restrict__ g,
                                                        int64_t elems, float* __restrict__ part) {
@@ -1463,7 +1335,18 @@ __global__ __launch_bounds__(256) void ns_sumsq_kernel(const typename TT::S* __r
   const int64_t lo = p * per, hi = lo + per < elems ? lo + per : elems;
   const typename TT::S* gb = g + (int64_t)be * elems;
   float acc = 0.0f;
-  for (int64_t i = lo + threadIdx.x; i < hi; i += 256) {
+  int64_t i = lo + threadIdx.x;
+  for (; i + 7 * 256 < hi; i += 8 * 256) {
+    typename TT::S raw[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) raw[u] = gb[i + u * 256];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float x = bf16r(TT::load(raw[u]));
+      acc = __builtin_fmaf(x, x, acc);
+    }
+  }
+  for (; i < hi; i += 256) {
     const float x = bf16r(TT::load(gb[i]));
     acc = __builtin_fmaf(x, x, acc);
   }
@@ -1476,50 +1359,67 @@ __global__ __launch_bounds__(256) void ns_sumsq_kernel(const typename TT::S* __r
   if (threadIdx.x == 0) part[(int64_t)be * kNsParts + p] = red[0];
 }
 
-// denom[be] = bf16(bf16(sqrt(sum of parts)) + 1e-7) (fixed order); gs[be] = m.
-__global__ __launch_bounds__(256) void ns_norm_kernel(const float* __restrict__ part, int BE,
-                                                      int m, float* __restrict__ denom,
-                                                      int32_t* __restrict__ gs) {
-  const int be = blockIdx.x * 256 + threadIdx.x;
-  if (be >= BE) return;
+// bf16(bf16(sqrt(sum of matrix be's parts, in order)) + 1e-7), by every wave.
+__device__ __forceinline__ float ns_denom(const float* __restrict__ part, int be) {
+  static_assert(kNsParts == 64, "one part per lane");
+  const int v = __float_as_int(part[(int64_t)be * kNsParts + (threadIdx.x & 63)]);
   float s = 0.0f;
-  for (int p = 0; p < kNsParts; ++p) s += part[(int64_t)be * kNsParts + p];
-  denom[be] = bf16r(bf16r(sqrtf(s)) + 1e-7f);
-  gs[be] = m;
+#pragma unroll
+  for (int p = 0; p < kNsParts; ++p) s += __int_as_float(__builtin_amdgcn_readlane(v, p));
+  return bf16r(bf16r(sqrtf(s)) + 1e-7f);
 }
 
-// dst [BE, Rd, Cd] from src [BE, Rs, Cs] through 64x64 LDS tiles; TRANS: dst = src^T.
-//   PREP:  dst = bf16(bf16(src) / denom[be])
-//   FINAL: dst = bf16(src * scale)
-template <class TS, bool TRANS, bool PREP>
-__global__ __launch_bounds__(256) void ns_tile_kernel(const typename TS::S* __restrict__ src,
-                                                      int Rs, int Cs, const float* __restrict__ denom,
-                                                      float scale, uint16_t* __restrict__ dst,
-                                                      int rt, int ct) {
+// X = bf16(bf16(G) / denom): dst [BE, Cs, Rs] = src [BE, Rs, Cs]^T through
+// 64x64 LDS tiles.
+template <class TS>
+__global__ __launch_bounds__(256) void ns_prep_trans_kernel(
+    const typename TS::S* __restrict__ src, int Rs, int Cs, const float* __restrict__ part,
+    uint16_t* __restrict__ dst, int rt, int ct) {
   __shared__ float tile[64][65];
   const int bid = blockIdx.x;
   const int tc = bid % ct, tr = (bid / ct) % rt, be = bid / (ct * rt);
-  const int Rd = TRANS ? Cs : Rs, Cd = TRANS ? Rs : Cs;
   const typename TS::S* sb = src + (int64_t)be * Rs * Cs;
-  uint16_t* db = dst + (int64_t)be * Rd * Cd;
-  const float mul = PREP ? 0.0f : scale;
-  const float dv = PREP ? denom[be] : 1.0f;
+  uint16_t* db = dst + (int64_t)be * Rs * Cs;
+  const float dv = ns_denom(part, be);
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  // source tile rows/cols: the dst tile (tr, tc) maps to src tile (tc, tr) when transposing
-  const int sr0 = (TRANS ? tc : tr) * 64, sc0 = (TRANS ? tr : tc) * 64;
+  // dst tile (tr, tc) is src tile (tc, tr)
   for (int yy = ty; yy < 64; yy += 4) {
-    const int r = sr0 + yy, cc = sc0 + tx;
-    float v = 0.0f;
-    if (r < Rs && cc < Cs) {
-      const float x = TS::load(sb[(int64_t)r * Cs + cc]);
-      v = PREP ? bf16r(bf16r(x) / dv) : bf16r(x * mul);
-    }
-    tile[yy][tx] = v;
+    const int r = tc * 64 + yy, cc = tr * 64 + tx;
+    if (r < Rs && cc < Cs) tile[yy][tx] = bf16r(bf16r(TS::load(sb[(int64_t)r * Cs + cc])) / dv);
   }
   __syncthreads();
   for (int yy = ty; yy < 64; yy += 4) {
     const int r = tr * 64 + yy, cc = tc * 64 + tx;
-    if (r < Rd && cc < Cd) db[(int64_t)r * Cd + cc] = f32_to_bf16(TRANS ? tile[tx][yy] : tile[yy][tx]);
+    if (r < Cs && cc < Rs) db[(int64_t)r * Rs + cc] = f32_to_bf16(tile[tx][yy]);
+  }
+}
+
+// The same in the source's order, 8 elements per thread and step (elems: of a
+// matrix, a multiple of 8; src 16-byte aligned with VEC); four steps per block
+// share the denominator's 64-term sum.
+constexpr int kNsPrepSteps = 4;
+template <class TS, bool VEC>
+__global__ __launch_bounds__(256) void ns_prep_kernel(const typename TS::S* __restrict__ src,
+                                                      int64_t elems,
+                                                      const float* __restrict__ part,
+                                                      uint16_t* __restrict__ dst) {
+  const int be = blockIdx.y;
+  const float dv = ns_denom(part, be);
+#pragma unroll
+  for (int q = 0; q < kNsPrepSteps; ++q) {
+    const int64_t i = (((int64_t)blockIdx.x * kNsPrepSteps + q) * 256 + threadIdx.x) * 8;
+    if (i >= elems) return;
+    const typename TS::S* p = src + be * elems + i;
+    float v[8];
+    if constexpr (VEC) {
+      load8(p, v);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = TS::load(p[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = bf16r(v[u]) / dv;
+    store8(dst + be * elems + i, v);
   }
 }
 
@@ -1561,7 +1461,6 @@ TnArgs tn_args(const void* a0, const void* a1, const void* x, int K, int64_t lda
   t.E = E;
   t.N = N;
   t.two = 1;
-  t.sym = 0;
   t.gs = gs;
   (void)B;
   return t;
@@ -1769,20 +1668,6 @@ int launch_wide(const void* a, const void* x, int K, const void* a_2, const void
   const EpiStoreArgs<OutT> ea{y, M, {0, kTileRows}, {M, M}, N};
   if (aligned16(y)) return launch_tn<AMAJ, EpiStore<OutT, true>>(t, ea, B, st, what);
   return launch_tn<AMAJ, EpiStore<OutT>>(t, ea, B, st, what);
-}
-
-// y[b, n, m] = bf16(bf16(alpha in) + bf16(beta bf16(sum_k A(m, k) x[b, n, k]))) (and
-// y2 = bf16(gamma y) when y2), E = 1 group of N rows per batch, M rows in m-tiles of 256.
-template <int AMAJ>
-int launch_lincomb(const void* a, const void* x, int K, int M, int64_t lda, int64_t a_group,
-                   const uint16_t* in, float alpha, float beta, uint16_t* y, uint16_t* y2,
-                   float gamma, int B, int N, const int32_t* gs, hipStream_t st,
-                   const char* what, bool sym = false) {
-  TnArgs t = tn_args(a, a, x, K, lda, a_group, 0, kTileRows, M, M, 2 * kTileRows, M, B, 1, N, gs);
-  t.sym = sym ? 1 : 0;
-  const EpiLinCombArgs ea{y, y2, in, M, M, N, alpha, beta, gamma};
-  if (sym) return launch_tn<AMAJ, EpiLinComb<true>>(t, ea, B, st, what);
-  return launch_tn<AMAJ, EpiLinComb<>>(t, ea, B, st, what);
 }
 
 WgTask wg_task(const void* p, const void* q, void* out, int X, int Y) {
@@ -2368,15 +2253,11 @@ extern "C" int uttt_transpose_2byte(const void* in, int B, int R, int C, void* o
 // ============================================================ Newton-Schulz ==
 namespace {
 struct NsWs {
-  size_t gs, denom, part, x0, x1, a, ac, bm, total;
+  size_t part, x0, x1, a, bm, total;
 };
 NsWs ns_ws(int BE, int m, int n) {
   NsWs w{};
   size_t o = 0;
-  w.gs = o;
-  o += up256((size_t)BE * 4);
-  w.denom = o;
-  o += up256((size_t)BE * 4);
   w.part = o;
   o += up256((size_t)BE * kNsParts * 4);
   w.x0 = o;
@@ -2384,8 +2265,6 @@ NsWs ns_ws(int BE, int m, int n) {
   w.x1 = o;
   o += up256((size_t)BE * m * n * 2);
   w.a = o;
-  o += up256((size_t)BE * m * m * 2);
-  w.ac = o;
   o += up256((size_t)BE * m * m * 2);
   w.bm = o;
   o += up256((size_t)BE * m * m * 2);
@@ -2421,85 +2300,48 @@ extern "C" int uttt_newton_schulz5(const void* g, int g_dtype, int BE, int rows,
     return launch_ns_small(g, g_dtype, BE, rows, cols, out_scale, static_cast<uint16_t*>(out),
                            st);
   uint8_t* wb = static_cast<uint8_t*>(workspace);
-  int32_t* gs = reinterpret_cast<int32_t*>(wb + w.gs);
-  float* denom = reinterpret_cast<float*>(wb + w.denom);
   float* part = reinterpret_cast<float*>(wb + w.part);
   uint16_t* X = reinterpret_cast<uint16_t*>(wb + w.x0);
   uint16_t* Xn = reinterpret_cast<uint16_t*>(wb + w.x1);
   uint16_t* A = reinterpret_cast<uint16_t*>(wb + w.a);
-  uint16_t* Ac = reinterpret_cast<uint16_t*>(wb + w.ac);
   uint16_t* Bm = reinterpret_cast<uint16_t*>(wb + w.bm);
   const int64_t elems = (int64_t)m * n;
-  // 1. norm
+  UTTT_REQUIRE(n < (1 << 23), "newton_schulz5: rows of 2^23 or more elements are not supported");
+  const int rt = (m + 63) / 64, ct = (n + 63) / 64;
+  const int64_t prep_blocks = trans ? (int64_t)rt * ct * BE : (elems / 8 + 256 * kNsPrepSteps - 1) / (256 * kNsPrepSteps);
+  if (int rc = check_grid(prep_blocks, "newton_schulz5(prep)")) return rc;
   UTTT_DTYPE_SWITCH_LR(g_dtype, TT, {
-    hipLaunchKernelGGL((ns_sumsq_kernel<TT>), dim3(kNsParts, BE), dim3(256), 0, st,
-                       static_cast<const typename TT::S*>(g), elems, part);
+    using S = typename TT::S;
+    const S* gp = static_cast<const S*>(g);
+    // 1. norm
+    hipLaunchKernelGGL((ns_sumsq_kernel<TT>), dim3(kNsParts, BE), dim3(256), 0, st, gp, elems,
+                       part);
+    if (int rc = check_launch("newton_schulz5(norm)")) return rc;
+    // 2. X = bf16(bf16(G') / denom), G' = G^T when rows > cols
+    if (trans)
+      hipLaunchKernelGGL((ns_prep_trans_kernel<TT>), dim3((unsigned)prep_blocks), dim3(256), 0, st,
+                         gp, rows, cols, part, X, rt, ct);
+    else if (aligned16(g))
+      hipLaunchKernelGGL((ns_prep_kernel<TT, true>), dim3((unsigned)prep_blocks, BE), dim3(256), 0,
+                         st, gp, elems, part, X);
+    else
+      hipLaunchKernelGGL((ns_prep_kernel<TT, false>), dim3((unsigned)prep_blocks, BE), dim3(256),
+                         0, st, gp, elems, part, X);
   });
-  if (int rc = check_launch("newton_schulz5(norm)")) return rc;
-  hipLaunchKernelGGL(ns_norm_kernel, dim3((BE + 255) / 256), dim3(256), 0, st, part, BE, m, denom, gs);
-  if (int rc = check_launch("newton_schulz5(norm)")) return rc;
-  // 2. X = bf16(bf16(G') / denom), G' = G^T when rows > cols
-  {
-    const int rt = (m + 63) / 64, ct = (n + 63) / 64;
-    const int64_t blocks = (int64_t)rt * ct * BE;
-    if (int rc = check_grid(blocks, "newton_schulz5(prep)")) return rc;
-    UTTT_DTYPE_SWITCH_LR(g_dtype, TT, {
-      using S = typename TT::S;
-      if (trans)
-        hipLaunchKernelGGL((ns_tile_kernel<TT, true, true>), dim3((unsigned)blocks), dim3(256), 0,
-                           st, static_cast<const S*>(g), rows, cols, denom, 1.0f, X, rt, ct);
-      else
-        hipLaunchKernelGGL((ns_tile_kernel<TT, false, true>), dim3((unsigned)blocks), dim3(256),
-                           0, st, static_cast<const S*>(g), rows, cols, denom, 1.0f, X, rt, ct);
-    });
-    if (int rc = check_launch("newton_schulz5(prep)")) return rc;
-  }
-  // 3. five steps (the reference's coefficient table)
+  if (int rc = check_launch("newton_schulz5(prep)")) return rc;
+  // 3. five steps (the reference's coefficient table), the last one into `out`
   static const float kCoef[5][3] = {{4.0848f, -6.8946f, 2.9270f},
                                     {3.9505f, -6.3029f, 2.6377f},
                                     {3.7418f, -5.5913f, 2.3037f},
                                     {2.8769f, -3.1427f, 1.2046f},
                                     {2.8366f, -3.0525f, 1.2012f}};
   for (int it = 0; it < 5; ++it) {
-    const float ca = kCoef[it][0], cb = kCoef[it][1], cc = kCoef[it][2];
-    // A = X X^T and Ac = c A  ([m, m]: x = X as m rows of K = n, A operand = X).
-    // A is symmetric bit for bit (element (i, j) and (j, i) take the same
-    // products in the same k order): only the 256-tiles on or below the
-    // diagonal are multiplied and those below it also store their transposes
-    // (EpiLinComb), which takes 15 of the 36 tiles of a 1536-wide matrix off
-    // the matrix cores
-    if (int rc = launch_lincomb<KMajor>(X, X, n, m, n, elems, nullptr, 0.0f, 1.0f, A, Ac, cc, BE, m,
-                                        gs, st, "newton_schulz5(X X^T)", true))
+    const bool last = it == 4;
+    if (int rc = launch_ns192_step(X, A, Bm, last ? static_cast<uint16_t*>(out) : Xn, BE, m, n,
+                                   kCoef[it][0], kCoef[it][1], kCoef[it][2], last, out_scale,
+                                   trans, st))
       return rc;
-    // B = b A + (c A) A  (x = Ac, A operand = A: A is symmetric, so row j of A
-    // is column j).  The full product: (c A) A is symmetric in exact
-    // arithmetic only, since element (i, j) sums bf16(c A[i, k]) A[k, j] and
-    // element (j, i) sums A[i, k] bf16(c A[k, j]), so mirroring one triangle
-    // would round half of B differently from the reference's product
-    if (int rc = launch_lincomb<KMajor>(A, Ac, m, m, m, (int64_t)m * m, A, cb, 1.0f, Bm, nullptr,
-                                        0.0f, BE, m, gs, st, "newton_schulz5(B)", false))
-      return rc;
-    // X' = a X + B X  ([m, n]: x = B, A operand = X read row-major: A(j, k) = X[k, j])
-    if (int rc = launch_lincomb<RMajor>(X, Bm, m, n, n, elems, X, ca, 1.0f, Xn, nullptr, 0.0f, BE,
-                                        m, gs, st, "newton_schulz5(B X)"))
-      return rc;
-    uint16_t* tmp = X;
-    X = Xn;
-    Xn = tmp;
-  }
-  // 4. out = bf16(X * scale) in G's orientation
-  {
-    const int Rd = rows, Cd = cols;
-    const int rt = (Rd + 63) / 64, ct = (Cd + 63) / 64;
-    const int64_t blocks = (int64_t)rt * ct * BE;
-    if (int rc = check_grid(blocks, "newton_schulz5(out)")) return rc;
-    if (trans)
-      hipLaunchKernelGGL((ns_tile_kernel<BF16T, true, false>), dim3((unsigned)blocks), dim3(256), 0,
-                         st, X, m, n, nullptr, out_scale, static_cast<uint16_t*>(out), rt, ct);
-    else
-      hipLaunchKernelGGL((ns_tile_kernel<BF16T, false, false>), dim3((unsigned)blocks), dim3(256),
-                         0, st, X, m, n, nullptr, out_scale, static_cast<uint16_t*>(out), rt, ct);
-    if (int rc = check_launch("newton_schulz5(out)")) return rc;
+    std::swap(X, Xn);
   }
   return UTTT_OK;
 }

@@ -23,6 +23,8 @@
 //     k-rows k and k + 2 would share banks without the exchange.
 #pragma once
 
+#include <type_traits>
+
 #include "gemm_pipe.h"
 
 namespace uttt {
@@ -108,13 +110,15 @@ struct Loader {
       if constexpr (MAJOR == RMajor) {
         recs = (uint32_t)((k_end - step * kTK) * ld2 - col2);
       } else {
-        recs = 0x80000000u;
+        // lanes past k_end go past the bound; valid offsets (192 rows of under
+        // 2^23 elements) stay below it
+        recs = 0xFFFFFF00u;
         const int lane = threadIdx.x & 63, w = wofs >> 10, kt = k_end % kTK;
 #pragma unroll
         for (int t = 0; t < kTLoads; ++t) {
           const int sl = (t * 4 + w) * 64 + lane;
           const int r = sl >> 2;
-          if (((sl & 3) ^ ((r >> 2) & 3)) * 8 >= kt) off[t] |= 0x80000000u;
+          if (((sl & 3) ^ ((r >> 2) & 3)) * 8 >= kt) off[t] = 0xFFFFFFF0u;
         }
       }
     }
@@ -188,6 +192,17 @@ __device__ __forceinline__ void wait_frags(Frags& f) {
   }
 }
 
+// bf16(c * x) of a fragment.
+__device__ __forceinline__ bf16x8 scaled(const bf16x8& x, float c) {
+  i32x4 w = __builtin_bit_cast(i32x4, x);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t u = (uint32_t)w[k];
+    w[k] = (int)pack_bf16x2(c * __uint_as_float(u << 16), c * __uint_as_float(u & 0xffff0000u));
+  }
+  return __builtin_bit_cast(bf16x8, w);
+}
+
 typedef f32x16 Acc[kNBlk][kNBlk];
 
 __device__ __forceinline__ void mma9(Acc& acc, const Frags& f) {
@@ -204,9 +219,11 @@ __device__ __forceinline__ void mma9(Acc& acc, const Frags& f) {
 // waits (the compiler would drain the loads in flight in front of them).  The
 // products run in increasing k in 16-wide steps with A in the first operand,
 // as in gemm_pipe.h, so the results are the 256-tile kernels' bits.
-template <int AMAJ, int BMAJ>
+// SCALE_B: the second operand is bf16(b_scale * B), converted as its
+// fragments are read.
+template <int AMAJ, int BMAJ, bool SCALE_B = false>
 __device__ __forceinline__ void k_loop(Loader<AMAJ>& la, Loader<BMAJ>& lb, int nk, uint8_t* ring,
-                                       Acc& acc) {
+                                       Acc& acc, float b_scale = 1.0f) {
   const int w = wave_id();
   FragAddr<AMAJ> fa;
   FragAddr<BMAJ> fb;
@@ -241,9 +258,13 @@ __device__ __forceinline__ void k_loop(Loader<AMAJ>& la, Loader<BMAJ>& lb, int n
     }
     __builtin_amdgcn_sched_barrier(0);
     wait_frags<kOps>(f[0]);
+    if constexpr (SCALE_B)
+      static_for<kNBlk>([&](auto I) __attribute__((always_inline)) { f[0].b[I] = scaled(f[0].b[I], b_scale); });
     mma9(acc, f[0]);
     __builtin_amdgcn_sched_barrier(0);
     wait_frags<0>(f[1]);
+    if constexpr (SCALE_B)
+      static_for<kNBlk>([&](auto I) __attribute__((always_inline)) { f[1].b[I] = scaled(f[1].b[I], b_scale); });
     mma9(acc, f[1]);
     __builtin_amdgcn_sched_barrier(0);
     uint8_t* t = p0;
@@ -267,8 +288,16 @@ __device__ __forceinline__ void zero_acc(Acc& acc) {
 // the 192 rows of a column, 384 contiguous bytes of bf16 output.
 //   before(h, k, n, g) runs for each item before its half is staged (loads),
 //   body(h, k, n, g, v[8]) after; k = 0 .. kTItems - 1, n = column in the tile.
-template <class Before, class Body>
-__device__ __forceinline__ void staged(const Acc& acc, float* lds, Before&& before, Body&& body) {
+// With `transposed` (wave-uniform) the half is then read along the other side:
+// body's results (v as it leaves them) go back to LDS, and across(r, n, v[8])
+// gets columns n .. n + 7 of tile row r (consecutive lanes on consecutive rows:
+// conflict-free reads; the 16-byte stores of a row meet in L2).
+struct NoAcross {
+  __device__ void operator()(int, int, const float (&)[8]) const {}
+};
+template <class Before, class Body, class Across = NoAcross>
+__device__ __forceinline__ void staged(const Acc& acc, float* lds, Before&& before, Body&& body,
+                                       bool transposed = false, Across&& across = Across()) {
   const int w = wave_id();
   const int wm = w >> 1, wn = w & 1;
   block_barrier();  // every wave is done reading the ring
@@ -293,13 +322,33 @@ __device__ __forceinline__ void staged(const Acc& acc, float* lds, Before&& befo
     static_for<kTItems>([&](auto K) __attribute__((always_inline)) {
       const int it = threadIdx.x + kTThreads * K;
       const int n = it / 24, g = it % 24;
-      const float4 a =
-          *reinterpret_cast<const float4*>(lds + n * kT + (((2 * g) ^ (n & 15)) << 2));
-      const float4 b =
-          *reinterpret_cast<const float4*>(lds + n * kT + (((2 * g + 1) ^ (n & 15)) << 2));
-      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      float4* pa = reinterpret_cast<float4*>(lds + n * kT + (((2 * g) ^ (n & 15)) << 2));
+      float4* pb = reinterpret_cast<float4*>(lds + n * kT + (((2 * g + 1) ^ (n & 15)) << 2));
+      const float4 a = *pa, b = *pb;
+      float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
       body(H, K, h * kWT + n, g, v);
+      if constexpr (!std::is_same_v<std::decay_t<Across>, NoAcross>) {
+        if (transposed) {
+          *pa = make_float4(v[0], v[1], v[2], v[3]);
+          *pb = make_float4(v[4], v[5], v[6], v[7]);
+        }
+      }
     });
+    if constexpr (!std::is_same_v<std::decay_t<Across>, NoAcross>) {
+      if (transposed) {
+        block_barrier();
+#pragma unroll 1
+        for (int k = 0; k < kTItems; ++k) {
+          const int it = threadIdx.x + kTThreads * k;
+          const int r = it % kT, n = it / kT * 8;
+          float v[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+            v[u] = lds[(n + u) * kT + (((r >> 2) ^ ((n + u) & 15)) << 2) + (r & 3)];
+          across(r, h * kWT + n, v);
+        }
+      }
+    }
     if (h == 0) block_barrier();
   });
 }

@@ -1,7 +1,7 @@
 // Products of narrow matrices on 192 x 192 tiles (tile192.h): the weight
-// gradients of small experts, their token segments cut into chunks.  Called
-// through the C entries of grouped_gemm.hip, which choose between these and
-// the 256 x 256 tiles.
+// gradients of small experts, their token segments cut into chunks, and the
+// Newton-Schulz steps of mid-sized matrices.  Called through the C entries of
+// grouped_gemm.hip, which choose between these and the 256 x 256 tiles.
 #include <algorithm>
 
 #include "tile192.h"
@@ -20,6 +20,15 @@ __device__ __forceinline__ void store8_bf16(uint16_t* p, const float (&v)[8]) {
   u.z = pack_bf16x2(v[4], v[5]);
   u.w = pack_bf16x2(v[6], v[7]);
   *reinterpret_cast<uint4*>(p) = u;
+}
+
+__device__ __forceinline__ void unpack8_bf16(const uint4& u, float (&v)[8]) {
+  const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    v[2 * k] = bf16_to_f32((uint16_t)(w[k] & 0xffffu));
+    v[2 * k + 1] = bf16_to_f32((uint16_t)(w[k] >> 16));
+  }
 }
 
 // ======================================================= weight gradients ==
@@ -129,7 +138,7 @@ __global__ __launch_bounds__(kTThreads, 2) void wg192_kernel(Wg192Args a) {
   float* part = a.part + ((int64_t)b * a.parts_ub + (partial ? cp.part : 0)) * a.n_out + (first ? 0 : (int64_t)a.t[0].X * a.t[0].Y);
   staged(
       acc, reinterpret_cast<float*>(ring), [](auto, auto, int, int) {},
-      [&](auto, auto, int n, int g, const float (&v)[8]) __attribute__((always_inline)) {
+      [&](auto, auto, int n, int g, float (&v)[8]) __attribute__((always_inline)) {
         const int x = x0 + n, y = y0 + 8 * g;
         if (x >= X || y >= Y) return;
         const int64_t at = (int64_t)x * Y + y;
@@ -182,6 +191,99 @@ __global__ __launch_bounds__(256) void wg192_reduce_kernel(Wg192Args a) {
                          : a.t[1].out + ((int64_t)b * a.E + e) * (a.n_out - n0) + i - n0;
     store8_bf16(o, v);
   }
+}
+
+// ========================================================= Newton-Schulz ==
+// The three products of a step over BE matrices, with the rounding of the
+// reference's bf16 tensor arithmetic (grouped_gemm.hip's EpiLinComb):
+//   kNsA  A = bf16(X X^T).  Symmetric bit for bit: only the tiles on or below
+//         the diagonal run, and one below it also stores its transpose.
+//   kNsB  B = bf16(bf16(b A) + bf16((c A) A)): A's rows are both operands, the
+//         second rounded to bf16(c A) as its fragments are read, so that c A
+//         never goes through memory.
+//   kNsX  X' = bf16(bf16(a X) + bf16(B X)); the last step stores
+//         bf16(X' scale) into the caller's output, transposed for a matrix
+//         with more rows than columns.
+// 288 matrices of 384 x 384 read and write 85 MB per operand and product,
+// which is what bounds them; 256 x 256 tiles (half padding there) took 180 / 134
+// / 136 us per product.
+enum NsProduct { kNsA = 0, kNsB = 1, kNsX = 2 };
+
+struct Ns192Args {
+  const uint16_t* a;   // per matrix: [M, K] rows, or [K, M] (kNsX)
+  const uint16_t* x;   // per matrix [R, K]
+  const uint16_t* in;  // per matrix [R, M] (kNsB, kNsX)
+  uint16_t* y;         // per matrix [R, M], or [M, R] with `trans`
+  int K, M, R, BE, m_tiles, r_tiles;
+  float alpha, gamma;  // alpha: of `in`; gamma: c (kNsB), the output scale (kNsX, `last`)
+  int last, trans;
+};
+
+template <int P>
+__global__ __launch_bounds__(kTThreads, 2) void ns192_kernel(Ns192Args s) {
+  constexpr int kAMaj = P == kNsX ? RMajor : KMajor;
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kTRing * kTStage];
+  // the tiles of one matrix run on one XCD and share its L2
+  const int per = P == kNsA ? s.m_tiles * (s.m_tiles + 1) / 2 : s.m_tiles * s.r_tiles;
+  const int loc = blockIdx.x / kXcds;
+  const int mat = loc / per * kXcds + blockIdx.x % kXcds;
+  if (mat >= s.BE) return;
+  const int t = loc % per;
+  int mt = t % s.m_tiles, rt = t / s.m_tiles;
+  if constexpr (P == kNsA) {  // tile t of the lower triangle, row rt holding rt + 1
+    rt = 0;
+    mt = t;
+    while (mt > rt) mt -= ++rt;
+  }
+  const int m0 = mt * kT, r0 = rt * kT;
+  const int64_t om = (int64_t)mat * s.R * s.M;
+  const Operand A{s.a + (int64_t)mat * s.M * s.K, kAMaj == KMajor ? s.K : s.M, s.M, s.K};
+  const Operand X{s.x + (int64_t)mat * s.R * s.K, s.K, s.R, s.K};
+  Loader<kAMaj> la;
+  Loader<KMajor> lx;
+  la.init(A, m0);
+  lx.init(X, r0);
+  Acc acc;
+  zero_acc(acc);
+  k_loop<kAMaj, KMajor, P == kNsB>(la, lx, (s.K + kTK - 1) / kTK, ring, acc, s.gamma);
+  // the epilogue's coordinates from opaque copies, so that no address of it is
+  // held across the K loop
+  const int me = after_loop(m0), re = after_loop(r0);
+  // a half's `in` is loaded from clamped addresses before the half is staged
+  uint4 raw[kTItems];
+  const int64_t row0 = om + (int64_t)re * s.M;
+  const uint16_t* in = uniform_ptr(s.in + row0);
+  uint16_t* y = uniform_ptr(s.y + row0);
+  uint16_t* yt = uniform_ptr(s.y + om + (int64_t)me * s.R);
+  const bool trans = P == kNsX && s.trans;
+  staged(
+      acc, reinterpret_cast<float*>(ring),
+      [&](auto, auto K, int n, int g) __attribute__((always_inline)) {
+        if constexpr (P != kNsA) {
+          const int r = re + n, m = me + 8 * g;
+          const uint32_t at = r < s.R && m < s.M ? (uint32_t)(n * s.M + m) : 0u;
+          raw[K] = *reinterpret_cast<const uint4*>(in + at);
+        }
+      },
+      [&](auto, auto K, int n, int g, float (&v)[8]) __attribute__((always_inline)) {
+        const int r = re + n, m = me + 8 * g;
+        if constexpr (P != kNsA) {
+          float x[8];
+          unpack8_bf16(raw[K], x);
+#pragma unroll
+          for (int u = 0; u < 8; ++u) v[u] = bf16r(bf16r(s.alpha * x[u]) + bf16r(v[u]));
+          if (P == kNsX && s.last) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] *= s.gamma;
+          }
+        }
+        if (!trans && r < s.R && m < s.M) store8_bf16(y + (uint32_t)(n * s.M + m), v);
+      },
+      P == kNsA ? m0 != r0 : trans,
+      [&](int r, int n, const float (&v)[8]) __attribute__((always_inline)) {
+        if (me + r < s.M && re + n < s.R)  // R is a multiple of 8
+          store8_bf16(yt + (uint32_t)(r * s.R + re + n), v);
+      });
 }
 
 int tiles_of(int n) { return (n + kT - 1) / kT; }
@@ -237,6 +339,33 @@ int launch_wg192(const Wg192Plan& pl, const void* dy, const void* k, const void*
   const unsigned blocks = (unsigned)std::min<int64_t>((pl.n_out / 8 + 255) / 256, 64);
   hipLaunchKernelGGL(wg192_reduce_kernel, dim3(blocks, (unsigned)(B * E)), dim3(256), 0, st, a);
   return check_launch(what);
+}
+
+namespace {
+template <int P>
+int launch_ns(const Ns192Args& s, hipStream_t st, const char* what) {
+  const int64_t per = P == kNsA ? (int64_t)s.m_tiles * (s.m_tiles + 1) / 2
+                                : (int64_t)s.m_tiles * s.r_tiles;
+  const int64_t blocks = (int64_t)(s.BE + kXcds - 1) / kXcds * kXcds * per;
+  UTTT_REQUIRE(blocks <= 0x7fffffffLL, "%s: problem too large for one launch", what);
+  hipLaunchKernelGGL((ns192_kernel<P>), dim3((unsigned)blocks), dim3(kTThreads), 0, st, s);
+  return check_launch(what);
+}
+}  // namespace
+
+int launch_ns192_step(const uint16_t* x, uint16_t* a, uint16_t* b, uint16_t* xn, int BE, int m,
+                      int n, float ca, float cb, float cc, bool last, float out_scale, bool trans,
+                      hipStream_t st) {
+  const int mt = tiles_of(m), nt = tiles_of(n);
+  if (int rc = launch_ns<kNsA>({x, x, nullptr, a, n, m, m, BE, mt, mt, 0.0f, 1.0f, 0, 0}, st,
+                               "newton_schulz5(X X^T)"))
+    return rc;
+  if (int rc = launch_ns<kNsB>({a, a, a, b, m, m, m, BE, mt, mt, cb, cc, 0, 0}, st,
+                               "newton_schulz5(B)"))
+    return rc;
+  return launch_ns<kNsX>({x, b, x, xn, m, n, m, BE, nt, mt, ca, out_scale, last ? 1 : 0,
+                          last && trans ? 1 : 0},
+                         st, "newton_schulz5(B X)");
 }
 
 }  // namespace uttt

@@ -39,4 +39,11 @@ int launch_wg192(const Wg192Plan& plan, const void* dy, const void* k, const voi
                  const void* v, void* dw0_w2, void* dw1, const int32_t* gs, int B, int E, int I,
                  int D, int N, void* workspace, hipStream_t st, const char* what);
 
+// One Newton-Schulz step of BE matrices x [m, n] (m <= n): a [m, m] = x x^T,
+// b [m, m] = cb a + (cc a) a, xn [m, n] = ca x + b x; `last`: xn times
+// out_scale, as [n, m] with `trans`.
+int launch_ns192_step(const uint16_t* x, uint16_t* a, uint16_t* b, uint16_t* xn, int BE, int m,
+                      int n, float ca, float cb, float cc, bool last, float out_scale, bool trans,
+                      hipStream_t st);
+
 }  // namespace uttt
