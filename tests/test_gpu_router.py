@@ -231,3 +231,44 @@ def test_route_tokens_map_src_rows_refused_where_the_row_map_takes_more_launches
     assert not RT.src_rows_supported(5000, 16)
     with pytest.raises(RuntimeError, match="src_rows"):
         RT.route_tokens_map(x, Rw, 2, with_src_rows=True)
+
+
+@pytest.mark.parametrize("B,T,D,E,k", [
+    (2, 9, 192, 48, 1),        # the smallest batch off the few-token path
+    (1, 65, 40, 5, 3),         # one token past a block, a tail of 8 features
+    (3, 130, 256, 128, 4),     # every expert block, the widest of the narrow rows
+    (2, 100, 8, 33, 33),       # one chunk of one lane group, all experts selected
+    (1, 12289, 264, 17, 2),    # many tokens of wider rows: three groups of features
+])
+@pytest.mark.parametrize("rt", ["softmax", "norm_softmax", "norm_relu"])
+def test_route_tokens_wide(B, T, D, E, k, rt):
+    """The token-column router kernel (narrow rows, or 12 288 tokens and more):
+    logits against fp64 (three exact bf16 products per weight and fp32 sums of
+    at most D terms: D * 2^-24 of sum |x||w|), the selection on the kernel's own
+    logits against the oracle's, group sizes and balance sums; -inf biases
+    exclude experts."""
+    g = torch.Generator().manual_seed(B * 1000 + T + E)
+    x = torch.randn(B, T, D, generator=g)
+    x = (x / x.norm(dim=-1, keepdim=True)).to(torch.bfloat16)
+    Rw = torch.randn(B, E, D, generator=g)
+    bias = torch.randn(1, E, 1, generator=g) * 0.5
+    if k < E:
+        bias[0, E // 2] = -float("inf")
+    kw = dict(router_type=rt, combine_mode="topk_renorm" if k > 1 else "selected_prob", alpha=0.8)
+    mask, gs, comb, bal, lg = RT.route_tokens(x.to(DEV), Rw.to(DEV), k, routing_bias=bias.to(DEV),
+                                              return_logits=True, **kw)
+    x64, r64 = x.double(), Rw.double()
+    ref64 = r64 @ x64.transpose(1, 2)
+    bound = D * 2.0 ** -24 * (r64.abs() @ x64.abs().transpose(1, 2)) + 1e-30
+    assert bool(((lg.cpu().double() - ref64).abs() <= bound).all())
+    ref = OR.create_router_mask_sizes_probs(lg.cpu(), k, routing_bias=bias, **kw)
+    if rt == "softmax":
+        assert torch.equal(mask.cpu(), ref[0]) and torch.equal(gs.cpu(), ref[1])
+    assert torch.equal(gs, mask.sum(-1, dtype=torch.int32))
+    assert bool((mask.sum(1) == k).all())
+    same = (mask.cpu() == ref[0]).all(1, keepdim=True).expand_as(ref[2])
+    assert same.float().mean().item() >= 0.99          # near ties of the normalised scores
+    torch.testing.assert_close(comb.cpu()[same], ref[2][same], rtol=1e-5, atol=1e-7)
+    torch.testing.assert_close(bal.cpu(), ref[3], rtol=1e-5, atol=1e-7)
+    _, _, _, _, bsum = RT.route_tokens_lb(x.to(DEV), Rw.to(DEV), k, routing_bias=bias.to(DEV), **kw)
+    torch.testing.assert_close(bsum.cpu(), bal.cpu().double().sum(-1).float(), rtol=1e-5, atol=1e-5)

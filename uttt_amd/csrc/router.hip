@@ -19,6 +19,8 @@
 //   freq_e = mean_b(group_sizes) / sum_e mean_b(group_sizes).
 //
 // Kernels:
+//   router_wide_kernel   : the same for narrow rows or many tokens, a token's
+//                          logits in the registers of four lanes;
 //   router_select_kernel : one thread per token, logits given ([B,E,T] strided);
 //   router_mfma_kernel   : logits = R x^T for 32 tokens x all experts per
 //                          workgroup (fp32 matrix cores, the waves splitting
@@ -722,6 +724,344 @@ __global__ __launch_bounds__(NW * kWave) void router_mfma_kernel(
   }
 }
 
+// Fused router for narrow rows: the same logits and selection as
+// router_mfma_kernel with the roles of the MFMA operands exchanged.  A wave
+// multiplies the weights of all experts (NE blocks of 16 rows, A operand of
+// v_mfma_f32_16x16x32_bf16) with blocks of 16 tokens (B operand), so accumulator
+// v of lane l is expert 16 j + 4 (l / 16) + v of token l % 16: a token's logits
+// sit in the registers of four lanes, its selection runs there with two
+// exchanges per reduction, and every output store covers 16 consecutive tokens
+// of four experts.  router_mfma_kernel spreads a token over 32 lanes (five
+// exchanges per reduction), pads the experts to 32 and stores 4 bytes per expert
+// row and token, which is most of its time where the dot products are short.
+// The weights are split exactly
+// into three bf16 parts by truncation (8 + 8 + 8 mantissa bits) once per wave
+// and 32 features.  The high parts' products accumulate in groups of 128
+// features that are added to the total, the other two parts' apart from them, so
+// the logits' error stays that of router_mfma_kernel's split over waves.
+constexpr int kWideWaves = 4;
+constexpr int kWideBlocks = 1;  // token blocks per wave (two: 16 384 tokens 12.2 -> 15.6 us,
+                                // 196 608 tokens 59 -> 56)
+constexpr int kWideGroup = 4;   // 32-feature chunks per group
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// Sum over the 16 lanes of a row (in every lane), DPP adds in a fixed order.
+template <int CTRL, class V>
+__device__ __forceinline__ V row_dpp(V v) {
+  return __builtin_bit_cast(
+      V, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+template <class V>
+__device__ __forceinline__ V row_sum(V v) {
+  v += row_dpp<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  v += row_dpp<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  v += row_dpp<0x141>(v);  // row_half_mirror
+  v += row_dpp<0x140>(v);  // row_mirror
+  return v;
+}
+// Sum and maximum over the four lanes of one token.
+__device__ __forceinline__ float tok_sum(float v) {
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+__device__ __forceinline__ float tok_max(float v) {
+  v = fmaxf(v, __shfl_xor(v, 16, 64));
+  return fmaxf(v, __shfl_xor(v, 32, 64));
+}
+// The high 16 bits of two words as one (a in the low half).
+__device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x07060302u);
+}
+
+template <int NE>
+__global__ __launch_bounds__(kWideWaves* kWave) void router_wide_kernel(
+    const uint16_t* __restrict__ x, const float* __restrict__ rw, int64_t w_sb, int D,
+    float* __restrict__ logits_out, SelectArgs a) {
+  constexpr int EB = NE * 16, NB = kWideBlocks;
+  __shared__ uint4 wparts[2][3][NE][64];  // [buffer][part][expert block][lane]
+  __shared__ float sbal[kWideWaves][EB];
+  __shared__ int scnt[kWideWaves][EB];
+  const int blk = blockIdx.x, b = blockIdx.y;
+  const int w = threadIdx.x / kWave, lane = lane_id();
+  const int r = lane % 16, h = lane / 16;
+  const int t0 = (blk * kWideWaves + w) * 16 * NB;
+  const int E = a.E, T = a.T;
+  const float* R = rw + (int64_t)b * w_sb;
+  auto expert = [&](int j, int v) __attribute__((always_inline)) { return 16 * j + 4 * h + v; };
+  // the routing bias of this lane's experts (from a valid address without a bias)
+  float bias_v[NE][4];
+  {
+    const float* bp = a.bias != nullptr ? a.bias + (int64_t)b * a.bias_sb : R;
+#pragma unroll
+    for (int j = 0; j < NE; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int e = expert(j, v);
+        const float f = bp[e < E ? e : 0];
+        bias_v[j][v] = a.bias != nullptr && e < E ? f : 0.0f;
+      }
+  }
+
+  // ---- logits: 32 features per step, the loads two steps ahead in flight.  Each
+  // wave splits its share of the expert blocks (w, w + kWideWaves, ...) and all
+  // waves read the parts from LDS; two buffers, so one barrier per step.
+  f32x4_t hi_acc[NE][NB], rest[NE][NB], total[NE][NB];
+#pragma unroll
+  for (int j = 0; j < NE; ++j)
+#pragma unroll
+    for (int n = 0; n < NB; ++n) hi_acc[j][n] = rest[j][n] = total[j][n] = f32x4_t{};
+  const uint16_t* xrow[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n)  // rows past T repeat the last one (never stored)
+    xrow[n] = x + ((int64_t)b * T + min(t0 + 16 * n + r, T - 1)) * D;
+  constexpr int NJ = (NE + kWideWaves - 1) / kWideWaves;
+  const float* wrow[NJ];
+#pragma unroll
+  for (int q = 0; q < NJ; ++q)
+    wrow[q] = R + (int64_t)min(16 * (w + kWideWaves * q) + r, E - 1) * D;
+  const int nch = (D + 31) / 32;
+  struct Chunk {
+    uint4 xv[NB];
+    float4 wv[NJ][2];
+  };
+  // features past D are read from the row's start and replaced by zeros in
+  // both operands
+  auto fetch = [&](int c, Chunk& q) __attribute__((always_inline)) {
+    const int d = 32 * min(c, nch - 1) + 8 * h;
+    const int dd = d + 8 <= D ? d : 0;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) q.xv[n] = *reinterpret_cast<const uint4*>(xrow[n] + dd);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      q.wv[j][0] = *reinterpret_cast<const float4*>(wrow[j] + dd);
+      q.wv[j][1] = *reinterpret_cast<const float4*>(wrow[j] + dd + 4);
+    }
+  };
+  auto step = [&](int c, const Chunk& q) __attribute__((always_inline)) {
+    const uint32_t in = 32 * c + 8 * h + 8 <= D ? 0xffffffffu : 0u;
+    uint4(*parts)[NE][64] = wparts[c & 1];
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj) {
+      const int j = w + kWideWaves * jj;
+      if (j < NE) {  // wave-uniform
+        const float4 p = q.wv[jj][0], s = q.wv[jj][1];
+        const float wf[8] = {p.x, p.y, p.z, p.w, s.x, s.y, s.z, s.w};
+        uint32_t hi[4], mid[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          uint32_t f[2], m[2], l[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            f[u] = __float_as_uint(wf[2 * i + u]) & in;
+            const float r1 = __uint_as_float(f[u]) - __uint_as_float(f[u] & 0xffff0000u);
+            m[u] = __float_as_uint(r1);
+            l[u] = __float_as_uint(r1 - __uint_as_float(m[u] & 0xffff0000u));
+          }
+          hi[i] = high_halves(f[0], f[1]);
+          mid[i] = high_halves(m[0], m[1]);
+          lo[i] = high_halves(l[0], l[1]);
+        }
+        parts[0][j][lane] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        parts[1][j][lane] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
+        parts[2][j][lane] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+      }
+    }
+    bf16x8_t xb[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      const uint4 u = q.xv[n];
+      xb[n] = __builtin_bit_cast(bf16x8_t, make_uint4(u.x & in, u.y & in, u.z & in, u.w & in));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+      const bf16x8_t fh = __builtin_bit_cast(bf16x8_t, parts[0][j][lane]);
+      const bf16x8_t fm = __builtin_bit_cast(bf16x8_t, parts[1][j][lane]);
+      const bf16x8_t fl = __builtin_bit_cast(bf16x8_t, parts[2][j][lane]);
+#pragma unroll
+      for (int n = 0; n < NB; ++n) {
+        hi_acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh, xb[n], hi_acc[j][n], 0, 0, 0);
+        rest[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fm, xb[n], rest[j][n], 0, 0, 0);
+        rest[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl, xb[n], rest[j][n], 0, 0, 0);
+      }
+    }
+    if ((c + 1) % kWideGroup == 0 || c + 1 == nch) {
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+          total[j][n] += hi_acc[j][n];
+          hi_acc[j][n] = f32x4_t{};
+        }
+    }
+  };
+  Chunk ring[3];
+  fetch(0, ring[0]);
+  fetch(1, ring[1]);
+  for (int c = 0; c < nch; c += 3) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      if (c + u < nch) {  // uniform over the workgroup
+        fetch(c + u + 2, ring[(u + 2) % 3]);
+        step(c + u, ring[u]);
+      }
+    }
+  }
+
+  // ---- selection
+  float bsum[NE][4];
+  uint32_t csum[NE];  // counts of a lane's 4 experts of a block, a byte each
+  static_assert(16 * NB <= 255, "a count fits its byte");
+#pragma unroll
+  for (int j = 0; j < NE; ++j) {
+    csum[j] = 0u;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) bsum[j][v] = 0.0f;
+  }
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+    const int t = t0 + 16 * n + r;
+    const bool live = t < T;
+    const int64_t base = (int64_t)b * E * T + t;
+    float val[NE][4];
+#pragma unroll
+    for (int j = 0; j < NE; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int e = expert(j, v);
+        val[j][v] = e < E ? total[j][n][v] + rest[j][n][v] : 0.0f;
+        if (logits_out != nullptr && live && e < E) logits_out[base + (int64_t)e * T] = val[j][v];
+      }
+    if (a.router_type != 0) {  // val <- selection scores
+      float ss = 0.0f;
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) ss += val[j][v] * val[j][v];
+      const float nrm = fmaxf(sqrtf(tok_sum(ss)), a.norm_eps);
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float z = val[j][v] / nrm;
+          val[j][v] = expert(j, v) < E ? (a.router_type == 1 ? z : fmaxf(z, 0.0f)) * a.scale : 0.0f;
+        }
+    }
+    // top-k of score + bias: k arg-max passes, equal scores to the lower expert
+    uint32_t sel = 0u;  // bit 4 j + v
+    for (int k = 0; k < a.topk; ++k) {
+      float bv = -INFINITY;
+      int bi = 0x7fffffff;  // no candidate
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int e = expert(j, v);
+          const float s = a.bias != nullptr ? val[j][v] + bias_v[j][v] : val[j][v];
+          const bool cand =
+              e < E && !((sel >> (4 * j + v)) & 1u) && (bi == 0x7fffffff || s > bv);
+          bv = cand ? s : bv;
+          bi = cand ? e : bi;
+        }
+#pragma unroll
+      for (int o = 16; o <= 32; o *= 2) {
+        const float ov = __shfl_xor(bv, o, 64);
+        const int oi = __shfl_xor(bi, o, 64);
+        if (ov > bv || (ov == bv && oi < bi)) {
+          bv = ov;
+          bi = oi;
+        }
+      }
+      if (bi < E && ((bi >> 2) & 3) == h) sel |= 1u << (4 * (bi >> 4) + (bi & 3));
+    }
+    // balance probabilities in place of the scores
+    if (a.router_type == 2) {
+      float s = 0.0f;
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) s += val[j][v];
+      s = tok_sum(s);
+      const float den = fmaxf(s, 1e-9f);
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) val[j][v] = s > 0.0f ? val[j][v] / den : 1.0f / (float)E;
+    } else {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (expert(j, v) < E) mx = fmaxf(mx, val[j][v]);
+      mx = tok_max(mx);
+      float s = 0.0f;
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          val[j][v] = expert(j, v) < E ? expf(val[j][v] - mx) : 0.0f;
+          s += val[j][v];
+        }
+      s = tok_sum(s);
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) val[j][v] = val[j][v] / s;
+    }
+    float rsum = 0.0f;
+    if (a.combine_mode == 1) {
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) rsum += (sel >> (4 * j + v)) & 1u ? val[j][v] : 0.0f;
+      rsum = tok_sum(rsum);
+    }
+    const float rden = fmaxf(rsum, 1e-9f);
+#pragma unroll
+    for (int j = 0; j < NE; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int e = expert(j, v);
+        const bool on = (sel >> (4 * j + v)) & 1u;
+        if (live && e < E) {
+          const int64_t i = base + (int64_t)e * T;
+          a.mask[i] = on ? 1 : 0;
+          a.balance[i] = val[j][v];
+          const float c = a.combine_mode == 1 ? (on ? val[j][v] : 0.0f) / rden : val[j][v];
+          a.combine[i] = c * a.alpha;
+        }
+        bsum[j][v] += live ? val[j][v] : 0.0f;
+        csum[j] += (live && on ? 1u : 0u) << (8 * v);
+      }
+  }
+  // ---- the block's sums: a fixed tree over the 16 token lanes, then the waves
+#pragma unroll
+  for (int j = 0; j < NE; ++j) {
+    const uint32_t c = row_sum(csum[j]);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float s = row_sum(bsum[j][v]);
+      if (r == 0) {
+        sbal[w][expert(j, v)] = s;
+        scnt[w][expert(j, v)] = (int)((c >> (8 * v)) & 255u);
+      }
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  for (int e = threadIdx.x; e < E; e += kWideWaves * kWave) {
+    float s = sbal[0][e];
+    int c = scnt[0][e];
+#pragma unroll
+    for (int q = 1; q < kWideWaves; ++q) {
+      s += sbal[q][e];
+      c += scnt[q][e];
+    }
+    put_partial(a, b, blk, e, s, c);
+  }
+}
+
 // group_sizes[b][e] and the balance sum of (b, e) over the select blocks:
 // one workgroup per (b, e); thread i adds blocks i, i + 256, ... in order, then
 // a fixed tree over the 256 thread sums (deterministic).
@@ -860,12 +1200,49 @@ int finish(const Ws& w, int B, int E, int T, int32_t* group_sizes, float* lb_los
   return check_launch(what);
 }
 
-// The fused logits + selection launch of route_tokens (nblk blocks of 32
-// tokens per batch).
+// rows of whole 16-byte vectors: every feature load is one unconditional vector load
+bool route_vec(const void* x, const float* router_w, int64_t w_sb, int D) {
+  return D % 8 == 0 && w_sb % 4 == 0 &&
+         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(router_w)) & 15u) == 0;
+}
+
+// Tokens per block of the fused logits + selection launch: 32
+// (router_mfma_kernel, whose waves share a token block's features) or
+// router_wide_kernel's.  The latter for bf16 rows of at most 256 features (E =
+// 48, D = 192: 800 tokens 11.8 -> 10.8 us, 16 384 tokens 22.7 -> 12.2, 196 608
+// tokens 232 -> 59), whose few steps a wave runs by itself, and from 12 288
+// tokens on, where its waves fill the chip: 16 384 tokens of 384 features and 96
+// experts 30.7 -> 24.4 us (6000: 19.7 / 22.0), 24 576 of 768 and 16 24.5 ->
+// 17.0 (2048: 11.8 / 14.0), 49 152 of 1536 and 32 76 -> 51 (2048: 15.4 / 27).
+int route_block_tokens(const void* x, int x_dtype, const float* router_w, int64_t w_sb, int B,
+                       int T, int D) {
+  const bool wide = x_dtype == UTTT_BF16 && T > kSmallT && route_vec(x, router_w, w_sb, D) &&
+                    (D <= 256 || (int64_t)B * T >= 12288);
+  return wide ? kWideWaves * 16 * kWideBlocks : 32;
+}
+
+// The fused logits + selection launch of route_tokens (nblk blocks of
+// blk_tokens tokens per batch).
 int launch_route_kernel(const void* x, int x_dtype, const float* router_w, int64_t w_sb, int B,
-                        int T, int D, int E, int nblk, const SelectArgs& a, float* logits_out,
-                        hipStream_t st) {
+                        int T, int D, int E, int nblk, int blk_tokens, const SelectArgs& a,
+                        float* logits_out, hipStream_t st) {
+  const bool wide = blk_tokens != 32;
   const int net = (E + 31) / 32;
+  if (wide) {
+#define UTTT_WIDE_LAUNCH(NE)                                                             \
+  hipLaunchKernelGGL((router_wide_kernel<NE>), dim3(nblk, B), dim3(kWideWaves * kWave), 0, \
+                     st, static_cast<const uint16_t*>(x), router_w, w_sb, D, logits_out, a)
+    switch ((E + 15) / 16) {
+      case 1: UTTT_WIDE_LAUNCH(1); break;
+      case 2: UTTT_WIDE_LAUNCH(2); break;
+      case 3: UTTT_WIDE_LAUNCH(3); break;
+      case 4: UTTT_WIDE_LAUNCH(4); break;
+      case 5: case 6: UTTT_WIDE_LAUNCH(6); break;
+      default: UTTT_WIDE_LAUNCH(8); break;
+    }
+#undef UTTT_WIDE_LAUNCH
+    return check_launch("route_tokens");
+  }
 #define UTTT_ROUTE_LAUNCH(NET, NW, SMALL)                                                       \
   if (vec)                                                                                      \
     hipLaunchKernelGGL((router_mfma_kernel<XT, NET, NW, SMALL, true>), dim3(nblk, B),          \
@@ -877,9 +1254,7 @@ int launch_route_kernel(const void* x, int x_dtype, const float* router_w, int64
                        logits_out, a)
   // a few tokens per batch (generation): vector-ALU logits, no padded MFMA rows
   const bool small = T <= kSmallT;
-  // rows of whole 16-byte vectors: every feature load is one unconditional vector load
-  const bool vec = D % 8 == 0 && w_sb % 4 == 0 &&
-                   ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(router_w)) & 15u) == 0;
+  const bool vec = route_vec(x, router_w, w_sb, D);
   UTTT_DTYPE_SWITCH_LR(x_dtype, XT, {
     using S = typename XT::S;
     switch (net) {
@@ -946,7 +1321,9 @@ extern "C" int uttt_route_tokens(const void* x, int x_dtype, const float* router
   UTTT_REQUIRE(D >= 1, "route_tokens: D=%d", D);
   if (B == 0 || T == 0) return UTTT_OK;
   UTTT_REQUIRE(x && router_w && mask && combine && balance, "route_tokens: null pointer");
-  Ws w = ws_layout(workspace, B, T, E, 32);
+  // the workspace query assumes blocks of 32 tokens: larger ones need less
+  const int blk_tokens = route_block_tokens(x, x_dtype, router_w, w_sb, B, T, D);
+  Ws w = ws_layout(workspace, B, T, E, blk_tokens);
   UTTT_REQUIRE(workspace != nullptr && workspace_bytes >= w.bytes,
                "route_tokens: workspace %zu < %zu bytes", workspace_bytes, w.bytes);
   if (balance_sum != nullptr) w.bal_sum = balance_sum;
@@ -954,8 +1331,8 @@ extern "C" int uttt_route_tokens(const void* x, int x_dtype, const float* router
                                  alpha, router_scale, norm_eps, mask, combine, balance,
                                  group_sizes);
   hipStream_t st = as_stream(stream);
-  if (int rc = launch_route_kernel(x, x_dtype, router_w, w_sb, B, T, D, E, w.nblk, a, logits_out,
-                                   st))
+  if (int rc = launch_route_kernel(x, x_dtype, router_w, w_sb, B, T, D, E, w.nblk, blk_tokens, a,
+                                   logits_out, st))
     return rc;
   return finish(w, B, E, T, group_sizes, lb_loss, st, "route_tokens");
 }
@@ -990,7 +1367,8 @@ extern "C" int uttt_route_tokens_map(const void* x, int x_dtype, const float* ro
   UTTT_REQUIRE(x && router_w && mask && combine && balance && group_sizes && balance_sum &&
                    row_id_map,
                "route_tokens_map: null pointer");
-  Ws w = ws_layout(workspace, B, T, E, 32);
+  const int blk_tokens = route_block_tokens(x, x_dtype, router_w, w_sb, B, T, D);
+  Ws w = ws_layout(workspace, B, T, E, blk_tokens);
   const size_t rm_off = align256(w.bytes);
   const size_t need = rm_off + uttt_row_id_map_workspace_bytes(B, T, E);
   UTTT_REQUIRE(workspace != nullptr && workspace_bytes >= need,
@@ -1000,8 +1378,8 @@ extern "C" int uttt_route_tokens_map(const void* x, int x_dtype, const float* ro
                                  alpha, router_scale, norm_eps, mask, combine, balance,
                                  group_sizes);
   hipStream_t st = as_stream(stream);
-  if (int rc = launch_route_kernel(x, x_dtype, router_w, w_sb, B, T, D, E, w.nblk, a, nullptr,
-                                   st))
+  if (int rc = launch_route_kernel(x, x_dtype, router_w, w_sb, B, T, D, E, w.nblk, blk_tokens, a,
+                                   nullptr, st))
     return rc;
   // the one-launch row map also adds the selection blocks' balance partials
   // (group sizes are its own counts), so no reduce launch runs
