@@ -264,3 +264,33 @@ def test_permute_roundtrip_full_size_property():
     xp, _, rm = TP.permute_with_expert_mask(x, mask.to(DEV), comb.to(DEV), k)
     back = TP.unpermute_and_merge_with_probs(xp, rm, comb.to(DEV))
     torch.testing.assert_close(back.float(), x.float(), rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("T,E", [(1, 25), (63, 64), (64, 65), (65, 128), (129, 33), (4112, 48),
+                                 (5000, 96), (70001, 27)])
+@pytest.mark.parametrize("form", ["bool", "uint8_values", "int32", "token_major"])
+def test_row_map_from_64_token_tiles(T, E, form):
+    """The general row map (E > 24, or too many tokens for one launch): every
+    mask form it accepts, tokens with none to all experts, experts with no
+    token; bit-exact, with the group sizes."""
+    B = 2
+    g = torch.Generator().manual_seed(T * 131 + E)
+    n = torch.randint(0, 4, (B, 1, T), generator=g)
+    if T > 2:
+        n[:, :, 1] = E                                   # a token with every expert
+    rank = torch.rand(B, E, T, generator=g).argsort(1).argsort(1)
+    mask = rank < n
+    mask[1, E // 2] = False
+    ref = OP.make_row_id_map(mask)
+    if form == "bool":
+        m = mask.to(DEV)
+    elif form == "uint8_values":
+        m = (mask.to(torch.uint8) * torch.randint(1, 256, mask.shape, generator=g).to(torch.uint8)).to(DEV)
+    elif form == "int32":
+        m = (mask.to(torch.int32) * 256).to(DEV)
+    else:
+        m = mask.to(DEV).transpose(1, 2).contiguous().transpose(1, 2)
+    gs = torch.empty(B, E, dtype=torch.int32, device=DEV)
+    rm = TP.make_row_id_map(m, B, T, E, group_sizes=gs)
+    assert torch.equal(rm.cpu(), ref)
+    assert torch.equal(gs.cpu(), mask.sum(-1).to(torch.int32))

@@ -272,3 +272,27 @@ def test_route_tokens_wide(B, T, D, E, k, rt):
     torch.testing.assert_close(bal.cpu(), ref[3], rtol=1e-5, atol=1e-7)
     _, _, _, _, bsum = RT.route_tokens_lb(x.to(DEV), Rw.to(DEV), k, routing_bias=bias.to(DEV), **kw)
     torch.testing.assert_close(bsum.cpu(), bal.cpu().double().sum(-1).float(), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("B,T,D,E,k", [
+    (2, 517, 768, 16, 2),      # blocks of 32 tokens, a ragged last tile
+    (1, 31, 768, 48, 1),       # one block per batch
+    (3, 4100, 192, 48, 1),     # blocks of 64 tokens
+    (1, 4128, 1536, 96, 3),    # more than 64 experts
+])
+def test_route_tokens_map_from_the_selection_counts(B, T, D, E, k):
+    """Shapes off the one-launch row map: the map built from the selection's
+    own counts equals make_row_id_map of the mask, with group sizes and balance
+    sums."""
+    g = torch.Generator().manual_seed(T + E)
+    x = torch.randn(B, T, D, generator=g)
+    x = (x / x.norm(dim=-1, keepdim=True)).to(torch.bfloat16).to(DEV)
+    Rw = torch.randn(E, D, generator=g).to(DEV)
+    mask, gs, comb, bal, bsum, rmap = RT.route_tokens_map(x, Rw, k, combine_mode="topk_renorm")
+    from oracle import permute as OP
+
+    assert torch.equal(rmap.cpu(), OP.make_row_id_map(mask.cpu()))
+    assert torch.equal(gs, mask.sum(-1, dtype=torch.int32))
+    torch.testing.assert_close(bsum.cpu(), bal.cpu().double().sum(-1).float(), rtol=1e-5, atol=1e-5)
+    m2, gs2, comb2, bal2 = RT.route_tokens(x, Rw, k, combine_mode="topk_renorm")
+    assert torch.equal(mask, m2) and torch.equal(gs, gs2) and torch.equal(comb, comb2)

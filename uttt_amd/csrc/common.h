@@ -33,6 +33,16 @@ bool launch_rowmap_fused(const uint8_t* mask, int64_t s_b, int64_t s_e, int B, i
                          int nblk_r, float* bal_sum, hipStream_t st, int32_t* src_rows = nullptr,
                          int64_t src_sb = 0);
 
+// The row map of a bool mask (token stride 1) whose per-tile expert counts
+// [B, ceil(T / tile_tokens), E] are known (tile_tokens 32 or 64), in two
+// launches; also group_sizes and, with part_bal [B, nblk, E], bal_sum [B, E] =
+// its sum over the blocks.  workspace: the offsets, as many entries as counts.
+int launch_rowmap_from_counts(const uint8_t* mask, int64_t s_b, int64_t s_e, int B, int T, int E,
+                              const int32_t* counts, int tile_tokens, void* workspace,
+                              int32_t* group_sizes, const float* part_bal, int nblk,
+                              float* bal_sum, int32_t* row_id_map, hipStream_t st,
+                              const char* what);
+
 // Newton-Schulz of BE small matrices [rows, cols] in one launch (one
 // workgroup per matrix, the whole computation in LDS; ns_small.hip), for the
 // shapes ns_small_fits accepts; g fp32 or bf16 (g_dtype), 16-byte aligned.

@@ -3,17 +3,13 @@
 // Row map (reference: make_row_id_map, L/triton_permute.py:283-393).  The
 // destination of (token t, expert e) is row(e, t) = off_e + rank(e, t): the
 // permuted buffer is expert-major and token-ascending.  For E <= 24 two
-// launches (count, then rowmap_scan_emit_kernel, which derives each tile's
-// offsets from the counts itself); else three:
-//   count : one workgroup per 256-token tile; each wave ballots the 0/1 mask
-//           of every expert and the per-tile counts go to a [B, E, tiles]
-//           table (expert-major, so the global order is a linear scan);
-//   scan  : one workgroup per batch does the exclusive prefix over that table
-//           (it also yields group_sizes);
-//   emit  : re-ballots the tile's mask, ranks each routed token inside its
-//           wave with popcount, and writes the packed per-token entry in the
-//           reference format (rows and experts in descending order, n_routed
-//           last, the reference's stale values in columns [n, E)).
+// launches (count per 256-token tile, then rowmap_scan_emit_kernel, which
+// derives each tile's offsets from the counts itself); else three over 64-token
+// tiles: rowmap_count64_kernel, rowmap_offsets_kernel (also group_sizes),
+// rowmap_emit64_kernel; after a router, whose selection leaves the counts, the
+// last two.  The packed per-token entry has the reference's format (rows and
+// experts in descending order, n_routed last, the reference's stale values in
+// columns [n, E)).
 // No atomics are used, so the result is deterministic by construction.
 // Short batches of a contiguous bool mask (T <= 4096, E <= 64: one apply's
 // routing) take one launch instead (rowmap_fused_kernel): each workgroup
@@ -117,91 +113,27 @@ __host__ __device__ __forceinline__ int padded_experts(int E) {
   return p;
 }
 
-// EP > 0: the count table is tile-major, [B, tiles, EP] with EP =
-// padded_experts(E) (read by rowmap_scan_emit_kernel<MB, EP>), else
-// expert-major, [B, E, tiles] (rowmap_scan_kernel).
-template <int MB, int EP = 0>
+// The count table of rowmap_scan_emit_kernel<MB, EP>: [B, tiles, EP] with EP =
+// padded_experts(E).
+template <int MB, int EP>
 __global__ __launch_bounds__(kTile) void rowmap_count_kernel(
     const void* map, int64_t s_b, int64_t s_e, int64_t s_t, int T, int E, int ntiles,
     int32_t* counts) {
-  constexpr bool TM = EP > 0;
-  constexpr int NMAX = TM ? EP : kMaxExperts;
   __shared__ int wcnt[kTile / kWave][kMaxExperts];
   const int tile = blockIdx.x, b = blockIdx.y;
   const int t = tile * kTile + threadIdx.x;
   const int64_t base = (int64_t)b * s_b + (int64_t)min(t, T - 1) * s_t;
   uint32_t bits[kMaxExperts / 32];
-  load_mask_bits<MB, NMAX>(map, base, s_e, E, t < T, bits);
-  wave_counts<NMAX>(bits, E, wcnt);
+  load_mask_bits<MB, EP>(map, base, s_e, E, t < T, bits);
+  wave_counts<EP>(bits, E, wcnt);
   __syncthreads();
-  const int Ep = TM ? EP : E;
-  for (int e = threadIdx.x; e < Ep; e += kTile) {
+  for (int e = threadIdx.x; e < EP; e += kTile) {
     int c = 0;
     if (e < E) {
 #pragma unroll
       for (int i = 0; i < kTile / kWave; ++i) c += wcnt[i][e];
     }
-    counts[TM ? ((int64_t)b * ntiles + tile) * Ep + e : ((int64_t)b * E + e) * ntiles + tile] = c;
-  }
-}
-
-// Exclusive scan of counts[b] (E * ntiles entries, expert-major) in place.
-constexpr int kScanThreads = 1024;
-constexpr int kScanPer = 4;
-
-__global__ __launch_bounds__(kScanThreads) void rowmap_scan_kernel(int32_t* counts, int E,
-                                                                   int ntiles,
-                                                                   int32_t* group_sizes) {
-  __shared__ int wave_tot[kScanThreads / kWave];
-  __shared__ int expert_start[kMaxExperts + 1];
-  __shared__ int carry_s;
-  const int b = blockIdx.x;
-  const int n = E * ntiles;
-  int32_t* c = counts + (int64_t)b * n;
-  const int tid = threadIdx.x, w = tid / kWave, lane = lane_id();
-  if (tid == 0) carry_s = 0;
-  __syncthreads();
-  for (int base = 0; base < n; base += kScanThreads * kScanPer) {
-    int v[kScanPer];
-    int sum = 0;
-#pragma unroll
-    for (int i = 0; i < kScanPer; ++i) {
-      int idx = base + tid * kScanPer + i;
-      v[i] = idx < n ? c[idx] : 0;
-      sum += v[i];
-    }
-    // inclusive scan of per-thread sums across the wave
-    int incl = sum;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      int o = __shfl_up(incl, d, kWave);
-      if (lane >= d) incl += o;
-    }
-    if (lane == kWave - 1) wave_tot[w] = incl;
-    __syncthreads();
-    int wave_off = 0;
-    for (int i = 0; i < w; ++i) wave_off += wave_tot[i];
-    int block_tot = 0;
-    for (int i = 0; i < kScanThreads / kWave; ++i) block_tot += wave_tot[i];
-    int run = carry_s + wave_off + incl - sum;  // exclusive prefix of this thread
-#pragma unroll
-    for (int i = 0; i < kScanPer; ++i) {
-      int idx = base + tid * kScanPer + i;
-      if (idx < n) {
-        c[idx] = run;
-        if (idx % ntiles == 0) expert_start[idx / ntiles] = run;
-      }
-      run += v[i];
-    }
-    __syncthreads();
-    if (tid == 0) carry_s += block_tot;
-    __syncthreads();
-  }
-  if (tid == 0) expert_start[E] = carry_s;
-  __syncthreads();
-  if (group_sizes != nullptr) {
-    for (int e = tid; e < E; e += kScanThreads)
-      group_sizes[(int64_t)b * E + e] = expert_start[e + 1] - expert_start[e];
+    counts[((int64_t)b * ntiles + tile) * EP + e] = c;
   }
 }
 
@@ -209,7 +141,6 @@ __global__ __launch_bounds__(kScanThreads) void rowmap_scan_kernel(int32_t* coun
 // output) are assembled in LDS and written out with consecutive lanes on
 // consecutive words; without it each lane stores its own entry directly,
 // which strides the lanes 4 * (2E+1) bytes apart.
-constexpr int kStageMaxW = 57;  // STAGE: kTile * (2E+1) * 4 bytes plus the 6.5 KiB of tables <= 64 KiB
 
 // Packed entries of one 256-token tile, given its tokens' selection bits, the
 // per-wave counts (wcnt) and selection ballots (wmask) of the tile and each
@@ -270,24 +201,235 @@ __device__ __forceinline__ void emit_tile(const uint32_t bits[kMaxExperts / 32],
   }
 }
 
-template <int MB, bool STAGE>
-__global__ __launch_bounds__(kTile) void rowmap_emit_kernel(
-    const void* map, int64_t s_b, int64_t s_e, int64_t s_t, int T, int E, int ntiles,
-    const int32_t* offsets, int32_t* row_id_map) {
-  extern __shared__ int32_t stage[];
-  __shared__ int wcnt[kTile / kWave][kMaxExperts];
-  __shared__ uint64_t wmask[kTile / kWave][kMaxExperts];
-  __shared__ int toff[kMaxExperts];
-  const int tile = blockIdx.x, b = blockIdx.y;
-  const int t = tile * kTile + threadIdx.x;
-  const int64_t base = (int64_t)b * s_b + (int64_t)min(t, T - 1) * s_t;
-  uint32_t bits[kMaxExperts / 32];
-  load_mask_bits<MB>(map, base, s_e, E, t < T, bits);
-  wave_counts(bits, E, wcnt, wmask);
-  for (int e = threadIdx.x; e < E; e += kTile)
-    toff[e] = offsets[((int64_t)b * E + e) * ntiles + tile];
-  __syncthreads();
-  emit_tile<STAGE>(bits, T, E, tile, b, wcnt, wmask, toff, stage, row_id_map);
+// -------------------------------------------- row map from 64-token tiles ---
+// The general row map: per-tile expert counts ([B, tiles, E], from
+// rowmap_count64_kernel or a router's own selection), then rowmap_offsets_kernel
+// (each tile's first row per expert), then rowmap_emit64_kernel.  A lane stands
+// for an expert: it reads the 64 mask bytes of its expert's tokens and packs
+// them into one word, so no ballot runs per expert, and an entry of the map is
+// written by consecutive lanes on consecutive words whatever 2E + 1 is (a lane
+// per token wrote 4 bytes every 4 (2E + 1): 96 us at T = 196 608, E = 48, for 76 MB).
+constexpr int kTile64 = 64;
+constexpr int kExpertWords = kMaxExperts / kWave;  // experts per lane
+
+struct MaskView {
+  const void* map;
+  int64_t s_b, s_e, s_t;
+  int fast;  // bool mask, unit token stride, every tile's bytes 8-byte aligned
+};
+
+// The selection bits of the 64 tokens from t0 on (bit i = token t0 + i, 0 past
+// T) for the experts lane, lane + 64 of batch b.
+template <int MB>
+__device__ __forceinline__ void tile_bits(const MaskView& m, int b, int t0, int T, int E,
+                                          uint64_t (&bits)[kExpertWords]) {
+  const int lane = lane_id();
+#pragma unroll
+  for (int q = 0; q < kExpertWords; ++q) bits[q] = 0;
+  if (MB == 1 && m.fast && t0 + kTile64 <= T) {
+#pragma unroll
+    for (int q = 0; q < kExpertWords; ++q) {
+      if (64 * q >= E) break;  // wave-uniform
+      const int e = min(lane + 64 * q, E - 1);
+      const uint64_t* p = reinterpret_cast<const uint64_t*>(
+          static_cast<const uint8_t*>(m.map) + (int64_t)b * m.s_b + (int64_t)e * m.s_e + t0);
+      uint64_t w[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) w[i] = p[i];
+      uint64_t r = 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        // 1 in every nonzero byte, then the eight ones gathered in the top byte
+        constexpr uint64_t k7f = 0x7f7f7f7f7f7f7f7full;
+        const uint64_t one = ((((w[i] & k7f) + k7f) | w[i]) & ~k7f) >> 7;
+        r |= ((one * 0x0102040810204080ull) >> 56) << (8 * i);
+      }
+      bits[q] = lane + 64 * q < E ? r : 0;
+    }
+    return;
+  }
+  // any other mask: a lane per token, one ballot per expert
+  const int t = min(t0 + lane, T - 1);
+  const int64_t base = (int64_t)b * m.s_b + (int64_t)t * m.s_t;
+  for (int e0 = 0; e0 < E; e0 += 8) {
+    bool on[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) on[i] = mask_bit<MB>(m.map, base + (int64_t)min(e0 + i, E - 1) * m.s_e);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint64_t bal = __ballot(on[i] && t0 + lane < T && e0 + i < E);
+#pragma unroll
+      for (int q = 0; q < kExpertWords; ++q)
+        bits[q] = lane + 64 * q == e0 + i ? bal : bits[q];
+    }
+  }
+}
+
+// counts[b, tile, e]: one wave per tile.
+template <int MB>
+__global__ __launch_bounds__(kTile) void rowmap_count64_kernel(MaskView m, int T, int E,
+                                                               int ntiles, int32_t* counts) {
+  const int tile = blockIdx.x * (kTile / kWave) + threadIdx.x / kWave, b = blockIdx.y;
+  if (tile >= ntiles) return;
+  uint64_t bits[kExpertWords];
+  tile_bits<MB>(m, b, tile * kTile64, T, E, bits);
+#pragma unroll
+  for (int q = 0; q < kExpertWords; ++q) {
+    const int e = lane_id() + 64 * q;
+    if (e < E) counts[((int64_t)b * ntiles + tile) * E + e] = __popcll(bits[q]);
+  }
+}
+
+// offsets[b, tile, e] = row of tile `tile`'s first token of expert e: the rows
+// of the experts before e plus those of e's earlier tiles.  One workgroup per
+// (e, b): it adds the whole table's columns before e (all loads independent)
+// instead of waiting for another workgroup's total.  Also group_sizes[b, e],
+// and bal_sum[b, e] = the sum of a router's partials part_bal[b, blk, e] (thread
+// i adds blocks i, i + THREADS, ..., then a fixed tree).
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void rowmap_offsets_kernel(
+    const int32_t* __restrict__ counts, int E, int ntiles, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ group_sizes, const float* __restrict__ part_bal, int nblk,
+    float* __restrict__ bal_sum) {
+  __shared__ int wtot[THREADS / kWave];
+  __shared__ float fred[THREADS];
+  const int e = blockIdx.x, b = blockIdx.y;
+  const int tid = threadIdx.x, w = tid / kWave, lane = lane_id();
+  const int32_t* tab = counts + (int64_t)b * ntiles * E;
+  int32_t* out = offsets + (int64_t)b * ntiles * E;
+  // sum over the workgroup, in every thread
+  auto block_sum = [&](int v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+    __syncthreads();
+    if (lane == 0) wtot[w] = v;
+    __syncthreads();
+    int s = 0;
+#pragma unroll
+    for (int i = 0; i < THREADS / kWave; ++i) s += wtot[i];
+    return s;
+  };
+  int before = 0;
+  {
+    const int n = ntiles * E, stepmod = THREADS % E;
+    int col = tid % E;
+    constexpr int U = 16;
+    for (int i = tid; i < n; i += U * THREADS) {
+      int v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = tab[min(i + u * THREADS, n - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        before += i + u * THREADS < n && col < e ? v[u] : 0;
+        col += stepmod;
+        col -= col >= E ? E : 0;
+      }
+    }
+  }
+  int run = block_sum(before);
+  const int first = run;
+  for (int base = 0; base < ntiles; base += THREADS) {
+    const int t = base + tid;
+    const int v = t < ntiles ? tab[(int64_t)t * E + e] : 0;
+    int incl = v;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int o = __shfl_up(incl, d, kWave);
+      if (lane >= d) incl += o;
+    }
+    __syncthreads();
+    if (lane == kWave - 1) wtot[w] = incl;
+    __syncthreads();
+    int wo = 0, tot = 0;
+#pragma unroll
+    for (int i = 0; i < THREADS / kWave; ++i) {
+      wo += i < w ? wtot[i] : 0;
+      tot += wtot[i];
+    }
+    if (t < ntiles) out[(int64_t)t * E + e] = run + wo + incl - v;
+    run += tot;
+  }
+  if (tid == 0 && group_sizes != nullptr) group_sizes[(int64_t)b * E + e] = run - first;
+  if (part_bal != nullptr) {  // uniform
+    float f = 0.0f;
+    for (int k = tid; k < nblk; k += THREADS) f += part_bal[((int64_t)b * nblk + k) * E + e];
+    fred[tid] = f;
+    __syncthreads();
+    for (int o = THREADS / 2; o > 0; o >>= 1) {
+      if (tid < o) fred[tid] += fred[tid + o];
+      __syncthreads();
+    }
+    if (tid == 0) bal_sum[(int64_t)b * E + e] = fred[0];
+  }
+}
+
+// The map of one 64-token tile per workgroup, TPW tokens per wave (offsets in
+// tiles of `tt` = 32 or 64 tokens).  Per token, the lanes' routed flags are one
+// ballot per 64 experts: n and the experts come from it, the rows from the
+// lanes' running counters (Appendix format: rows and experts in descending
+// order, n at 2E, the row or -1 in columns [n, E), zeros in [E + n, 2E)).
+template <int MB, int TPW>
+__global__ __launch_bounds__(kTile64 / TPW * kWave) void rowmap_emit64_kernel(MaskView m, int T, int E, int tt,
+                                                              const int32_t* __restrict__ offsets,
+                                                              int32_t* __restrict__ row_id_map) {
+  constexpr int kPasses = (2 * kMaxExperts + 1 + kWave - 1) / kWave;
+  const int b = blockIdx.y, t0 = blockIdx.x * kTile64;
+  const int w = threadIdx.x / kWave, lane = lane_id();
+  const int first = TPW * w;                      // this wave's first token in the tile
+  if (t0 + first >= T) return;
+  const int W = 2 * E + 1;
+  uint64_t bits[kExpertWords];
+  tile_bits<MB>(m, b, t0, T, E, bits);
+  const int nt = (T + tt - 1) / tt;
+  const int toff = first / tt * tt;               // its offset tile's first token in the tile
+  int next[kExpertWords];
+#pragma unroll
+  for (int q = 0; q < kExpertWords; ++q) {
+    const int e = min(lane + 64 * q, E - 1);
+    const int off = offsets[((int64_t)b * nt + (t0 + toff) / tt) * E + e];
+    const uint64_t before = (bits[q] >> toff) & ((1ull << (first - toff)) - 1ull);
+    next[q] = off + __popcll(before);
+  }
+  for (int i = first; i < first + TPW && t0 + i < T; ++i) {
+    int32_t* row = row_id_map + ((int64_t)b * T + t0 + i) * W;
+    uint64_t sel[kExpertWords];
+    int r[kExpertWords];
+    int n = 0;
+#pragma unroll
+    for (int q = 0; q < kExpertWords; ++q) {
+      const bool on = (bits[q] >> i) & 1ull;
+      sel[q] = __ballot(on);
+      r[q] = on ? next[q] : -1;
+      next[q] += on ? 1 : 0;
+      n += __popcll(sel[q]);
+    }
+    int out[kPasses];
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      const int c = lane + 64 * p;
+      out[p] = p < kExpertWords && c < E ? r[p] : 0;  // columns past n of the row half
+      out[p] = c == 2 * E ? n : out[p];
+    }
+    int j = 0;
+#pragma unroll
+    for (int q = kExpertWords - 1; q >= 0; --q) {
+      uint64_t s = sel[q];
+      while (s != 0ull) {  // highest expert first; wave-uniform
+        const int eb = 63 - __clzll((long long)s);
+        s &= ~(1ull << eb);
+        const int rr = __builtin_amdgcn_readlane(r[q], eb);
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) {
+          const int c = lane + 64 * p;
+          out[p] = c == j ? rr : c == E + j ? 64 * q + eb : out[p];
+        }
+        ++j;
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p)
+      if (lane + 64 * p < W) row[lane + 64 * p] = out[p];
+  }
 }
 
 // Scan and emit in one launch (after rowmap_count_kernel<MB, EP>: two
@@ -1109,6 +1251,49 @@ int pick_ve(int H, std::initializer_list<const void*> ptrs) {
 
 }  // namespace
 
+namespace {
+MaskView mask_view(const void* map, int mask_bytes, int64_t s_b, int64_t s_e, int64_t s_t) {
+  const bool fast = mask_bytes == 1 && s_t == 1 && s_e % 8 == 0 && s_b % 8 == 0 &&
+                    (reinterpret_cast<uintptr_t>(map) & 7u) == 0;
+  return MaskView{map, s_b, s_e, s_t, fast ? 1 : 0};
+}
+
+// The offsets of per-tile counts (tiles of tt tokens) and the map from them.
+template <int MB>
+void launch_offsets_emit(const MaskView& m, int B, int T, int E, const int32_t* counts, int tt,
+                         int32_t* offsets, int32_t* group_sizes, const float* part_bal, int nblk,
+                         float* bal_sum, int32_t* row_id_map, hipStream_t st) {
+  const int nt = (T + tt - 1) / tt;
+  if ((int64_t)nt * E > 4096)
+    hipLaunchKernelGGL(rowmap_offsets_kernel<1024>, dim3(E, B), dim3(1024), 0, st, counts, E, nt,
+                       offsets, group_sizes, part_bal, nblk, bal_sum);
+  else
+    hipLaunchKernelGGL(rowmap_offsets_kernel<256>, dim3(E, B), dim3(256), 0, st, counts, E, nt,
+                       offsets, group_sizes, part_bal, nblk, bal_sum);
+  // few tiles: 4 tokens per wave (a token's entry is a serial chain: T = 517,
+  // E = 16 9.2 -> 7.9 us); many: 16, which read the tile's mask four times
+  // less often
+  const int tiles = (T + kTile64 - 1) / kTile64;
+  if ((int64_t)tiles * B <= 512)
+    hipLaunchKernelGGL((rowmap_emit64_kernel<MB, 4>), dim3(tiles, B), dim3(1024), 0, st, m, T, E, tt,
+                       offsets, row_id_map);
+  else
+    hipLaunchKernelGGL((rowmap_emit64_kernel<MB, 16>), dim3(tiles, B), dim3(256), 0, st, m, T, E, tt,
+                       offsets, row_id_map);
+}
+}  // namespace
+
+int launch_rowmap_from_counts(const uint8_t* mask, int64_t s_b, int64_t s_e, int B, int T, int E,
+                              const int32_t* counts, int tile_tokens, void* workspace,
+                              int32_t* group_sizes, const float* part_bal, int nblk,
+                              float* bal_sum, int32_t* row_id_map, hipStream_t st,
+                              const char* what) {
+  launch_offsets_emit<1>(mask_view(mask, 1, s_b, s_e, 1), B, T, E, counts, tile_tokens,
+                         static_cast<int32_t*>(workspace), group_sizes, part_bal, nblk, bal_sum,
+                         row_id_map, st);
+  return check_launch(what);
+}
+
 bool rowmap_fused_fits(int T, int E) {
   const int ntiles = (T + kTile - 1) / kTile;
   return T >= 1 && T % 16 == 0 && ntiles <= kFusedMaxTiles && E >= 1 && E <= kFusedMaxE;
@@ -1145,9 +1330,13 @@ using namespace uttt;
 
 extern "C" size_t uttt_row_id_map_workspace_bytes(int B, int T, int E) {
   if (B <= 0 || T <= 0 || E <= 0) return 0;
-  const int ntiles = (T + kTile - 1) / kTile;
-  const int per_tile = E <= kScanEmitMaxE ? padded_experts(E) : E;  // count-table row
-  return (size_t)B * per_tile * ntiles * sizeof(int32_t);
+  // 64-token tiles: the counts and the offsets (or the offsets of a router's
+  // 32-token counts); 256-token tiles for E <= kScanEmitMaxE
+  const size_t general = (size_t)2 * B * E * ((T + kTile64 - 1) / kTile64);
+  const size_t two = E <= kScanEmitMaxE
+                         ? (size_t)B * padded_experts(E) * ((T + kTile - 1) / kTile)
+                         : 0;
+  return (general > two ? general : two) * sizeof(int32_t);
 }
 
 extern "C" int uttt_make_row_id_map(const void* routing_map, int mask_bytes, int64_t s_b,
@@ -1206,18 +1395,12 @@ extern "C" int uttt_make_row_id_map(const void* routing_map, int mask_bytes, int
       }
       return;
     }
-    hipLaunchKernelGGL(rowmap_count_kernel<MB>, dim3(ntiles, B), dim3(kTile), 0, st, routing_map,
-                       s_b, s_e, s_t, T, E, ntiles, counts);
-    hipLaunchKernelGGL(rowmap_scan_kernel, dim3(B), dim3(kScanThreads), 0, st, counts, E, ntiles,
-                       group_sizes);
-    if (2 * E + 1 <= kStageMaxW) {
-      hipLaunchKernelGGL((rowmap_emit_kernel<MB, true>), dim3(ntiles, B), dim3(kTile),
-                         sizeof(int32_t) * kTile * (2 * E + 1), st, routing_map, s_b, s_e, s_t, T,
-                         E, ntiles, counts, row_id_map);
-    } else {
-      hipLaunchKernelGGL((rowmap_emit_kernel<MB, false>), dim3(ntiles, B), dim3(kTile), 0, st,
-                         routing_map, s_b, s_e, s_t, T, E, ntiles, counts, row_id_map);
-    }
+    const MaskView m = mask_view(routing_map, mask_bytes, s_b, s_e, s_t);
+    const int nt = (T + kTile64 - 1) / kTile64;
+    hipLaunchKernelGGL(rowmap_count64_kernel<MB>, dim3((nt + 3) / 4, B), dim3(kTile), 0, st, m, T, E,
+                       nt, counts);
+    launch_offsets_emit<MB>(m, B, T, E, counts, kTile64, counts + (int64_t)B * E * nt, group_sizes,
+                            nullptr, 0, nullptr, row_id_map, st);
   };
   if (mask_bytes == 1) {
     launch(std::integral_constant<int, 1>{});

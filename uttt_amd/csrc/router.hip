@@ -1392,9 +1392,11 @@ extern "C" int uttt_route_tokens_map(const void* x, int x_dtype, const float* ro
   UTTT_REQUIRE(src_rows == nullptr,
                "route_tokens_map: the inverse map (src_rows) needs 16-byte aligned mask and "
                "row map");
-  if (int rc = finish(w, B, E, T, group_sizes, nullptr, st, "route_tokens_map")) return rc;
-  return uttt_make_row_id_map(mask, 1, s_b, s_e, 1, B, T, E, row_id_map, nullptr,
-                              static_cast<uint8_t*>(workspace) + rm_off, workspace_bytes - rm_off,
-                              stream);
+  // otherwise the selection's counts per block are the row map's tile counts,
+  // and its offsets launch adds the balance partials (one block per batch: the
+  // sums are final)
+  return launch_rowmap_from_counts(m8, s_b, s_e, B, T, E, w.nblk > 1 ? w.part_cnt : w.cnt_sum,
+                                   blk_tokens, static_cast<uint8_t*>(workspace) + rm_off,
+                                   group_sizes, w.nblk > 1 ? w.part_bal : nullptr, w.nblk,
+                                   balance_sum, row_id_map, st, "route_tokens_map");
 }
-
