@@ -294,3 +294,69 @@ def test_row_map_from_64_token_tiles(T, E, form):
     rm = TP.make_row_id_map(m, B, T, E, group_sizes=gs)
     assert torch.equal(rm.cpu(), ref)
     assert torch.equal(gs.cpu(), mask.sum(-1).to(torch.int32))
+
+
+@pytest.mark.parametrize("H", [8, 24, 192, 200, 384, 520, 768, 2048, 2056])
+@pytest.mark.parametrize("B,T,E,k", [(1, 1, 1, 1), (2, 65, 128, 4), (1, 700, 16, 2)])
+def test_grouped_lane_kernels_of_16_bit_rows(H, B, T, E, k):
+    """The 16-bit backward kernels and the k / v / lr permute at the edges of
+    their lane groups (and past them: H = 2056), tokens with none to k + 1
+    experts, gates of zero, rows past num_out.  k / v / lr outputs bit-exact.
+    Backward: fp32 sums of the same bf16 values in slot order, one bf16 rounding
+    (2^-8 relative); dot products in another order: H * 2^-24 of sum |x||y|."""
+    g = torch.Generator().manual_seed(H + T)
+    n = torch.randint(0, k + 2, (B, 1, T), generator=g).clamp(max=E)
+    mask = torch.rand(B, E, T, generator=g).argsort(1).argsort(1) < n
+    probs = torch.rand(B, E, T, generator=g) * mask
+    probs[:, :, T // 2] = 0.0
+    N = k * T
+    rm = OP.make_row_id_map(mask)
+    wr = OP.written_rows(rm, N)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    kx, vx, go, y = bf(B, T, H), bf(B, T, H), bf(B, T, H), bf(B, N, H)
+    lrs = [torch.rand(B, T, generator=g).to(torch.bfloat16) for _ in range(3)]
+    # rows past num_out stay unwritten, their slots absent
+    refs = OP.permute_kv_lrs(kx, vx, *lrs, rm, probs, N)
+    ins = [t.to(DEV).requires_grad_() for t in (kx, vx, *lrs, probs)]
+    outs = TP.permute_kv_and_lrs(*ins[:5], mask.to(DEV), ins[5], k)
+    for o, r in zip(outs, refs):
+        assert torch.equal(bits(o)[wr], bits(r)[wr])
+    gk, gv = bf(B, N, H), bf(B, N, H)
+    gl = [torch.randn(B, N, generator=g).to(torch.bfloat16) for _ in range(3)]
+    grads = torch.autograd.grad(outs, ins, [t.to(DEV).view(o.shape) for t, o in zip((gk, gv, *gl), outs)])
+    close = lambda a, r: bool(((a.cpu().double() - r).abs() <= 2.0 ** -8 * r.abs() + 1e-5).all())
+    slots = [(b, t, int(rm[b, t, j]), int(rm[b, t, E + j])) for b in range(B) for t in range(T)
+             for j in range(int(rm[b, t, 2 * E])) if int(rm[b, t, j]) < N]
+    b_, t_, r_, e_ = (torch.tensor(c, dtype=torch.long) for c in zip(*slots)) if slots else [torch.empty(0, dtype=torch.long)] * 4
+    p_ = probs[b_, e_, t_].double()
+    sum_rows = lambda rows: torch.zeros(B, T, *rows.shape[1:], dtype=torch.float64).index_put_((b_, t_), rows, accumulate=True)
+    assert close(grads[0], sum_rows(gk[b_, r_].double()))
+    assert close(grads[1], sum_rows(gv[b_, r_].double() * p_[:, None]))
+    for q in range(3):
+        assert close(grads[2 + q], sum_rows(gl[q][b_, r_].double()))
+    tol = lambda a, c: H * 2.0 ** -24 * (a.double().abs() * c.double().abs()).sum(-1) + 1e-30
+
+    def check_gp(got, a, c, zero_gate):
+        ref, bound = torch.zeros(B, E, T, dtype=torch.float64), torch.zeros(B, E, T, dtype=torch.float64)
+        live = (p_ != 0) if zero_gate else torch.ones_like(p_, dtype=torch.bool)
+        ref[b_, e_, t_] = (a.double() * c.double()).sum(-1) * live
+        bound[b_, e_, t_] = tol(a, c)
+        assert bool(((got.cpu().double() - ref).abs() <= bound).all())
+
+    check_gp(grads[5], gv[b_, r_], vx[b_, t_], True)
+    # unpermute backward
+    yd, pd = y.to(DEV).requires_grad_(), probs.to(DEV).requires_grad_()
+    out = TP.unpermute_and_merge_with_probs(yd, rm.to(DEV), pd)
+    gy, gp = torch.autograd.grad(out, [yd, pd], go.to(DEV))
+    if slots:
+        assert torch.equal(bits(gy)[b_, r_], bits((go[b_, t_].float() * p_.float()[:, None]).to(torch.bfloat16)))
+    check_gp(gp, go[b_, t_], y[b_, r_], False)
+    # permute backward
+    xd, pd = kx.to(DEV).requires_grad_(), probs.to(DEV).requires_grad_()
+    xp, pp, _ = TP.permute_with_expert_mask(xd, mask.to(DEV), pd, k)
+    gpp = torch.randn(B, N, generator=g)
+    gx, gp = torch.autograd.grad([xp, pp], [xd, pd], [gk.to(DEV), gpp.to(DEV)])
+    assert close(gx, sum_rows(gk[b_, r_].double()))
+    ref = torch.zeros(B, E, T)
+    ref[b_, e_, t_] = gpp[b_, r_]
+    assert torch.equal(gp.cpu(), ref)

@@ -18,8 +18,8 @@
 // Payload kernels move rows in 16-byte vectors: permute reads a token's row
 // once and writes it to each of the token's slots; unpermute gathers the slots
 // and reduces in fp32 registers.  The forward pair spreads (token, chunk)
-// pairs over all lanes; the backward and k/v/lr kernels give one 64-lane wave
-// to one token.
+// pairs over all lanes; the backward and k/v/lr kernels give a group of 8 to 64
+// lanes to one token (one wave for rows that are not 16-bit vectors).
 #include "common.h"
 
 namespace uttt {
@@ -1233,6 +1233,425 @@ int pick_ve(int H, std::initializer_list<const void*> ptrs) {
   return ve >= 8 ? 8 : ve >= 4 ? 4 : ve >= 2 ? 2 : 1;
 }
 
+// ------------------------------------------ rows of 16-bit elements, grouped ---
+// The kernels above give a 64-lane wave to one token: a row of 192 elements
+// fills 24 lanes, the slot -> gate -> payload loads are one token's chain, and the
+// prob gradients go out as 4 bytes per (expert, token). Here G lanes (a power of
+// two) own a token and hold its row in NI 16-byte chunks each (lane c of the
+// group: chunks c, c + G, ...), so 64 / G tokens run in a wave and all of a
+// token's loads are in flight together; the prob gradients of a workgroup's
+// TOK tokens are collected in LDS ([E][TOK] fp32, zeros where not routed) and
+// stored as runs of TOK tokens.  Bound by the rows' memory traffic; payload
+// loads are non-temporal (read once), stores are not (the next kernel reads
+// them): permute_kv backward of 196 608 tokens of 192, 48 experts 269 -> 85 us,
+// forward 127 -> 62; unpermute / permute backward of 65 536 x 768, top-2 116 -> 85
+// and 89 -> 55 us (with non-temporal stores 100 and 63, with plain loads 101 and
+// 72).  For 16-bit payloads of 16-byte rows (H a multiple of 8, H <= 2048, aligned
+// pointers), E <= 128 and num_out >= 1; the kernels above take the rest.
+// Workgroups of TOK tokens (64, or 16 where those would leave CUs idle) and at
+// most 512 threads.
+constexpr int grp_threads(int g, int tok) { return g * tok < 512 ? g * tok : 512; }
+
+template <int G>
+__device__ __forceinline__ float group_sum(float v) {
+#pragma unroll
+  for (int o = G / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, G);
+  return v;
+}
+
+// A token's first two slots (the rest is read when used), from its row of the
+// map; rows outside [0, num_out) count as absent but keep their slot.
+struct GrpSlots {
+  int n, r0, r1, e0, e1;
+  bool ok0, ok1;
+  __device__ __forceinline__ void load(const int32_t* rm, int E, int num_out) {
+    const int j1 = E > 1 ? 1 : 0;
+    n = rm[2 * E];
+    r0 = rm[0];
+    r1 = rm[j1];
+    e0 = rm[E];
+    e1 = rm[E + j1];
+    ok0 = n > 0 && r0 >= 0 && r0 < num_out;
+    ok1 = n > 1 && r1 >= 0 && r1 < num_out;
+  }
+};
+
+template <int NI>
+struct Row {
+  uint4 c[NI];
+  // chunk i of this lane at p + 8 (cl + G i), chunks past CH re-read the last
+  template <int G>
+  __device__ __forceinline__ void load(const uint16_t* p, int cl, int CH) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      c[i] = *reinterpret_cast<const uint4*>(p + 8 * min(cl + G * i, CH - 1));
+  }
+  template <int G>
+  __device__ __forceinline__ void load_nt(const uint16_t* p, int cl, int CH) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const auto v = __builtin_nontemporal_load(reinterpret_cast<const Vec<16>::T*>(p + 8 * min(cl + G * i, CH - 1)));
+      __builtin_memcpy(&c[i], &v, 16);
+    }
+  }
+};
+template <class TT>
+__device__ __forceinline__ void grp_unpack(const uint4& u, float (&v)[8]) {
+  const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    v[2 * k] = TT::load((uint16_t)(w[k] & 0xffffu));
+    v[2 * k + 1] = TT::load((uint16_t)(w[k] >> 16));
+  }
+}
+template <class TT>
+__device__ __forceinline__ uint4 grp_pack(const float (&v)[8]) {
+  uint4 u;
+  u.x = (uint32_t)TT::store(v[0]) | ((uint32_t)TT::store(v[1]) << 16);
+  u.y = (uint32_t)TT::store(v[2]) | ((uint32_t)TT::store(v[3]) << 16);
+  u.z = (uint32_t)TT::store(v[4]) | ((uint32_t)TT::store(v[5]) << 16);
+  u.w = (uint32_t)TT::store(v[6]) | ((uint32_t)TT::store(v[7]) << 16);
+  return u;
+}
+__device__ __forceinline__ void grp_store(uint16_t* p, const uint4& u) {
+  *reinterpret_cast<uint4*>(p) = u;
+}
+
+// The workgroup's tile of prob gradients.
+template <int TOK, int THREADS>
+__device__ __forceinline__ void gp_zero(float* tile, int E) {
+  for (int i = threadIdx.x; i < E * TOK; i += THREADS) tile[i] = 0.0f;
+  __syncthreads();
+}
+template <int TOK, int THREADS>
+__device__ __forceinline__ void gp_store(const float* tile, int E, int t0, int T, float* gprobs,
+                                         int64_t s_e, int64_t s_t) {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // LDS only
+  for (int i = threadIdx.x; i < E * TOK; i += THREADS) {
+    const int e = i / TOK, t = t0 + i % TOK;
+    if (t < T) gprobs[(int64_t)e * s_e + (int64_t)t * s_t] = tile[i];
+  }
+}
+
+// grad_inp[t] = sum_j grad_out[row_j] (fp32, slot order); grad_probs from gpp.
+template <class TT, int G, int NI, int TOK>
+__global__ __launch_bounds__(grp_threads(G, TOK)) void permute_bwd_grp_kernel(
+    const uint16_t* __restrict__ gout, int H, int T, const int32_t* __restrict__ rmap, int E,
+    int num_out, const float* __restrict__ gpp, uint16_t* __restrict__ ginp,
+    float* __restrict__ gprobs) {
+  extern __shared__ float gp[];
+  constexpr int kThr = grp_threads(G, TOK);
+  const int b = blockIdx.y, t0 = blockIdx.x * TOK;
+  const int cl = threadIdx.x % G, CH = H / 8;
+  if (gprobs != nullptr) gp_zero<TOK, kThr>(gp, E);
+  const uint16_t* gb = gout + (int64_t)b * num_out * H;
+  for (int tl = threadIdx.x / G; tl < TOK; tl += kThr / G) {
+    const int t = t0 + tl;
+    const int64_t bt = (int64_t)b * T + min(t, T - 1);
+    const int32_t* rm = rmap + bt * (2 * E + 1);
+    GrpSlots s;
+    s.load(rm, E, num_out);
+    Row<NI> x0, x1;
+    x0.template load_nt<G>(gb + (int64_t)(s.ok0 ? s.r0 : 0) * H, cl, CH);
+    const bool two = __any(s.n > 1);
+    if (two) x1.template load_nt<G>(gb + (int64_t)(s.ok1 ? s.r1 : 0) * H, cl, CH);
+    if (t < T && gprobs != nullptr && cl == 0) {
+      for (int j = 0; j < s.n; ++j) {
+        const int row = rm[j];
+        if (row >= 0 && row < num_out) gp[rm[E + j] * TOK + tl] = gpp[(int64_t)b * num_out + row];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      float acc[8] = {}, v[8];
+      if (s.ok0) {
+        grp_unpack<TT>(x0.c[i], v);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc[u] += v[u];
+      }
+      if (two && s.ok1) {
+        grp_unpack<TT>(x1.c[i], v);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc[u] += v[u];
+      }
+      const int ch = cl + G * i;
+      for (int j = 2; j < s.n; ++j) {
+        const int row = rm[j];
+        if (row < 0 || row >= num_out) continue;
+        grp_unpack<TT>(*reinterpret_cast<const uint4*>(gb + (int64_t)row * H + 8 * min(ch, CH - 1)), v);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc[u] += v[u];
+      }
+      if (t < T && ch < CH) grp_store(ginp + bt * H + 8 * ch, grp_pack<TT>(acc));
+    }
+  }
+  if (gprobs != nullptr) gp_store<TOK, kThr>(gp, E, t0, T, gprobs + (int64_t)b * E * T, T, 1);
+}
+
+// grad_inp[row_j] = grad_out[t] p_j; grad_probs[e_j, t] = <y[row_j], grad_out[t]>.
+template <class TT, int G, int NI, int TOK>
+__global__ __launch_bounds__(grp_threads(G, TOK)) void unpermute_bwd_grp_kernel(
+    const uint16_t* __restrict__ gout, const uint16_t* __restrict__ fwd_inp, int H, int T,
+    const int32_t* __restrict__ rmap, int E, int num_out, const float* __restrict__ probs,
+    int64_t p_sb, int64_t p_se, int64_t p_st, uint16_t* __restrict__ ginp,
+    float* __restrict__ gprobs, int64_t g_sb, int64_t g_se, int64_t g_st) {
+  extern __shared__ float gp[];
+  constexpr int kThr = grp_threads(G, TOK);
+  const int b = blockIdx.y, t0 = blockIdx.x * TOK;
+  const int cl = threadIdx.x % G, CH = H / 8;
+  gp_zero<TOK, kThr>(gp, E);
+  const uint16_t* yb = fwd_inp + (int64_t)b * num_out * H;
+  uint16_t* gb = ginp + (int64_t)b * num_out * H;
+  for (int tl = threadIdx.x / G; tl < TOK; tl += kThr / G) {
+    const int t = t0 + tl;
+    const int tc = min(t, T - 1);
+    const int64_t bt = (int64_t)b * T + tc;
+    const int32_t* rm = rmap + bt * (2 * E + 1);
+    Row<NI> g, y0, y1;
+    g.template load_nt<G>(gout + bt * H, cl, CH);
+    GrpSlots s;
+    s.load(rm, E, num_out);
+    const float* pt = probs + b * p_sb + (int64_t)tc * p_st;
+    const float p0 = pt[(s.n > 0 ? s.e0 : 0) * p_se];
+    y0.template load_nt<G>(yb + (int64_t)(s.ok0 ? s.r0 : 0) * H, cl, CH);
+    const bool two = __any(s.n > 1);
+    float p1 = 0.0f;
+    if (two) {
+      p1 = pt[(s.n > 1 ? s.e1 : 0) * p_se];
+      y1.template load_nt<G>(yb + (int64_t)(s.ok1 ? s.r1 : 0) * H, cl, CH);
+    }
+    auto slot = [&](const Row<NI>& y, int row, int e, float p, bool ok) __attribute__((always_inline)) {
+      float dot = 0.0f;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int ch = cl + G * i;
+        float gv[8], yv[8], o[8];
+        grp_unpack<TT>(g.c[i], gv);
+        grp_unpack<TT>(y.c[i], yv);
+        float d = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          o[u] = gv[u] * p;
+          d = __builtin_fmaf(yv[u], gv[u], d);
+        }
+        if (ch < CH) {
+          dot += d;
+          if (ok) grp_store(gb + (int64_t)row * H + 8 * ch, grp_pack<TT>(o));
+        }
+      }
+      dot = group_sum<G>(dot);
+      if (ok && cl == 0) gp[e * TOK + tl] = dot;
+    };
+    slot(y0, s.r0, s.e0, p0, s.ok0 && t < T);
+    if (two) slot(y1, s.r1, s.e1, p1, s.ok1 && t < T);
+    const int more = t < T ? s.n : 0;
+    for (int j = 2; __any(j < more); ++j) {
+      const bool in = j < more;
+      const int row = in ? rm[j] : 0, e = in ? rm[E + j] : 0;
+      const bool ok = in && row >= 0 && row < num_out;
+      y0.template load<G>(yb + (int64_t)(ok ? row : 0) * H, cl, CH);
+      slot(y0, row, e, pt[e * p_se], ok);
+    }
+  }
+  gp_store<TOK, kThr>(gp, E, t0, T, gprobs + b * g_sb, g_se, g_st);
+}
+
+// k rows copied, v rows times the gate, lr entries copied, to every slot.
+template <class KT, class VT, int G, int NI, int TOK>
+__global__ __launch_bounds__(grp_threads(G, TOK)) void permute_kv_fwd_grp_kernel(
+    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const uint8_t* __restrict__ lr0, const uint8_t* __restrict__ lr1,
+    const uint8_t* __restrict__ lr2, int lr_bytes, int H, int T,
+    const int32_t* __restrict__ rmap, int E, const float* __restrict__ probs, int64_t p_sb,
+    int64_t p_se, int64_t p_st, uint16_t* __restrict__ k_out, uint16_t* __restrict__ v_out,
+    uint8_t* __restrict__ lr0_out, uint8_t* __restrict__ lr1_out,
+    uint8_t* __restrict__ lr2_out, int num_out) {
+  constexpr int kThr = grp_threads(G, TOK);
+  const int b = blockIdx.y, t0 = blockIdx.x * TOK;
+  const int cl = threadIdx.x % G, CH = H / 8;
+  for (int tl = threadIdx.x / G; tl < TOK; tl += kThr / G) {
+    const int t = t0 + tl;
+    const int tc = min(t, T - 1);
+    const int64_t bt = (int64_t)b * T + tc;
+    const int32_t* rm = rmap + bt * (2 * E + 1);
+    Row<NI> kr, vr;
+    kr.template load_nt<G>(k + bt * H, cl, CH);
+    vr.template load_nt<G>(v + bt * H, cl, CH);
+    // lane q < 3 of the group carries lr q
+    const uint8_t* lsrc = (cl == 0 ? lr0 : cl == 1 ? lr1 : lr2) + bt * lr_bytes;
+    uint8_t* ldst = cl == 0 ? lr0_out : cl == 1 ? lr1_out : lr2_out;
+    const uint32_t lv = lr_bytes == 4 ? *reinterpret_cast<const uint32_t*>(lsrc)
+                                      : *reinterpret_cast<const uint16_t*>(lsrc);
+    GrpSlots s;
+    s.load(rm, E, num_out);
+    const float* pt = probs + b * p_sb + (int64_t)tc * p_st;
+    const float p0 = pt[(s.n > 0 ? s.e0 : 0) * p_se];
+    const bool two = __any(s.n > 1);
+    const float p1 = two ? pt[(s.n > 1 ? s.e1 : 0) * p_se] : 0.0f;
+    auto put = [&](int row, float p) __attribute__((always_inline)) {
+      const int64_t r = (int64_t)b * num_out + row;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int ch = cl + G * i;
+        float o[8];
+        grp_unpack<VT>(vr.c[i], o);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) o[u] *= p;
+        if (ch < CH) {
+          grp_store(k_out + r * H + 8 * ch, kr.c[i]);
+          grp_store(v_out + r * H + 8 * ch, grp_pack<KT>(o));
+        }
+      }
+      if (cl < 3) {
+        if (lr_bytes == 4)
+          *reinterpret_cast<uint32_t*>(ldst + r * 4) = lv;
+        else
+          *reinterpret_cast<uint16_t*>(ldst + r * 2) = (uint16_t)lv;
+      }
+    };
+    if (t >= T) continue;
+    if (s.ok0) put(s.r0, p0);
+    if (s.ok1) put(s.r1, p1);
+    for (int j = 2; j < s.n; ++j) {
+      const int row = rm[j];
+      if (row >= 0 && row < num_out) put(row, pt[(int64_t)rm[E + j] * p_se]);
+    }
+  }
+}
+
+// grad_k = sum_j gk[row_j], grad_v = sum_j gv[row_j] p_j, grad_lr = sum_j glr[row_j],
+// grad_probs[e_j, t] = <gv[row_j], v[t]> (0 where p_j = 0).
+template <class KT, class VT, class LT, int G, int NI, int TOK>
+__global__ __launch_bounds__(grp_threads(G, TOK)) void permute_kv_bwd_grp_kernel(
+    const uint16_t* __restrict__ gk, const uint16_t* __restrict__ gv,
+    const typename LT::S* __restrict__ glr0, const typename LT::S* __restrict__ glr1,
+    const typename LT::S* __restrict__ glr2, const uint16_t* __restrict__ v,
+    const float* __restrict__ probs, int64_t p_sb, int64_t p_se, int64_t p_st, int H, int T,
+    const int32_t* __restrict__ rmap, int E, int num_out, uint16_t* __restrict__ grad_k,
+    uint16_t* __restrict__ grad_v, typename LT::S* __restrict__ grad_lr0,
+    typename LT::S* __restrict__ grad_lr1, typename LT::S* __restrict__ grad_lr2,
+    float* __restrict__ grad_probs) {
+  extern __shared__ float gp[];
+  using SL = typename LT::S;
+  constexpr int kThr = grp_threads(G, TOK);
+  const int b = blockIdx.y, t0 = blockIdx.x * TOK;
+  const int cl = threadIdx.x % G, CH = H / 8;
+  gp_zero<TOK, kThr>(gp, E);
+  const uint16_t* gkb = gk + (int64_t)b * num_out * H;
+  const uint16_t* gvb = gv + (int64_t)b * num_out * H;
+  const SL* gl = (cl == 0 ? glr0 : cl == 1 ? glr1 : glr2) + (int64_t)b * num_out;
+  SL* go = (cl == 0 ? grad_lr0 : cl == 1 ? grad_lr1 : grad_lr2);
+  for (int tl = threadIdx.x / G; tl < TOK; tl += kThr / G) {
+    const int t = t0 + tl;
+    const int tc = min(t, T - 1);
+    const int64_t bt = (int64_t)b * T + tc;
+    const int32_t* rm = rmap + bt * (2 * E + 1);
+    Row<NI> vr, k0, v0;
+    vr.template load_nt<G>(v + bt * H, cl, CH);
+    GrpSlots s;
+    s.load(rm, E, num_out);
+    const float* pt = probs + b * p_sb + (int64_t)tc * p_st;
+    float ak[NI][8], av[NI][8], al = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int u = 0; u < 8; ++u) ak[i][u] = av[i][u] = 0.0f;
+    auto slot = [&](int row, int e, bool ok) __attribute__((always_inline)) {
+      const int64_t r = ok ? row : 0;
+      const float p = pt[(ok ? e : 0) * p_se];
+      k0.template load_nt<G>(gkb + r * H, cl, CH);
+      v0.template load_nt<G>(gvb + r * H, cl, CH);
+      const float l = LT::load(gl[r]);
+      float dot = 0.0f;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        float a[8], c[8], x[8];
+        grp_unpack<KT>(k0.c[i], a);
+        grp_unpack<KT>(v0.c[i], c);
+        grp_unpack<VT>(vr.c[i], x);
+        float d = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          ak[i][u] += ok ? a[u] : 0.0f;
+          av[i][u] = ok ? __builtin_fmaf(c[u], p, av[i][u]) : av[i][u];
+          d = __builtin_fmaf(c[u], x[u], d);
+        }
+        dot += cl + G * i < CH ? d : 0.0f;
+      }
+      al += ok ? l : 0.0f;
+      dot = group_sum<G>(dot);
+      if (ok && cl == 0) gp[e * TOK + tl] = p != 0.0f ? dot : 0.0f;
+    };
+    const int n = t < T ? s.n : 0;
+    slot(s.r0, s.e0, s.ok0 && n > 0);
+    if (__any(n > 1)) slot(s.r1, s.e1, s.ok1 && n > 1);
+    for (int j = 2; __any(j < n); ++j) {
+      const bool in = j < n;
+      const int row = in ? rm[j] : -1, e = in ? rm[E + j] : 0;
+      slot(row, e, in && row >= 0 && row < num_out);
+    }
+    if (t < T) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int ch = cl + G * i;
+        if (ch < CH) {
+          grp_store(grad_k + bt * H + 8 * ch, grp_pack<KT>(ak[i]));
+          grp_store(grad_v + bt * H + 8 * ch, grp_pack<VT>(av[i]));
+        }
+      }
+      if (cl < 3) go[bt] = LT::store(al);
+    }
+  }
+  gp_store<TOK, kThr>(gp, E, t0, T, grad_probs + (int64_t)b * E * T, T, 1);
+}
+
+// Lanes per token: at most four 16-byte chunks per lane, at least 8 lanes.
+inline int grp_lanes(int H) {
+  const int CH = H / 8;
+  int g = 8;
+  while (g < 64 && 4 * g < CH) g *= 2;
+  return g;
+}
+template <class TT>
+bool grp_fits(int H, int E, int num_out, std::initializer_list<const void*> ptrs) {
+  if (sizeof(typename TT::S) != 2 || H < 8 || H > 2048 || E > 128 || num_out < 1) return false;
+  return pick_ve<TT>(H, ptrs) == 8;
+}
+// f(G, NI, TOK) with compile-time lanes per token, chunks per lane and tokens
+// per workgroup
+template <class F>
+void grp_dispatch(int H, int T, int B, F&& f) {
+  const int g = grp_lanes(H), ni = (H / 8 + g - 1) / g;
+  const bool many = (int64_t)B * ((T + 63) / 64) >= 512;
+  auto with = [&](auto G) {
+    auto tok = [&](auto NI) {
+      if (many) f(G, NI, std::integral_constant<int, 64>{});
+      else f(G, NI, std::integral_constant<int, 16>{});
+    };
+    switch (ni) {
+      case 1: tok(std::integral_constant<int, 1>{}); break;
+      case 2: tok(std::integral_constant<int, 2>{}); break;
+      case 3: tok(std::integral_constant<int, 3>{}); break;
+      default: tok(std::integral_constant<int, 4>{}); break;
+    }
+  };
+  switch (g) {
+    case 8: with(std::integral_constant<int, 8>{}); break;
+    case 16: with(std::integral_constant<int, 16>{}); break;
+    case 32: with(std::integral_constant<int, 32>{}); break;
+    default: with(std::integral_constant<int, 64>{}); break;
+  }
+}
+// The launch of grouped-lane kernel K<types..., G, NI, TOK> over T tokens per batch.
+#define UTTT_GRP_LAUNCH(LDS_E, ...)                                                            \
+  grp_dispatch(H, T, B, [&](auto g_, auto ni_, auto tok_) {                                    \
+    constexpr int G = decltype(g_)::value, NI = decltype(ni_)::value,                          \
+                  TOK = decltype(tok_)::value;                                                 \
+    const dim3 grid((T + TOK - 1) / TOK, B), block(grp_threads(G, TOK));                       \
+    const size_t lds = sizeof(float) * (LDS_E) * TOK;                                          \
+    __VA_ARGS__;                                                                               \
+  })
+
 #define UTTT_VE_SWITCH(ve, ...)          \
   switch (ve) {                          \
     case 8: { constexpr int VE = 8; __VA_ARGS__; } break; \
@@ -1469,6 +1888,14 @@ extern "C" int uttt_permute_bwd(const void* grad_out, int dtype, int B, int T, i
   hipStream_t st = as_stream(stream);
   UTTT_DTYPE_SWITCH(dtype, TT, {
     using S = typename TT::S;
+    if constexpr (sizeof(S) == 2) {
+      if (grp_fits<TT>(H, E, num_out, {grad_out, grad_inp})) {
+        UTTT_GRP_LAUNCH(E, hipLaunchKernelGGL((permute_bwd_grp_kernel<TT, G, NI, TOK>), grid, block, lds, st,
+                             reinterpret_cast<const S*>(grad_out), H, T, row_id_map, E, num_out,
+                             grad_permuted_probs, reinterpret_cast<S*>(grad_inp), grad_probs));
+        return check_launch("permute_bwd");
+      }
+    }
     const int ve = pick_ve<TT>(H, {grad_out, grad_inp});
     UTTT_VE_SWITCH(ve, hipLaunchKernelGGL((permute_bwd_kernel<TT, VE>), tok_grid(T, B), tok_block(),
                                           0, st, reinterpret_cast<const S*>(grad_out), H, T,
@@ -1519,6 +1946,16 @@ extern "C" int uttt_unpermute_bwd(const void* grad_out, const void* fwd_inp, int
   hipStream_t st = as_stream(stream);
   UTTT_DTYPE_SWITCH(dtype, TT, {
     using S = typename TT::S;
+    if constexpr (sizeof(S) == 2) {
+      if (grp_fits<TT>(H, E, num_out, {grad_out, fwd_inp, grad_inp})) {
+        UTTT_GRP_LAUNCH(E, hipLaunchKernelGGL((unpermute_bwd_grp_kernel<TT, G, NI, TOK>), grid, block, lds, st,
+                             reinterpret_cast<const S*>(grad_out),
+                             reinterpret_cast<const S*>(fwd_inp), H, T, row_id_map, E, num_out,
+                             probs, p_sb, p_se, p_st, reinterpret_cast<S*>(grad_inp), grad_probs,
+                             gp_sb, gp_se, gp_st));
+        return check_launch("unpermute_bwd");
+      }
+    }
     const int ve = pick_ve<TT>(H, {grad_out, fwd_inp, grad_inp});
     UTTT_VE_SWITCH(ve, hipLaunchKernelGGL((unpermute_bwd_kernel<TT, VE>), tok_grid(T, B),
                                           tok_block(), 0, st,
@@ -1538,6 +1975,19 @@ int launch_permute_kv_fwd(const void* k, const void* v, const void* lr0, const v
                           const int32_t* row_id_map, int E, const float* probs, int64_t p_sb,
                           int64_t p_se, int64_t p_st, void* k_out, void* v_out, void* lr0_out,
                           void* lr1_out, void* lr2_out, int num_out, hipStream_t st) {
+  if constexpr (sizeof(typename KT::S) == 2 && sizeof(typename VT::S) == 2) {
+    if (grp_fits<KT>(H, 1, num_out, {k, v, k_out, v_out})) {
+      UTTT_GRP_LAUNCH(0, hipLaunchKernelGGL((permute_kv_fwd_grp_kernel<KT, VT, G, NI, TOK>), grid, block, lds, st,
+                           reinterpret_cast<const uint16_t*>(k), reinterpret_cast<const uint16_t*>(v),
+                           reinterpret_cast<const uint8_t*>(lr0), reinterpret_cast<const uint8_t*>(lr1),
+                           reinterpret_cast<const uint8_t*>(lr2), lr_bytes, H, T, row_id_map, E,
+                           probs, p_sb, p_se, p_st, reinterpret_cast<uint16_t*>(k_out),
+                           reinterpret_cast<uint16_t*>(v_out), reinterpret_cast<uint8_t*>(lr0_out),
+                           reinterpret_cast<uint8_t*>(lr1_out), reinterpret_cast<uint8_t*>(lr2_out),
+                           num_out));
+      return check_launch("permute_kv_lrs_fwd");
+    }
+  }
   const int vek = pick_ve<KT>(H, {k, k_out, v_out});
   const int vev = pick_ve<VT>(H, {v});
   const int ve = vek < vev ? vek : vev;
@@ -1563,6 +2013,20 @@ int launch_permute_kv_bwd(const void* gk, const void* gv, const void* glr0, cons
                           const int32_t* row_id_map, int E, int num_out, void* grad_k,
                           void* grad_v, void* grad_lr0, void* grad_lr1, void* grad_lr2,
                           float* grad_probs, hipStream_t st) {
+  if constexpr (sizeof(typename KT::S) == 2 && sizeof(typename VT::S) == 2) {
+    if (grp_fits<KT>(H, E, num_out, {gk, gv, grad_k, v, grad_v})) {
+      using SL = typename LT::S;
+      UTTT_GRP_LAUNCH(E, hipLaunchKernelGGL((permute_kv_bwd_grp_kernel<KT, VT, LT, G, NI, TOK>), grid, block, lds, st,
+                           reinterpret_cast<const uint16_t*>(gk), reinterpret_cast<const uint16_t*>(gv),
+                           reinterpret_cast<const SL*>(glr0), reinterpret_cast<const SL*>(glr1),
+                           reinterpret_cast<const SL*>(glr2), reinterpret_cast<const uint16_t*>(v),
+                           probs, p_sb, p_se, p_st, H, T, row_id_map, E, num_out,
+                           reinterpret_cast<uint16_t*>(grad_k), reinterpret_cast<uint16_t*>(grad_v),
+                           reinterpret_cast<SL*>(grad_lr0), reinterpret_cast<SL*>(grad_lr1),
+                           reinterpret_cast<SL*>(grad_lr2), grad_probs));
+      return check_launch("permute_kv_lrs_bwd");
+    }
+  }
   const int vek = pick_ve<KT>(H, {gk, gv, grad_k});
   const int vev = pick_ve<VT>(H, {v, grad_v});
   const int ve = vek < vev ? vek : vev;
