@@ -262,3 +262,25 @@ def test_routed_read_without_gradient_equals_the_permuted_path():
         torch.cuda.synchronize()
         assert torch.equal(fast, slow.detach()), f"E={E}: gathered read differs"
         assert torch.equal(lb[1], lb2[1])
+
+
+@pytest.mark.parametrize("D,rope_dim", [(8, 0), (64, 64), (192, 64), (256, 256), (384, 128), (520, 0),
+                                        (768, 16), (1032, 0), (1536, 64), (2048, 256), (4096, 32)])
+@pytest.mark.parametrize("norm", [None, "l2", "rms"])
+def test_rows_preprocess_row_widths(D, rope_dim, norm):
+    """Every lane-group width and chunk count of the row kernels, a row count
+    that does not fill the last workgroup, forward and backward."""
+    B, Lx = 1, 37
+    g = torch.Generator().manual_seed(D)
+    x = torch.randn(B, Lx, D, generator=g).to(torch.bfloat16)
+    gy = torch.randn(B, Lx, D, generator=g).to(torch.bfloat16)
+    rp = orp = None
+    if rope_dim:
+        cos, sin = moe.Rope.tables(rope_dim, 10000.0, Lx + 5, "cpu")
+        rp, orp = moe.Rope(cos.to(DEV), sin.to(DEV), 5), (cos, sin, 5)
+    xd = x.to(DEV).requires_grad_()
+    y = moe.rows_preprocess(xd, silu=True, norm=norm, rows_of=D, rope=rp)
+    _close(y, MU.preprocess_rows(x, silu=True, norm=norm, rows_of=D, rope=orp), 8e-3, "forward")
+    y.backward(gy.to(DEV))
+    ref = MU.preprocess_rows_bwd(x, gy, silu=True, norm=norm, rows_of=D, rope=orp)
+    _close(xd.grad, ref, 2e-2, "backward")

@@ -19,12 +19,15 @@
 // stores bf16, the compiled norm's backward and the silu backward store the
 // input dtype.
 //
-// One wave per row, 8 elements (one 16-byte bf16 vector or two fp32 ones)
-// per lane step; the row stays in registers between the reductions and the
-// element pass, so the row is read once and written once.  A rotary pair
-// (j, j + R) of a block sits R / 8 lanes apart in the same lane step (blocks
-// of 2R elements tile the 512 elements of a step when 2R divides 512), so the
-// partner values come from one lane exchange.
+// G lanes (8 to 64, a power of two) per row, NI chunks of 8 elements (one
+// 16-byte bf16 vector or two fp32 ones) per lane: chunk i of lane c is c + G i;
+// the row stays in registers between the reductions and the element pass, so
+// it is read once and written once.  A rotary pair (j, j + R) of a block sits
+// R / 8 lanes apart in the same lane step (G is a multiple of a block's 2R / 8
+// chunks), so the partner values come from one lane exchange.  Bound by
+// memory; with one wave per row and always 8 chunks per lane a 384-element row
+// paid the loads and exponentials of 4096: forward with rotary over 16 384 such
+// rows 46 us, backward 68, now 15 and 19.
 #include <type_traits>
 
 #include "common.h"
@@ -33,6 +36,7 @@ namespace uttt {
 namespace {
 
 constexpr int kMaxChunksPerLane = 8;  // rows of up to 64 * 8 * 8 = 4096 elements
+constexpr int kPrepThreads = 256;
 
 template <class TT>
 __device__ __forceinline__ void load8(const typename TT::S* p, float (&v)[8]) {
@@ -73,9 +77,10 @@ __device__ __forceinline__ float rnd(float x) {
   return TT::load(TT::store(x));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
+template <int G>
+__device__ __forceinline__ float row_sum(float v) {
 #pragma unroll
-  for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+  for (int d = G / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, G);
   return v;
 }
 
@@ -93,19 +98,28 @@ struct Rows {
   int rope_half, rows_per_token, seq_len, pos_offset;
 };
 
+// The rotary table row of a row (its token's position); 32-bit divisions where
+// the row count fits.
+__device__ __forceinline__ int64_t rope_row(const Rows& a, int64_t row) {
+  if (a.rows > 0xffffffffLL)  // uniform
+    return ((row / a.rows_per_token) % a.seq_len + a.pos_offset) * a.rope_half;
+  const uint32_t tok = (uint32_t)row / (uint32_t)a.rows_per_token;
+  return (int64_t)((int)(tok % (uint32_t)a.seq_len) + a.pos_offset) * a.rope_half;
+}
+
 // The rotary step of one lane step's chunk (8 elements of a row at element
-// offset e0 of the token): x -> the rotated values, with `conj` the conjugate
-// (the backward).  Every lane of the wave calls it (the exchange is a
-// shuffle); lanes past the row end carry values that are never stored.
-__device__ __forceinline__ void rope8(float (&x)[8], const Rows& a, int64_t row, int e0,
+// offset e0 of the row, a multiple of whole blocks into the token): x -> the
+// rotated values, with `conj` the conjugate (the backward).  Every lane of the
+// group calls it (the exchange is a shuffle); lanes past the row end carry
+// values that are never stored.
+__device__ __forceinline__ void rope8(float (&x)[8], const Rows& a, int64_t table, int e0,
                                       bool conj) {
-  const int R = a.rope_half;
-  const int tok_pos = (int)((row / a.rows_per_token) % a.seq_len) + a.pos_offset;
-  const int j0 = e0 % (2 * R);
+  const int R = a.rope_half;     // a power of two
+  const int j0 = e0 & (2 * R - 1);
   const bool first = j0 < R;
   const int jj = first ? j0 : j0 - R;
-  const uint4 cu = *reinterpret_cast<const uint4*>(a.cos + (int64_t)tok_pos * R + jj);
-  const uint4 su = *reinterpret_cast<const uint4*>(a.sin + (int64_t)tok_pos * R + jj);
+  const uint4 cu = *reinterpret_cast<const uint4*>(a.cos + table + jj);
+  const uint4 su = *reinterpret_cast<const uint4*>(a.sin + table + jj);
   const uint32_t cw[4] = {cu.x, cu.y, cu.z, cu.w}, sw[4] = {su.x, su.y, su.z, su.w};
   const int dl = R / 8;  // partner lane distance
 #pragma unroll
@@ -119,28 +133,29 @@ __device__ __forceinline__ void rope8(float (&x)[8], const Rows& a, int64_t row,
   }
 }
 
-template <class TI, bool ROPE>
-__global__ __launch_bounds__(256) void rows_prep_kernel(const typename TI::S* __restrict__ in,
+template <class TI, bool ROPE, int G, int NI>
+__global__ __launch_bounds__(kPrepThreads) void rows_prep_kernel(const typename TI::S* __restrict__ in,
                                                         Rows a,
                                                         typename std::conditional<ROPE, BF16T, TI>::type::S* __restrict__ out) {
   using TO = typename std::conditional<ROPE, BF16T, TI>::type;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= a.rows) return;  // wave-uniform
-  const int lane = threadIdx.x & 63;
+  const int64_t row0 = (int64_t)blockIdx.x * (kPrepThreads / G) + threadIdx.x / G;
+  const bool live = row0 < a.rows;
+  const int64_t row = live ? row0 : a.rows - 1;  // every lane takes part in the exchanges
+  const int lane = threadIdx.x % G;
   const int chunks = a.D / 8;
   const typename TI::S* src = in + row * a.ld_in;
   typename TO::S* dst = out + row * a.ld_out;
-  float v[kMaxChunksPerLane][8];
+  float v[NI][8];
 #pragma unroll
-  for (int c = 0; c < kMaxChunksPerLane; ++c) {
-    const int ch = lane + 64 * c;
+  for (int c = 0; c < NI; ++c) {
+    const int ch = lane + G * c;
     // clamped (always valid) address, every load issued before any use
     load8<TI>(src + 8 * (ch < chunks ? ch : chunks - 1), v[c]);
   }
   float ss = 0.0f;
 #pragma unroll
-  for (int c = 0; c < kMaxChunksPerLane; ++c) {
-    const bool ok = lane + 64 * c < chunks;
+  for (int c = 0; c < NI; ++c) {
+    const bool ok = lane + G * c < chunks;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       float x = v[c][u];
@@ -151,15 +166,14 @@ __global__ __launch_bounds__(256) void rows_prep_kernel(const typename TI::S* __
   }
   float den = 1.0f, scale = 1.0f;
   if (a.norm == kL2) {
-    den = sqrtf(wave_sum(ss)) + 1e-5f;
+    den = sqrtf(row_sum<G>(ss)) + 1e-5f;
   } else if (a.norm == kRms) {
-    scale = __builtin_amdgcn_rsqf(wave_sum(ss) / (float)a.D + 1e-5f);
+    scale = __builtin_amdgcn_rsqf(row_sum<G>(ss) / (float)a.D + 1e-5f);
   }
-  const int e_row = ROPE ? (int)(row % a.rows_per_token) * a.D : 0;
+  const int64_t table = ROPE ? rope_row(a, row) : 0;
 #pragma unroll
-  for (int c = 0; c < kMaxChunksPerLane; ++c) {
-    if (64 * c >= chunks) break;  // wave-uniform
-    const int ch = lane + 64 * c;
+  for (int c = 0; c < NI; ++c) {
+    const int ch = lane + G * c;
     float o[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -171,9 +185,9 @@ __global__ __launch_bounds__(256) void rows_prep_kernel(const typename TI::S* __
     if constexpr (ROPE) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) o[u] = rnd<BF16T>(o[u]);  // cast to the tables' dtype
-      rope8(o, a, row, e_row + 8 * (ch < chunks ? ch : chunks - 1), false);
+      rope8(o, a, table, 8 * (ch < chunks ? ch : chunks - 1), false);
     }
-    if (ch < chunks) store8<TO>(dst + 8 * ch, o);
+    if (live && ch < chunks) store8<TO>(dst + 8 * ch, o);
   }
 }
 
@@ -181,39 +195,38 @@ __global__ __launch_bounds__(256) void rows_prep_kernel(const typename TI::S* __
 // conjugate rotation (bf16), the norm's backward on the recomputed silu
 // output (fp32, rounded to the input dtype), the silu backward (rounded to
 // the input dtype).
-template <class TI, bool ROPE>
-__global__ __launch_bounds__(256) void rows_prep_bwd_kernel(
+template <class TI, bool ROPE, int G, int NI>
+__global__ __launch_bounds__(kPrepThreads) void rows_prep_bwd_kernel(
     const typename TI::S* __restrict__ in, Rows a,
     const typename std::conditional<ROPE, BF16T, TI>::type::S* __restrict__ gout,
     typename TI::S* __restrict__ gin) {
   using TO = typename std::conditional<ROPE, BF16T, TI>::type;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= a.rows) return;  // wave-uniform
-  const int lane = threadIdx.x & 63;
+  const int64_t row0 = (int64_t)blockIdx.x * (kPrepThreads / G) + threadIdx.x / G;
+  const bool live = row0 < a.rows;
+  const int64_t row = live ? row0 : a.rows - 1;  // every lane takes part in the exchanges
+  const int lane = threadIdx.x % G;
   const int chunks = a.D / 8;
   const typename TI::S* src = in + row * a.ld_in;
   const typename TO::S* gsrc = gout + row * a.ld_out;
   typename TI::S* dst = gin + row * a.ld_in;
-  float x[kMaxChunksPerLane][8], g[kMaxChunksPerLane][8];
+  float x[NI][8], g[NI][8];
 #pragma unroll
-  for (int c = 0; c < kMaxChunksPerLane; ++c) {
-    const int ch = lane + 64 * c;
+  for (int c = 0; c < NI; ++c) {
+    const int ch = lane + G * c;
     const int cc = ch < chunks ? ch : chunks - 1;
     load8<TI>(src + 8 * cc, x[c]);
     load8<TO>(gsrc + 8 * cc, g[c]);
   }
-  const int e_row = ROPE ? (int)(row % a.rows_per_token) * a.D : 0;
+  const int64_t table = ROPE ? rope_row(a, row) : 0;
   float ss = 0.0f, dot = 0.0f;
 #pragma unroll
-  for (int c = 0; c < kMaxChunksPerLane; ++c) {
-    const int ch = lane + 64 * c;
+  for (int c = 0; c < NI; ++c) {
+    const int ch = lane + G * c;
     const bool ok = ch < chunks;
     if constexpr (ROPE) {
-      if (64 * c < chunks) {  // wave-uniform
-        rope8(g[c], a, row, e_row + 8 * (ok ? ch : chunks - 1), true);
+      rope8(g[c], a, table, 8 * (ok ? ch : chunks - 1), true);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) g[c][u] = rnd<TI>(rnd<BF16T>(g[c][u]));
-      }
+      for (int u = 0; u < 8; ++u) g[c][u] = rnd<TI>(rnd<BF16T>(g[c][u]));
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -226,19 +239,19 @@ __global__ __launch_bounds__(256) void rows_prep_bwd_kernel(
   }
   float den = 1.0f, coef = 0.0f, scale = 1.0f;
   if (a.norm == kL2) {
-    const float n = sqrtf(wave_sum(ss));
-    dot = wave_sum(dot);
+    const float n = sqrtf(row_sum<G>(ss));
+    dot = row_sum<G>(dot);
     den = n + 1e-5f;
     coef = n > 0.0f ? dot / (n * den * den) : 0.0f;
   } else if (a.norm == kRms) {
-    scale = __builtin_amdgcn_rsqf(wave_sum(ss) / (float)a.D + 1e-5f);
-    dot = wave_sum(dot);
+    scale = __builtin_amdgcn_rsqf(row_sum<G>(ss) / (float)a.D + 1e-5f);
+    dot = row_sum<G>(dot);
     coef = dot * scale * scale * scale / (float)a.D;
   }
 #pragma unroll
-  for (int c = 0; c < kMaxChunksPerLane; ++c) {
-    const int ch = lane + 64 * c;
-    if (ch >= chunks) continue;
+  for (int c = 0; c < NI; ++c) {
+    const int ch = lane + G * c;
+    if (!live || ch >= chunks) continue;
     float o[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -309,6 +322,35 @@ Rows make_rows(int64_t rows, int D, int64_t ld_in, int64_t ld_out, int silu, int
   return a;
 }
 
+// f(G, NI): the fewest lanes per row (at least 8 and whole rotary blocks) that
+// hold it in at most four chunks each, rounded up to a compiled chunk count.
+template <class F>
+void prep_dispatch(int D, int rope_half, F&& f) {
+  const int CH = D / 8, block = rope_half / 4;
+  int g = 8;
+  while (g < 64 && (4 * g < CH || g < block)) g *= 2;
+  const int ni = (CH + g - 1) / g;
+  auto with = [&](auto G) {
+    if (ni <= 1) f(G, std::integral_constant<int, 1>{});
+    else if (ni <= 3) f(G, std::integral_constant<int, 3>{});
+    else f(G, std::integral_constant<int, 4>{});
+  };
+  switch (g) {
+    case 8: with(std::integral_constant<int, 8>{}); break;
+    case 16: with(std::integral_constant<int, 16>{}); break;
+    case 32: with(std::integral_constant<int, 32>{}); break;
+    default:
+      if (ni > 4)
+        f(std::integral_constant<int, 64>{}, std::integral_constant<int, kMaxChunksPerLane>{});
+      else
+        with(std::integral_constant<int, 64>{});
+  }
+}
+inline unsigned prep_blocks(int64_t rows, int g) {
+  const int per = kPrepThreads / g;
+  return (unsigned)((rows + per - 1) / per);
+}
+
 }  // namespace
 }  // namespace uttt
 
@@ -326,16 +368,19 @@ extern "C" int uttt_rows_preprocess(const void* in, int dtype, int64_t rows, int
   UTTT_REQUIRE(rope_dim == 0 || pos_offset + seq_len <= table_rows,
                "rows_preprocess: positions up to %d past the rotary table's %d rows",
                pos_offset + seq_len, table_rows);
-  const unsigned blocks = (unsigned)((rows + 3) / 4);
   hipStream_t st = as_stream(stream);
   UTTT_DTYPE_SWITCH_LR(dtype, TT, {
     using S = typename TT::S;
-    if (rope_dim > 0)
-      hipLaunchKernelGGL((rows_prep_kernel<TT, true>), dim3(blocks), dim3(256), 0, st,
-                         static_cast<const S*>(in), a, static_cast<uint16_t*>(out));
-    else
-      hipLaunchKernelGGL((rows_prep_kernel<TT, false>), dim3(blocks), dim3(256), 0, st,
-                         static_cast<const S*>(in), a, static_cast<S*>(out));
+    prep_dispatch(D, a.rope_half, [&](auto g, auto ni) {
+      constexpr int G = decltype(g)::value, NI = decltype(ni)::value;
+      const dim3 grid(prep_blocks(rows, G));
+      if (rope_dim > 0)
+        hipLaunchKernelGGL((rows_prep_kernel<TT, true, G, NI>), grid, dim3(kPrepThreads), 0, st,
+                           static_cast<const S*>(in), a, static_cast<uint16_t*>(out));
+      else
+        hipLaunchKernelGGL((rows_prep_kernel<TT, false, G, NI>), grid, dim3(kPrepThreads), 0, st,
+                           static_cast<const S*>(in), a, static_cast<S*>(out));
+    });
   });
   return check_launch("rows_preprocess");
 }
@@ -355,18 +400,21 @@ extern "C" int uttt_rows_preprocess_bwd(const void* in, int dtype, const void* g
   UTTT_REQUIRE(rope_dim == 0 || pos_offset + seq_len <= table_rows,
                "rows_preprocess_bwd: positions up to %d past the rotary table's %d rows",
                pos_offset + seq_len, table_rows);
-  const unsigned blocks = (unsigned)((rows + 3) / 4);
   hipStream_t st = as_stream(stream);
   UTTT_DTYPE_SWITCH_LR(dtype, TT, {
     using S = typename TT::S;
-    if (rope_dim > 0)
-      hipLaunchKernelGGL((rows_prep_bwd_kernel<TT, true>), dim3(blocks), dim3(256), 0, st,
-                         static_cast<const S*>(in), a, static_cast<const uint16_t*>(grad_out),
-                         static_cast<S*>(grad_in));
-    else
-      hipLaunchKernelGGL((rows_prep_bwd_kernel<TT, false>), dim3(blocks), dim3(256), 0, st,
-                         static_cast<const S*>(in), a, static_cast<const S*>(grad_out),
-                         static_cast<S*>(grad_in));
+    prep_dispatch(D, a.rope_half, [&](auto g, auto ni) {
+      constexpr int G = decltype(g)::value, NI = decltype(ni)::value;
+      const dim3 grid(prep_blocks(rows, G));
+      if (rope_dim > 0)
+        hipLaunchKernelGGL((rows_prep_bwd_kernel<TT, true, G, NI>), grid, dim3(kPrepThreads), 0, st,
+                           static_cast<const S*>(in), a, static_cast<const uint16_t*>(grad_out),
+                           static_cast<S*>(grad_in));
+      else
+        hipLaunchKernelGGL((rows_prep_bwd_kernel<TT, false, G, NI>), grid, dim3(kPrepThreads), 0,
+                           st, static_cast<const S*>(in), a, static_cast<const S*>(grad_out),
+                           static_cast<S*>(grad_in));
+    });
   });
   return check_launch("rows_preprocess_bwd");
 }
