@@ -1,0 +1,71 @@
+"""The narrow-expert UPDATE kernels (csrc/narrow.hip: 64 hidden units x 128
+tokens, stages of 32 k) against the general tiles, which the reference-layout
+output and the backward without saved tensors take.  Both multiply in the same
+order and round at the same places: stage 1, whose pointwise part has one way
+to contract its multiply-adds, gives the same bits; the backward's may contract
+differently, so an intermediate can land on the other side of a rounding tie
+(one bf16 ulp, 2^-8, of a few elements)."""
+import pytest
+import torch
+
+from uttt_amd.lact_moe_triton import _grouped as G
+from uttt_amd.lact_moe_triton import _update_bwd as UB
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# (group sizes per batch, D, I, N or None): one and several unit and token
+# tiles, their remainders, a k tail, two stages (the smallest), the widest
+CASES = {
+    "tile_edges": ([[128, 129, 0, 127, 256, 31, 33, 1]], 192, 192, None),
+    "ragged_two_batches": ([[70, 0, 130], [1, 199, 0]], 200, 104, None),
+    "two_stages_one_unit_group": ([[5, 300, 2]], 40, 8, None),
+    "widest": ([[33, 200]], 512, 512, None),
+    "over_64_experts": ([[7 * (i % 5) for i in range(70)]], 64, 72, None),
+    "slack_rows": ([[60, 40]], 384, 384, 160),
+    "over_count": ([[60, 90, 70]], 96, 200, 140),
+    "all_empty": ([[0, 0, 0]], 192, 64, 32),
+}
+
+
+@pytest.mark.parametrize("lr_dtype", [torch.bfloat16, torch.float32, None])
+@pytest.mark.parametrize("name", list(CASES))
+def test_narrow_update_equals_general_tiles(name, lr_dtype):
+    sizes, D, I, N = CASES[name]
+    gs = torch.tensor(sizes, dtype=torch.int32, device=DEV)
+    B, E = gs.shape
+    N = int(gs.sum(1).max()) if N is None else N
+    g = torch.Generator().manual_seed(N + D)
+    rnd = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).to(torch.bfloat16).to(DEV)
+    W02, gW02 = (rnd(B, E, 2 * I, D, scale=D ** -0.5) for _ in range(2))
+    W1, gW1 = (rnd(B, E, D, I, scale=I ** -0.5) for _ in range(2))
+    K, V = rnd(B, N, D), rnd(B, N, D)
+    lrs = [None] * 3 if lr_dtype is None else \
+        [torch.rand(B, N, generator=g).to(lr_dtype).to(DEV) for _ in range(3)]
+    rows = torch.arange(N, device=DEV) < gs.sum(1, keepdim=True).clamp(max=N)  # [B, N] routed
+
+    dy, hid, ys, dhs = G.update_stage1(W02, W1, K, V, *lrs, gs, True, save=True)
+    dy_g, hid_g = G.update_stage1(W02, W1, K, V, *lrs, gs, False)
+    for a, b in ((dy, dy_g), (hid, hid_g)):
+        assert torch.equal(a[rows], b.transpose(1, 2)[rows])
+    plain = G.update_stage1(W02, W1, K, V, *lrs, gs, True)
+    assert torch.equal(plain[0][rows], dy[rows]) and torch.equal(plain[1][rows], hid[rows])
+    if lr_dtype is None:
+        return
+
+    ours = UB._backward(W02, W1, K, V, *lrs, gs, gW02, gW1, ys, dhs)
+    gen = UB._backward(W02, W1, K, V, *lrs, gs, gW02, gW1, None, None)
+    # 2^-8 of the whole if every element of an intermediate were an ulp off; one
+    # wrong token row of n would be n ** -0.5
+    for a, b in zip(ours[:4], gen[:4]):
+        if a.shape[:2] == (B, N):
+            a, b = a[rows], b[rows]
+        assert (a.double() - b.double()).norm() <= 2.0 ** -8 * b.double().norm()
+    # one output rounding where a sum lands on the other side of a tie, and the
+    # fp32 sums of I products of about one in two orders
+    ulp = 2.0 ** -7 if lr_dtype == torch.bfloat16 else 0.0
+    for a, b in zip(ours[4:], gen[4:]):
+        a, b = a.double(), b.double()
+        assert bool((a[~rows] == 0).all())
+        scale = max(1.0, b.abs().max().item())
+        assert bool(((a - b).abs() <= ulp * b.abs() + I * 2.0 ** -23 * scale).all())

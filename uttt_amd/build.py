@@ -40,7 +40,7 @@ COMMON_FLAGS = [
 # the value from before the read;
 # the one-launch Newton-Schulz holds its accumulators and the products it
 # writes back across barriers, where a spill would cost more than the work.
-NO_SCRATCH = {"grouped_gemm.hip", "tile192.hip", "ns_small.hip", "dense_update.hip"}
+NO_SCRATCH = {"grouped_gemm.hip", "tile192.hip", "narrow.hip", "ns_small.hip", "dense_update.hip"}
 
 
 def _scratch_kernels(remarks: str) -> list:

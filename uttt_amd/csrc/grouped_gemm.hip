@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "gemm_pipe.h"
+#include "narrow.h"
 #include "tile192_host.h"
 
 namespace uttt {
@@ -1941,6 +1942,10 @@ extern "C" int uttt_grouped_update_stage1(const void* w0_w2, const void* w1, con
   UTTT_REQUIRE(workspace_bytes >= need, "grouped_update_stage1: workspace %zu < %zu bytes",
                workspace_bytes, need);
   hipStream_t st = as_stream(stream);
+  if (token_major && narrow_experts(I, D))
+    return launch_narrow_stage1(w0_w2, w1, k, v, lr0, lr1, lr2, lr_dtype, group_sizes, B, E, I, D, N,
+                                dy0_dy2, hidden, y0_y2_save, dh_save, st,
+                                "grouped_update_stage1");
   float* dh = static_cast<float*>(workspace);
   // DH = w1^T v (fp32, token-major [N, I]): the reference keeps DH in fp32
   if (int rc = launch_wide<RMajor>(w1, v, D, nullptr, nullptr, 0, I, I, (int64_t)D * I, dh, B, E,
@@ -2075,7 +2080,8 @@ struct UpdateBwdWs {
 };
 UpdateBwdWs update_bwd_ws(int B, int I, int N) {
   const size_t t2 = up256((size_t)B * N * 2 * I * 2), t1 = up256((size_t)B * N * I * 2);
-  const int m_tiles = (I + kTileRows - 1) / kTileRows;
+  // one row per 128 hidden units, or per block of the narrow kernels
+  const int m_tiles = std::max((I + kTileRows - 1) / kTileRows, I <= 512 ? narrow_m_tiles(I) : 0);
   UpdateBwdWs w;
   w.dhg = 0;
   w.gy = w.dhg + t2;
@@ -2133,7 +2139,19 @@ extern "C" int uttt_grouped_update_bwd(
   const int64_t g02 = (int64_t)2 * I * D, g1 = (int64_t)D * I;
   const int m_tiles = (I + kTileRows - 1) / kTileRows;
 
-  if (y0_y2_saved != nullptr) {
+  if (y0_y2_saved != nullptr && narrow_experts(I, D)) {
+    if (int rc = launch_narrow_bwd(grad_dw0_w2, grad_dw1, k, v, lr0, lr1, lr2, lr_dtype, group_sizes,
+                                   B, E, I, D, N, y0_y2_saved, dh_saved, gdh, gx, dx, hlr, part, st,
+                                   "grouped_update_bwd(second order)"))
+      return rc;
+    UTTT_DTYPE_SWITCH_LR(lr_dtype, LR, {
+      using S = typename LR::S;
+      hipLaunchKernelGGL((lr_grad_reduce_kernel<LR>), dim3((N + 255) / 256, B), dim3(256), 0, st,
+                         part, group_sizes, B, E, N, narrow_m_tiles(I), static_cast<S*>(grad_lr0),
+                         static_cast<S*>(grad_lr1), static_cast<S*>(grad_lr2));
+      if (int rc = check_launch("grouped_update_bwd(lr grads)")) return rc;
+    });
+  } else if (y0_y2_saved != nullptr) {
     // from the forward's saved bf16 Y0 | Y2 and DH: GD = gw1^T v (bf16 [N, I]),
     // then GY0 | GY2 = gw0_w2 k with the second-order pass on the registers
     uint16_t* gd = dhg;

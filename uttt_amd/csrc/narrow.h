@@ -1,0 +1,28 @@
+// Host side of the narrow-expert UPDATE kernels (narrow.hip).
+#pragma once
+
+#include "common.h"
+
+namespace uttt {
+
+// Expert widths that narrow.hip's kernels take (any token counts).
+bool narrow_experts(int I, int D);
+// Row blocks of its lr-gradient partials, lr_part[3][narrow_m_tiles][B][N].
+int narrow_m_tiles(int I);
+
+// Stage 1 with token-major outputs (uttt_grouped_update_stage1) without the
+// fp32 workspace; lr0 .. lr2 and the saves may be null.
+int launch_narrow_stage1(const void* w0_w2, const void* w1, const void* k, const void* v,
+                         const void* lr0, const void* lr1, const void* lr2, int lr_dtype,
+                         const int32_t* gs, int B, int E, int I, int D, int N, void* dy, void* hid,
+                         void* y_save, void* dh_save, hipStream_t st, const char* what);
+
+// The backward's second-order pass from the saved values: grad_dh [B, N, I],
+// grad_x0_x2 and dx0_x2 [B, N, 2I], hidden_lr1 [B, N, I], lr-gradient partials.
+int launch_narrow_bwd(const void* gw0_w2, const void* gw1, const void* k, const void* v,
+                      const void* lr0, const void* lr1, const void* lr2, int lr_dtype,
+                      const int32_t* gs, int B, int E, int I, int D, int N, const void* y_saved,
+                      const void* dh_saved, uint16_t* gdh, uint16_t* gx, uint16_t* dx,
+                      uint16_t* hlr, float* lr_part, hipStream_t st, const char* what);
+
+}  // namespace uttt

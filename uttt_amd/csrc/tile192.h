@@ -43,21 +43,22 @@ constexpr int kTThreads = 256;
 constexpr int kTLoads = kTTile / 16 / kTThreads;  // 3 loads per wave and operand tile
 constexpr int kTItems = kWT * (kT / 8) / kTThreads;  // epilogue items per thread and half
 
-// The loads of one operand's 192-row tile over a K loop (see TileLoader in
+// The loads of one operand's tile of ROWS rows over a K loop (see TileLoader in
 // gemm_pipe.h: rows past the end repeat the last valid row, k past the end
-// reads zeros through the descriptor's record bound).  `split`: tile rows from
-// `split` on are operand rows r2 + (row - split) instead (two row blocks of
-// one matrix in one tile; KMajor only).
-template <int MAJOR>
+// reads zeros through the descriptor's record bound).  `split` (KMajor): tile
+// rows from `split` on are the operand's rows r0 .. again, `second` elements
+// further on (two row blocks of one matrix in one tile).
+template <int MAJOR, int ROWS = kT>
 struct Loader {
+  static constexpr int kLoads = ROWS * kTK * 2 / 16 / kTThreads;
   const uint8_t* base;
   int64_t kstep;
   int last, k_end, ld2, col2;
-  uint32_t off[kTLoads];
+  uint32_t off[kLoads];
   int wofs;
 
-  __device__ __forceinline__ void init(const Operand& op, int r0, int split = kT, int r2 = 0,
-                                       int rows2 = 0) {
+  __device__ __forceinline__ void init(const Operand& op, int r0, int split = ROWS,
+                                       int second = 0) {
     const int lane = threadIdx.x & 63;
     const int w = wave_id();
     k_end = op.k_end;
@@ -78,22 +79,16 @@ struct Loader {
     base = uniform_ptr(reinterpret_cast<const uint8_t*>(org));
     kstep = MAJOR == KMajor ? (int64_t)kTK * 2 : (int64_t)kTK * op.ld * 2;
 #pragma unroll
-    for (int t = 0; t < kTLoads; ++t) {
+    for (int t = 0; t < kLoads; ++t) {
       const int s = (t * 4 + w) * 64 + lane;
       if constexpr (MAJOR == KMajor) {
         const int r = s >> 2;
         const int c = (s & 3) ^ ((r >> 2) & 3);
-        int rr = r < nrows ? r : nrows - 1;
-        if (split < kT) {
-          // r2 - r0 rows further on (a constant offset inside the matrix)
-          if (r >= split)
-            rr = r2 - r0 + (r - split < rows2 ? r - split : rows2 - 1);
-          else
-            rr = r < nrows && r < split ? r : (nrows < split ? nrows : split) - 1;
-        }
-        off[t] = (uint32_t)(rr * (int)op.ld + c * 8) * 2u;
+        const int rr = r < split ? r : r - split;
+        off[t] = (uint32_t)((rr < nrows ? rr : nrows - 1) * (int)op.ld + c * 8 +
+                            (r < split ? 0 : second)) * 2u;
       } else {
-        const int k = s / 24, cc = s - k * 24;
+        const int k = s / (ROWS / 8), cc = s - k * (ROWS / 8);
         const int c = cc ^ (((k >> 1) & 1) << 2);
         const int cmax = (nrows >> 3) - 1;
         off[t] = (uint32_t)(k * (int)op.ld + (c < cmax ? c : cmax) * 8) * 2u;
@@ -115,7 +110,7 @@ struct Loader {
         recs = 0xFFFFFF00u;
         const int lane = threadIdx.x & 63, w = wofs >> 10, kt = k_end % kTK;
 #pragma unroll
-        for (int t = 0; t < kTLoads; ++t) {
+        for (int t = 0; t < kLoads; ++t) {
           const int sl = (t * 4 + w) * 64 + lane;
           const int r = sl >> 2;
           if (((sl & 3) ^ ((r >> 2) & 3)) * 8 >= kt) off[t] = 0xFFFFFFF0u;
@@ -125,7 +120,7 @@ struct Loader {
     const Rsrc rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(sb), (short)0,
                                                       (int)recs, kBufferWord3);
 #pragma unroll
-    for (int t = 0; t < kTLoads; ++t)
+    for (int t = 0; t < kLoads; ++t)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, UTTT_LDS(dst + t * 4096 + wofs), 16, off[t], 0,
                                                0, 0);
   }
