@@ -5,9 +5,12 @@ order and round at the same places: stage 1, whose pointwise part has one way
 to contract its multiply-adds, gives the same bits; the backward's may contract
 differently, so an intermediate can land on the other side of a rounding tie
 (one bf16 ulp, 2^-8, of a few elements)."""
+import contextlib
+
 import pytest
 import torch
 
+from uttt_amd import _lib as L
 from uttt_amd.lact_moe_triton import _grouped as G
 from uttt_amd.lact_moe_triton import _update_bwd as UB
 
@@ -69,3 +72,60 @@ def test_narrow_update_equals_general_tiles(name, lr_dtype):
         assert bool((a[~rows] == 0).all())
         scale = max(1.0, b.abs().max().item())
         assert bool(((a - b).abs() <= ulp * b.abs() + I * 2.0 ** -23 * scale).all())
+
+
+@contextlib.contextmanager
+def general_tiles():
+    """The 256-token tiles: a forced wave layout takes every product there."""
+    prev = L.lib().uttt_debug_set_gemm_layout(2)
+    try:
+        yield
+    finally:
+        L.lib().uttt_debug_set_gemm_layout(prev)
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_narrow_products_equal_general_tiles(name):
+    """Gate/up (rows in expert order and gathered) and the plain and chained
+    products (192 x 192 tiles): the same multiplications in the same order."""
+    sizes, D, I, N = CASES[name]
+    gs = torch.tensor(sizes, dtype=torch.int32, device=DEV)
+    B, E = gs.shape
+    N = int(gs.sum(1).max()) if N is None else N
+    g = torch.Generator().manual_seed(N + I)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    W02, W1, W2 = rnd(B, E, 2 * I, D), rnd(B, E, D, I), rnd(B, E, D, I)
+    X, H, H2, Y = rnd(B, N, D), rnd(B, N, I), rnd(B, N, I), rnd(B, N, 2 * I)
+    rows = torch.arange(N, device=DEV) < gs.sum(1, keepdim=True).clamp(max=N)
+    src = torch.randint(0, N, (B, N), generator=g, dtype=torch.int32).to(DEV)
+
+    def products():
+        out = [G.gate_up(W02, X, gs, token_major=True), G.gemm_nt(W1, H, gs), G.gemm_tn(W1, X, gs),
+               G.gemm_tn(W02, Y, gs), G.gemm_nt2(W1, H, W2, H2, gs), G.gemm_tn2(W1, X, W2, X, gs)]
+        if G.gate_up_gathers(N, E):
+            out.append(G.gate_up_gather(W02, X, src, gs))
+        return out
+
+    ours = products()
+    with general_tiles():
+        general = products()
+    for i, (a, b) in enumerate(zip(ours, general, strict=True)):
+        assert torch.equal(a[rows], b[rows]), i
+
+
+def test_short_segments_on_192_tiles_equal_general_tiles():
+    """Experts past the narrow widths with at most 256 tokens each."""
+    gs = torch.tensor([[200, 0, 193, 1, 300, 192]], dtype=torch.int32, device=DEV)
+    B, E, D, I, N = 1, 6, 520, 776, 890
+    g = torch.Generator().manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    W02, W1, W2 = rnd(B, E, 2 * I, D), rnd(B, E, D, I), rnd(B, E, D, I)
+    X, H, Y = rnd(B, N, D), rnd(B, N, I), rnd(B, N, 2 * I)
+    products = lambda: [G.gemm_tn(W02, Y, gs), G.gemm_nt2(W1, H, W2, H, gs),
+                        G.gemm_tn2(W02, Y, W02, Y, gs)]
+    ours = products()
+    with general_tiles():
+        general = products()
+    n = int(gs.sum())
+    for a, b in zip(ours, general):
+        assert torch.equal(a[:, :n], b[:, :n])

@@ -1600,6 +1600,11 @@ bool use_apply_kernel(int64_t N, int E) {
          (g_apply_path < 0 && N <= (int64_t)kBRows * E);
 }
 
+bool general_forced();
+bool use_narrow_gate_up(int I, int D) {
+  return g_apply_path < 0 && narrow_experts(I, D) && !general_forced();
+}
+
 // The down projection (and every uttt_grouped_gemm_nt): the skinny tiles
 // (128 weight rows x 128 tokens) when the general 256x256 tiles would not
 // fill the chip once even at their upper-bound count, else the general tiles.
@@ -1654,12 +1659,36 @@ ApArgs apply_args(const void* w, const void* x, int K, int64_t a_group, int row_
   return a;
 }
 
+// Tests force a layout or tile order of the general tiles: everything takes them then.
+bool general_forced() { return g_gemm_na != 0 || g_xcd_map_min_tiles != kXcdMapMinTiles; }
+
+// bf16 products on 192 x 192 tiles with two workgroups per CU instead of 256 x
+// 256 with one (the same bits):
+//   - narrow experts (M <= 512 rows, K <= 1024), bound by the token rows: 48
+//     experts of 192 x 192 over 196 608 tokens 107 -> 88 us (grad_K) and 70 ->
+//     55 (grad_V); 96 of 384 x 384 over 16 384 evenly / unevenly routed ones 43
+//     -> 36 / 77 -> 49 and 26 -> 23 / 40 -> 32;
+//   - short segments (at most 256 tokens per expert on average) of experts up
+//     to 768 x 3072: 16 over 3062 tokens 120 -> 112 and 66 -> 60 us.
+// Larger experts re-read their weights per 192 tokens from beyond the L2: 32 of
+// 1536 x 3072 over 4096 unevenly routed tokens 358 / 401 us, over 98 304 3176 /
+// 3540; 16 of 768 x 1536 over 49 152 257 / 265 (grad_V).
+bool use_tn192(int M, int K, int N, int E) {
+  if (general_forced() || K <= 0) return false;
+  return (M <= 512 && K <= 1024) ||
+         (N <= 256 * (int64_t)E && (int64_t)M * K <= (int64_t)768 * 3072);
+}
+
 // Wide single product: y[b, n, m] = sum_k A(m, k) x[b, n, k] with M rows in
 // m-tiles of 256 (tile 1 = rows +128).  Optional second pair chained on K.
 template <int AMAJ, class OutT>
 int launch_wide(const void* a, const void* x, int K, const void* a_2, const void* x_2, int K_2,
                 int M, int64_t lda, int64_t a_group, OutT* y, int B, int E, int N,
                 const int32_t* gs, hipStream_t st, const char* what) {
+  if constexpr (std::is_same_v<OutT, uint16_t>) {
+    if (aligned16(y) && use_tn192(M, K, N, E))
+      return launch_tn192(AMAJ == KMajor, a, x, K, a_2, x_2, K_2, M, y, B, E, N, gs, st, what);
+  }
   TnArgs t = tn_args(a, a, x, K, lda, a_group, 0, kTileRows, M, M, 2 * kTileRows, M, B, E, N, gs);
   if (K_2 > 0) {
     t.a[1][0] = t.a[1][1] = static_cast<const uint16_t*>(a_2);
@@ -1776,6 +1805,9 @@ extern "C" int uttt_grouped_gate_up(const void* w0_w2, const void* x, const int3
   UTTT_REQUIRE(w0_w2 && x && group_sizes && hidden, "grouped_gate_up: null pointer");
   UTTT_REQUIRE(aligned16(w0_w2) && aligned16(x) && aligned16(hidden),
                "grouped_gate_up: tensors must be 16-byte aligned");
+  if (token_major && use_narrow_gate_up(I, D))
+    return launch_narrow_gate_up(w0_w2, x, nullptr, 0, group_sizes, B, E, I, D, N, 0, hidden,
+                                 as_stream(stream), "grouped_gate_up");
   if (token_major && use_apply_kernel(N, E)) {
     const ApArgs a = apply_args(w0_w2, x, D, (int64_t)2 * I * D, I, I, 2 * I, kTileRows, B, E, N,
                                 group_sizes);
@@ -1811,6 +1843,9 @@ extern "C" int uttt_grouped_gate_up_gather(const void* w0_w2, const void* x, int
                "grouped_gate_up_gather: null pointer");
   UTTT_REQUIRE(aligned16(w0_w2) && aligned16(x) && aligned16(hidden),
                "grouped_gate_up_gather: tensors must be 16-byte aligned");
+  if (use_narrow_gate_up(I, D))
+    return launch_narrow_gate_up(w0_w2, x, src_rows, src_sb, group_sizes, B, E, I, D, N, T, hidden,
+                                 as_stream(stream), "grouped_gate_up_gather");
   ApArgs a = apply_args(w0_w2, x, D, (int64_t)2 * I * D, I, I, 2 * I, kTileRows, B, E, N,
                         group_sizes);
   a.src = src_rows;
@@ -1942,7 +1977,7 @@ extern "C" int uttt_grouped_update_stage1(const void* w0_w2, const void* w1, con
   UTTT_REQUIRE(workspace_bytes >= need, "grouped_update_stage1: workspace %zu < %zu bytes",
                workspace_bytes, need);
   hipStream_t st = as_stream(stream);
-  if (token_major && narrow_experts(I, D))
+  if (token_major && narrow_experts(I, D) && !general_forced())
     return launch_narrow_stage1(w0_w2, w1, k, v, lr0, lr1, lr2, lr_dtype, group_sizes, B, E, I, D, N,
                                 dy0_dy2, hidden, y0_y2_save, dh_save, st,
                                 "grouped_update_stage1");
@@ -2139,7 +2174,7 @@ extern "C" int uttt_grouped_update_bwd(
   const int64_t g02 = (int64_t)2 * I * D, g1 = (int64_t)D * I;
   const int m_tiles = (I + kTileRows - 1) / kTileRows;
 
-  if (y0_y2_saved != nullptr && narrow_experts(I, D)) {
+  if (y0_y2_saved != nullptr && narrow_experts(I, D) && !general_forced()) {
     if (int rc = launch_narrow_bwd(grad_dw0_w2, grad_dw1, k, v, lr0, lr1, lr2, lr_dtype, group_sizes,
                                    B, E, I, D, N, y0_y2_saved, dh_saved, gdh, gx, dx, hlr, part, st,
                                    "grouped_update_bwd(second order)"))

@@ -17,6 +17,12 @@ int launch_narrow_stage1(const void* w0_w2, const void* w1, const void* k, const
                          const int32_t* gs, int B, int E, int I, int D, int N, void* dy, void* hid,
                          void* y_save, void* dh_save, hipStream_t st, const char* what);
 
+// The APPLY's gate/up, hidden [B, N, I] = silu(w0 x) * (w2 x); src_rows (rows of
+// src_sb entries, or null): row n of batch b is row src_rows[b][n] of x [B, T, D].
+int launch_narrow_gate_up(const void* w0_w2, const void* x, const int32_t* src_rows,
+                          long long src_sb, const int32_t* gs, int B, int E, int I, int D, int N,
+                          int T, void* hidden, hipStream_t st, const char* what);
+
 // The backward's second-order pass from the saved values: grad_dh [B, N, I],
 // grad_x0_x2 and dx0_x2 [B, N, 2I], hidden_lr1 [B, N, I], lr-gradient partials.
 int launch_narrow_bwd(const void* gw0_w2, const void* gw1, const void* k, const void* v,

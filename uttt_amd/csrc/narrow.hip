@@ -1,5 +1,5 @@
 // The grouped UPDATE's token products for narrow experts (I, D <= 512), one
-// launch instead of two and no fp32 intermediate.
+// launch instead of two and no fp32 intermediate, and the APPLY's gate/up.
 //
 // At the shipped expert widths (192 x 192, 384 x 384) the UPDATE's first stage
 // multiplies each token by three small matrices and writes six rows of results:
@@ -18,7 +18,8 @@
 // 48 experts of 192 x 192 over 196 608 tokens, bound by the rows' stream:
 //   stage 1 with the saves  273 us (two launches) -> 158 (600 MB, 3.8 TB/s)
 //   backward's second pass  302 us (two launches) -> 223 (830 MB, 3.7 TB/s)
-// 96 of 384 x 384 over 16 384 tokens, without saves: 89 -> 45 us.
+// 96 of 384 x 384 over 16 384 tokens, without saves: 89 -> 45 us; gate/up 42 ->
+// 31, of 48 x 192 x 192 17 -> 10.7 (against apply_kernel's 256 x 128 tiles).
 // Past 512 the products outweigh the rows and a token tile is read by more
 // than eight unit groups: the 256-token tiles' kernels.
 #include "narrow.h"
@@ -48,6 +49,9 @@ struct NarrowArgs {
   const uint16_t* v;    // [B, N, D]
   const int32_t* gs;
   int B, E, I, D, N, m_tiles, n_tiles_ub;
+  const int32_t* src;   // gate/up: rows of k [B, T, D] (optional)
+  long long src_sb;
+  int T;
 };
 
 // s_waitcnt lgkmcnt(N) that redefines the fragment registers.
@@ -153,11 +157,36 @@ __device__ __forceinline__ void unpack4(uint32_t x, uint32_t y, float (&v)[4]) {
   v[3] = bf16_to_f32((uint16_t)(y >> 16));
 }
 
+// --- APPLY gate/up (y0 = w0 x, y2 = w2 x)
+struct NarrowSwiGLU {
+  static constexpr int kWgsPerCu = 3;
+  static constexpr bool kThree = false;
+  struct Args {
+    uint16_t* hid;  // [B, N, I]
+  };
+  __device__ __forceinline__ static void apply(const Args& ea, const NarrowArgs& a,
+                                               const WaveCtx& c, const f32x16 (&)[2],
+                                               const f32x16 (&y)[4]) {
+    static_for<8>([&](auto Q) __attribute__((always_inline)) {
+      constexpr int i = decltype(Q)::value / 4, q = decltype(Q)::value % 4;
+      float y0[4], y2[4], h[4];
+      quad(y[i], q, y0);
+      quad(y[2 + i], q, y2);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) h[u] = y2[u] * (y0[u] * sigmoidf_(y0[u]));
+      c.put(0, i, q, h);
+    });
+    WaveCtx::fence();
+    c.store(0, ea.hid, a.I, 0, a.I);
+  }
+};
+
 // --- UPDATE stage 1 (dh = w1^T v, y0 = w0 k, y2 = w2 k): as EpiS1 of
 // grouped_gemm.hip, the same operations on the same values.
 template <class LR>
 struct NarrowS1 {
   static constexpr int kWgsPerCu = 3;
+  static constexpr bool kThree = true;  // the w1 product too
   using S = typename LR::S;
   struct Args {
     const S *lr0, *lr1, *lr2;           // [B, N] or null (1)
@@ -224,6 +253,7 @@ struct NarrowS1 {
 template <class LR>
 struct NarrowBwd {
   static constexpr int kWgsPerCu = 2;
+  static constexpr bool kThree = true;
   using S = typename LR::S;
   struct Args {
     const uint16_t *y_saved, *dh_saved;  // [B, N, 2I], [B, N, I]
@@ -426,10 +456,20 @@ __device__ __forceinline__ void narrow_body(const NarrowArgs& a, const typename 
   Loader<RMajor, kHid> l1;        // w1[:, h0 ..]
   Loader<KMajor, 2 * kHid> l02;   // w0[h0 ..] | w2[h0 ..]
   Loader<KMajor, kTok> lv, lk;
-  l1.init(Operand{a.w1 + ge * a.D * a.I, a.I, a.I, a.D}, h0);
-  lv.init(Operand{a.v + row * a.D, a.D, tt.size, a.D}, tt.n0);
+  if constexpr (Epi::kThree) {
+    l1.init(Operand{a.w1 + ge * a.D * a.I, a.I, a.I, a.D}, h0);
+    lv.init(Operand{a.v + row * a.D, a.D, tt.size, a.D}, tt.n0);
+  }
   l02.init(Operand{a.w02 + ge * 2 * a.I * a.D, a.D, a.I, a.D}, h0, kHid, a.I * a.D);
-  lk.init(Operand{a.k + row * a.D, a.D, tt.size, a.D}, tt.n0);
+  if (!Epi::kThree && a.src != nullptr) {
+    const int32_t* src = a.src + (int64_t)b * a.src_sb + tt.start;
+    lk.init_gather(a.k + (int64_t)b * a.T * a.D, a.D, a.D, [&](int r) __attribute__((always_inline)) {
+      // an index outside [0, T) reads row T - 1
+      return (int)min((uint32_t)src[min(tt.n0 + r, tt.size - 1)], (uint32_t)(a.T - 1));
+    });
+  } else {
+    lk.init(Operand{a.k + row * a.D, a.D, tt.size, a.D}, tt.n0);
+  }
 
   const int nk = (a.D + kTK - 1) / kTK;
   uint8_t *p0 = ring, *p1 = ring + kSlot, *p2 = ring + 2 * kSlot;
@@ -472,16 +512,22 @@ __device__ __forceinline__ void narrow_body(const NarrowArgs& a, const typename 
   dh_stage(dh, p0, w, ar, ak, [&]() __attribute__((always_inline)) { __VA_ARGS__; }), rotate()
 #define UTTT_Y_STAGE(...) \
   y_stage(y, p0, w, ak, [&]() __attribute__((always_inline)) { __VA_ARGS__; }), rotate()
-  issue_stage(l1, lv, 0, p0);
-  issue_stage(l1, lv, 1, p1);  // D > kTK: at least two stages of each product
-  for (int s = 0; s < nk - 2; ++s) {
+  // D > kTK: at least two stages of each product
+  if constexpr (Epi::kThree) {
+    issue_stage(l1, lv, 0, p0);
+    issue_stage(l1, lv, 1, p1);
+    for (int s = 0; s < nk - 2; ++s) {
+      wait_vmcnt<3>();
+      UTTT_DH_STAGE(issue_stage(l1, lv, s + 2, p2));
+    }
     wait_vmcnt<3>();
-    UTTT_DH_STAGE(issue_stage(l1, lv, s + 2, p2));
+    UTTT_DH_STAGE(issue_stage(l02, lk, 0, p2));
+    wait_vmcnt<4>();
+    UTTT_DH_STAGE(issue_stage(l02, lk, 1, p2));
+  } else {
+    issue_stage(l02, lk, 0, p0);
+    issue_stage(l02, lk, 1, p1);
   }
-  wait_vmcnt<3>();
-  UTTT_DH_STAGE(issue_stage(l02, lk, 0, p2));
-  wait_vmcnt<4>();
-  UTTT_DH_STAGE(issue_stage(l02, lk, 1, p2));
   for (int s = 0; s < nk - 2; ++s) {
     wait_vmcnt<4>();
     UTTT_Y_STAGE(issue_stage(l02, lk, s + 2, p2));
@@ -513,7 +559,7 @@ int narrow_args(NarrowArgs* a, const void* w0_w2, const void* w1, const void* k,
                 const char* what) {
   *a = NarrowArgs{static_cast<const uint16_t*>(w0_w2), static_cast<const uint16_t*>(w1),
                   static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), gs, B, E, I, D,
-                  N, narrow_m_tiles(I), (N + kTok - 1) / kTok + E};
+                  N, narrow_m_tiles(I), (N + kTok - 1) / kTok + E, nullptr, 0, 0};
   const int64_t units = ((int64_t)B * a->n_tiles_ub + kXcds - 1) / kXcds * kXcds;
   *blocks = units * a->m_tiles;
   UTTT_REQUIRE(*blocks <= 0x7fffffffLL, "%s: problem too large for one launch", what);
@@ -543,6 +589,21 @@ int launch_narrow_stage1(const void* w0_w2, const void* w1, const void* k, const
     hipLaunchKernelGGL((narrow_kernel<NarrowS1<LR>>), dim3((unsigned)blocks), dim3(kTThreads), 0,
                        st, a, ea);
   });
+  return check_launch(what);
+}
+
+int launch_narrow_gate_up(const void* w0_w2, const void* x, const int32_t* src_rows,
+                          long long src_sb, const int32_t* gs, int B, int E, int I, int D, int N,
+                          int T, void* hidden, hipStream_t st, const char* what) {
+  NarrowArgs a;
+  int64_t blocks;
+  if (int rc = narrow_args(&a, w0_w2, nullptr, x, nullptr, gs, B, E, I, D, N, &blocks, what))
+    return rc;
+  a.src = src_rows;
+  a.src_sb = src_sb;
+  a.T = T;
+  hipLaunchKernelGGL((narrow_kernel<NarrowSwiGLU>), dim3((unsigned)blocks), dim3(kTThreads), 0, st,
+                     a, NarrowSwiGLU::Args{static_cast<uint16_t*>(hidden)});
   return check_launch(what);
 }
 

@@ -97,6 +97,27 @@ struct Loader {
     }
   }
 
+  // A KMajor tile of gathered rows: row(r) of org for tile row r (below 2^30
+  // elements in).
+  template <class Row>
+  __device__ __forceinline__ void init_gather(const uint16_t* org, int ld, int k_end_, Row&& row) {
+    const int lane = threadIdx.x & 63;
+    const int w = wave_id();
+    k_end = k_end_;
+    last = (k_end + kTK - 1) / kTK - 1;
+    wofs = w * 1024;
+    asm volatile("" : "+s"(wofs));
+    base = uniform_ptr(reinterpret_cast<const uint8_t*>(org));
+    kstep = (int64_t)kTK * 2;
+#pragma unroll
+    for (int t = 0; t < kLoads; ++t) {
+      const int s = (t * 4 + w) * 64 + lane;
+      const int r = s >> 2;
+      off[t] = (uint32_t)(row(r) * ld + ((s & 3) ^ ((r >> 2) & 3)) * 8) * 2u;
+      asm volatile("" : "+v"(off[t]));
+    }
+  }
+
   // Step `step` (0 .. last, in order) into the tile at LDS `dst`.
   __device__ __forceinline__ void issue(int step, uint8_t* dst) {
     const uint8_t* sb = uniform_ptr(base + (int64_t)step * kstep);
@@ -215,10 +236,14 @@ __device__ __forceinline__ void mma9(Acc& acc, const Frags& f) {
 // products run in increasing k in 16-wide steps with A in the first operand,
 // as in gemm_pipe.h, so the results are the 256-tile kernels' bits.
 // SCALE_B: the second operand is bf16(b_scale * B), converted as its
-// fragments are read.
-template <int AMAJ, int BMAJ, bool SCALE_B = false>
+// fragments are read.  at(k), run before stage k is issued, gives the loaders'
+// step of it (a chained second pair points them at its operands there).
+struct SameStep {
+  __device__ int operator()(int k) const { return k; }
+};
+template <int AMAJ, int BMAJ, bool SCALE_B = false, class At = SameStep>
 __device__ __forceinline__ void k_loop(Loader<AMAJ>& la, Loader<BMAJ>& lb, int nk, uint8_t* ring,
-                                       Acc& acc, float b_scale = 1.0f) {
+                                       Acc& acc, float b_scale = 1.0f, At&& at = At()) {
   const int w = wave_id();
   FragAddr<AMAJ> fa;
   FragAddr<BMAJ> fb;
@@ -226,12 +251,13 @@ __device__ __forceinline__ void k_loop(Loader<AMAJ>& la, Loader<BMAJ>& lb, int n
   fb.init(w & 1);
   constexpr int kOps = kNBlk * (AMAJ == KMajor ? 1 : 2) + kNBlk * (BMAJ == KMajor ? 1 : 2);
   uint8_t *p0 = ring, *p1 = ring + kTStage, *p2 = ring + 2 * kTStage;
-  la.issue(0, p0);
-  lb.issue(0, p0 + kTTile);
-  if (nk > 1) {
-    la.issue(1, p1);
-    lb.issue(1, p1 + kTTile);
-  }
+  auto issue = [&](int k, uint8_t* slot) __attribute__((always_inline)) {
+    const int step = at(k);
+    la.issue(step, slot);
+    lb.issue(step, slot + kTTile);
+  };
+  issue(0, p0);
+  if (nk > 1) issue(1, p1);
   Frags f[2];
   for (int k = 0; k < nk; ++k) {
     if (k + 1 < nk)
@@ -247,10 +273,7 @@ __device__ __forceinline__ void k_loop(Loader<AMAJ>& la, Loader<BMAJ>& lb, int n
         f[KS].b[I] = fb.template read<decltype(KS)::value, decltype(I)::value>(tb);
       });
     });
-    if (k + 2 < nk) {
-      la.issue(k + 2, p2);
-      lb.issue(k + 2, p2 + kTTile);
-    }
+    if (k + 2 < nk) issue(k + 2, p2);
     __builtin_amdgcn_sched_barrier(0);
     wait_frags<kOps>(f[0]);
     if constexpr (SCALE_B)

@@ -193,6 +193,62 @@ __global__ __launch_bounds__(256) void wg192_reduce_kernel(Wg192Args a) {
   }
 }
 
+// ================================================= token-grouped products ==
+// y[b, n, m] = sum_k A(m, k) x[b, n, k] (+ a second pair chained along k) over
+// the tokens n of each expert, A [M, K] (KMajor) or [K, M] (RMajor) per expert;
+// bf16, the 256-token kernels' bits.  For narrow experts the token rows' stream
+// bounds it: 48 of 192 x 192 over 196 608 tokens 377 MB in 88 us (grad_K), 226
+// in 55 (grad_V).  Super-tiles as in tn_kernel, 64 workgroups to an XCD at once.
+struct Tn192Args {
+  const uint16_t* a[2];
+  const uint16_t* x[2];
+  int K[2];  // K[1] = 0: one product
+  uint16_t* y;
+  const int32_t* gs;
+  int B, E, N, M, m_tiles, n_tiles_ub;
+  int gm, gn, n_super_m;  // super-tiles: gm m-tiles x gn token tiles on one XCD
+};
+
+template <int AMAJ>
+__global__ __launch_bounds__(kTThreads, 2) void tn192_kernel(Tn192Args s) {
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kTRing * kTStage];
+  const int loc = blockIdx.x / kXcds, per = s.gm * s.gn;
+  const int sup = loc / per * kXcds + blockIdx.x % kXcds, p = loc % per;
+  const int mt = sup % s.n_super_m * s.gm + p % s.gm;
+  const int unit = sup / s.n_super_m * s.gn + p / s.gm;
+  if (mt >= s.m_tiles || unit >= s.B * s.n_tiles_ub) return;
+  const int b = unit / s.n_tiles_ub;
+  const TokenTile tt =
+      find_token_tile<kT>(s.gs + (int64_t)b * s.E, s.E, s.N, unit - b * s.n_tiles_ub);
+  if (tt.e < 0) return;
+  const int m0 = mt * kT;
+  const int64_t ge = (int64_t)b * s.E + tt.e, row = (int64_t)b * s.N + tt.start;
+  Loader<AMAJ> la;
+  Loader<KMajor> lx;
+  auto pair = [&](int i) __attribute__((always_inline)) {
+    const int K = s.K[i];
+    la.init(Operand{s.a[i] + ge * s.M * K, AMAJ == KMajor ? K : s.M, s.M, K}, m0);
+    lx.init(Operand{s.x[i] + row * K, K, tt.size, K}, tt.n0);
+  };
+  pair(0);
+  const int nk0 = (s.K[0] + kTK - 1) / kTK, nk1 = (s.K[1] + kTK - 1) / kTK;
+  Acc acc;
+  zero_acc(acc);
+  k_loop<AMAJ, KMajor>(la, lx, nk0 + nk1, ring, acc, 1.0f,
+                       [&](int k) __attribute__((always_inline)) {
+                         if (k == nk0) pair(1);
+                         return k < nk0 ? k : k - nk0;
+                       });
+  const int me = after_loop(m0), left = after_loop(tt.size) - after_loop(tt.n0);
+  uint16_t* y = uniform_ptr(s.y + ((int64_t)after_loop(b) * s.N + after_loop(tt.start) +
+                                   after_loop(tt.n0)) * s.M + me);
+  staged(
+      acc, reinterpret_cast<float*>(ring), [](auto, auto, int, int) {},
+      [&](auto, auto, int n, int g, float (&v)[8]) __attribute__((always_inline)) {
+        if (n < left && me + 8 * g < s.M) store8_bf16(y + (uint32_t)(n * s.M + 8 * g), v);
+      });
+}
+
 // ========================================================= Newton-Schulz ==
 // The three products of a step over BE matrices, with the rounding of the
 // reference's bf16 tensor arithmetic (grouped_gemm.hip's EpiLinComb):
@@ -338,6 +394,39 @@ int launch_wg192(const Wg192Plan& pl, const void* dy, const void* k, const void*
   if (pl.parts_ub == 0) return UTTT_OK;  // no expert has a second chunk
   const unsigned blocks = (unsigned)std::min<int64_t>((pl.n_out / 8 + 255) / 256, 64);
   hipLaunchKernelGGL(wg192_reduce_kernel, dim3(blocks, (unsigned)(B * E)), dim3(256), 0, st, a);
+  return check_launch(what);
+}
+
+int launch_tn192(bool a_kmajor, const void* a0, const void* x0, int K0, const void* a1,
+                 const void* x1, int K1, int M, void* y, int B, int E, int N, const int32_t* gs,
+                 hipStream_t st, const char* what) {
+  Tn192Args s{};
+  s.a[0] = static_cast<const uint16_t*>(a0);
+  s.x[0] = static_cast<const uint16_t*>(x0);
+  s.a[1] = static_cast<const uint16_t*>(K1 > 0 ? a1 : a0);
+  s.x[1] = static_cast<const uint16_t*>(K1 > 0 ? x1 : x0);
+  s.K[0] = K0;
+  s.K[1] = K1;
+  s.y = static_cast<uint16_t*>(y);
+  s.gs = gs;
+  s.B = B;
+  s.E = E;
+  s.N = N;
+  s.M = M;
+  s.m_tiles = tiles_of(M);
+  s.n_tiles_ub = tiles_of(N) + E;
+  const int64_t units = (int64_t)B * s.n_tiles_ub;
+  s.gm = std::min(s.m_tiles, 8);
+  s.gn = units * s.m_tiles >= 8 * 512 ? 64 / s.gm : 1;
+  s.n_super_m = (s.m_tiles + s.gm - 1) / s.gm;
+  const int64_t supers = s.n_super_m * ((units + s.gn - 1) / s.gn);
+  const int64_t blocks = (supers + kXcds - 1) / kXcds * kXcds * s.gm * s.gn;
+  UTTT_REQUIRE(blocks <= 0x7fffffffLL && K0 < (1 << 23) && K1 < (1 << 23) && M < (1 << 23),
+               "%s: problem too large for one launch", what);
+  if (a_kmajor)
+    hipLaunchKernelGGL((tn192_kernel<KMajor>), dim3((unsigned)blocks), dim3(kTThreads), 0, st, s);
+  else
+    hipLaunchKernelGGL((tn192_kernel<RMajor>), dim3((unsigned)blocks), dim3(kTThreads), 0, st, s);
   return check_launch(what);
 }
 

@@ -39,6 +39,12 @@ int launch_wg192(const Wg192Plan& plan, const void* dy, const void* k, const voi
                  const void* v, void* dw0_w2, void* dw1, const int32_t* gs, int B, int E, int I,
                  int D, int N, void* workspace, hipStream_t st, const char* what);
 
+// Token-grouped products y[b, n, m] = sum_k A(m, k) x[b, n, k], a second pair
+// chained along k when K1 > 0.  Widths multiples of 8, pointers 16-byte aligned.
+int launch_tn192(bool a_kmajor, const void* a0, const void* x0, int K0, const void* a1,
+                 const void* x1, int K1, int M, void* y, int B, int E, int N, const int32_t* gs,
+                 hipStream_t st, const char* what);
+
 // One Newton-Schulz step of BE matrices x [m, n] (m <= n): a [m, m] = x x^T,
 // b [m, m] = cb a + (cc a) a, xn [m, n] = ca x + b x; `last`: xn times
 // out_scale, as [n, m] with `trans`.
