@@ -232,7 +232,7 @@ def is_available() -> bool:
 
 
 def call(name: str, *args) -> None:
-    rc = getattr(lib(), name)(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if rc != 0:
         msg = lib().uttt_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed ({rc}): {msg}")

@@ -12,6 +12,7 @@ from __future__ import annotations
 import functools
 
 import torch
+from torch.autograd import forward_ad
 
 
 def traced_op(name, fake, mutates_args=()):
@@ -29,6 +30,31 @@ def traced_op(name, fake, mutates_args=()):
         return call
 
     return deco
+
+
+class _NoGraph:
+    """The ctx of a forward whose graph nobody keeps."""
+
+    def save_for_backward(self, *tensors):
+        pass
+
+    def mark_non_differentiable(self, *tensors):
+        pass
+
+
+def run_function(fn, *args):
+    """fn.apply(*args) of a torch.autograd.Function, or its forward alone where
+    nothing could see the difference: gradients are off and neither
+    torch.compile, jit tracing, a functorch transform nor a forward-mode level
+    is active (under which apply records, refuses or transforms the call).
+    apply costs 5 to 8 us of host time per call; a routed read without
+    gradients, three of them, is paced by its host time (88 us against 61 on
+    the GPU for 16 384 tokens of 192 over 48 experts)."""
+    if (torch.is_grad_enabled() or torch.compiler.is_compiling()
+            or torch._C._are_functorch_transforms_active()
+            or torch._C._get_tracing_state() is not None or forward_ad._current_level >= 0):
+        return fn.apply(*args)
+    return fn.forward(_NoGraph(), *args)
 
 
 def none_if_empty(t):

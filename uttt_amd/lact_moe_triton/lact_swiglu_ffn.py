@@ -13,6 +13,8 @@ from __future__ import annotations
 import torch
 from torch.autograd.function import once_differentiable
 
+from uttt_amd._ops import run_function  # absolute: the package also works mounted in the reference tree
+
 from . import _grouped
 
 
@@ -47,4 +49,4 @@ class FusedSwiGLUFFNFwd(torch.autograd.Function):
 
 def grouped_swiglu_ffn_fwd(W0_W2, W1, X, group_sizes):
     """F:107-108: the APPLY op of uttt_moe (modeling_recurrent_lact.py:329-334)."""
-    return FusedSwiGLUFFNFwd.apply(W0_W2, W1, X, group_sizes)
+    return run_function(FusedSwiGLUFFNFwd, W0_W2, W1, X, group_sizes)

@@ -16,7 +16,7 @@ import torch
 from torch import Tensor
 
 from uttt_amd import _lib as L  # absolute: the package also works mounted in the reference tree
-from uttt_amd._ops import none_if_empty, traced_op
+from uttt_amd._ops import none_if_empty, run_function, traced_op
 
 
 def _mask_arg(routing_map: torch.Tensor):
@@ -338,7 +338,7 @@ def permute_with_expert_mask(
     row_id_map: torch.Tensor = None,
 ):
     """(out [B, topk*T, H], permuted_probs [B, topk*T] or None, row_id_map) (P:1241-1248)."""
-    return PermuteWithMaskMap.apply(inp, expert_mask, probs, topk, row_id_map)
+    return run_function(PermuteWithMaskMap, inp, expert_mask, probs, topk, row_id_map)
 
 
 class UnPermuteWithMaskMap(torch.autograd.Function):
@@ -378,7 +378,7 @@ class UnPermuteWithMaskMap(torch.autograd.Function):
 
 def unpermute_and_merge_with_probs(permuted_x, row_id_map, original_probs):
     """[B, T, H] merge of the permuted rows with the router probs (P:1316-1325)."""
-    return UnPermuteWithMaskMap.apply(permuted_x, row_id_map, original_probs)
+    return run_function(UnPermuteWithMaskMap, permuted_x, row_id_map, original_probs)
 
 
 class PermuteKVAndLRs(torch.autograd.Function):

@@ -36,6 +36,7 @@ from typing import Sequence
 import torch
 
 from . import _lib as L
+from ._ops import run_function
 from .lact_moe_triton import _grouped
 from .lact_moe_triton.lact_fw_grad import grouped_lact_swiglu_ffn_fast_weight_grads
 from .lact_moe_triton.lact_swiglu_ffn import grouped_swiglu_ffn_fwd
@@ -244,7 +245,7 @@ def rows_preprocess(x: torch.Tensor, *, silu: bool = False, norm: str | None = N
     silu's backward on one kernel, rounded where the reference's autograd
     rounds.  Returns a new tensor (bf16 with rope, else x's dtype)."""
     assert norm in _NORMS, f"norm must be None, 'l2' or 'rms', got {norm!r}"
-    return _RowsPreprocess.apply(x, bool(silu), norm, rows_of, rope)
+    return run_function(_RowsPreprocess, x, bool(silu), norm, rows_of, rope)
 
 
 def _norm_name(flag: bool, kind: str):
