@@ -28,6 +28,7 @@ CASES = {
     "slack_rows": ([[60, 40]], 384, 384, 160),
     "over_count": ([[60, 90, 70]], 96, 200, 140),
     "all_empty": ([[0, 0, 0]], 192, 64, 32),
+    "short_segments_wide": ([[200, 0, 193, 1, 300, 192]], 520, 776, None),
 }
 
 

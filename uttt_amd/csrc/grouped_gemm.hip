@@ -1977,7 +1977,7 @@ extern "C" int uttt_grouped_update_stage1(const void* w0_w2, const void* w1, con
   UTTT_REQUIRE(workspace_bytes >= need, "grouped_update_stage1: workspace %zu < %zu bytes",
                workspace_bytes, need);
   hipStream_t st = as_stream(stream);
-  if (token_major && narrow_experts(I, D) && !general_forced())
+  if (token_major && narrow_stage1(I, D, N, E) && !general_forced())
     return launch_narrow_stage1(w0_w2, w1, k, v, lr0, lr1, lr2, lr_dtype, group_sizes, B, E, I, D, N,
                                 dy0_dy2, hidden, y0_y2_save, dh_save, st,
                                 "grouped_update_stage1");

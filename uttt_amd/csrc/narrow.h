@@ -7,6 +7,11 @@ namespace uttt {
 
 // Expert widths that narrow.hip's kernels take (any token counts).
 bool narrow_experts(int I, int D);
+// Sizes whose stage 1 it takes: also experts up to 768 x 1536 with at most 256
+// tokens on average, where half of the 256-token tiles is padding and the fp32
+// DH a round trip (16 over 3062 tokens: DH 34 + 64 us, here 69).  Their
+// backward gains nothing (GD 24 + 67 us, here 93 and twice the lr partials).
+bool narrow_stage1(int I, int D, int N, int E);
 // Row blocks of its lr-gradient partials, lr_part[3][narrow_m_tiles][B][N].
 int narrow_m_tiles(int I);
 

@@ -21,7 +21,7 @@
 // 96 of 384 x 384 over 16 384 tokens, without saves: 89 -> 45 us; gate/up 42 ->
 // 31, of 48 x 192 x 192 17 -> 10.7 (against apply_kernel's 256 x 128 tiles).
 // Past 512 the products outweigh the rows and a token tile is read by more
-// than eight unit groups: the 256-token tiles' kernels.
+// than eight unit groups: the 256-token tiles' kernels (but see narrow_stage1).
 #include "narrow.h"
 #include "tile192.h"
 
@@ -570,6 +570,10 @@ int narrow_args(NarrowArgs* a, const void* w0_w2, const void* w1, const void* k,
 
 // ------------------------------------------------------------------ host ----
 bool narrow_experts(int I, int D) { return I <= 512 && D <= 512 && D > kTK; }
+bool narrow_stage1(int I, int D, int N, int E) {
+  return narrow_experts(I, D) ||
+         (D > kTK && N <= 256 * (int64_t)E && (int64_t)I * D <= (int64_t)768 * 1536);
+}
 int narrow_m_tiles(int I) { return (I + kHid - 1) / kHid; }
 
 int launch_narrow_stage1(const void* w0_w2, const void* w1, const void* k, const void* v,
