@@ -1749,13 +1749,12 @@ using namespace uttt;
 
 extern "C" size_t uttt_row_id_map_workspace_bytes(int B, int T, int E) {
   if (B <= 0 || T <= 0 || E <= 0) return 0;
-  // 64-token tiles: the counts and the offsets (or the offsets of a router's
-  // 32-token counts); 256-token tiles for E <= kScanEmitMaxE
-  const size_t general = (size_t)2 * B * E * ((T + kTile64 - 1) / kTile64);
-  const size_t two = E <= kScanEmitMaxE
-                         ? (size_t)B * padded_experts(E) * ((T + kTile - 1) / kTile)
-                         : 0;
-  return (general > two ? general : two) * sizeof(int32_t);
+  // E <= kScanEmitMaxE: the 256-token tiles' counts; above, the 64-token
+  // tiles' counts and their offsets
+  const size_t entries = E <= kScanEmitMaxE
+                             ? (size_t)B * padded_experts(E) * ((T + kTile - 1) / kTile)
+                             : (size_t)2 * B * E * ((T + kTile64 - 1) / kTile64);
+  return entries * sizeof(int32_t);
 }
 
 extern "C" int uttt_make_row_id_map(const void* routing_map, int mask_bytes, int64_t s_b,

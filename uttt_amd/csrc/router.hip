@@ -1339,10 +1339,16 @@ extern "C" int uttt_route_tokens(const void* x, int x_dtype, const float* router
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// The map's own workspace behind the router's: the offsets of its blocks'
+// counts, 32 tokens per block at the least.
+static size_t map_offsets_bytes(int B, int T, int E) {
+  return (size_t)B * E * ((T + 31) / 32) * sizeof(int32_t);
+}
+
 extern "C" size_t uttt_route_tokens_map_workspace_bytes(int B, int T, int E, int D) {
   if (B <= 0 || T <= 0 || E <= 0) return 0;
   return align256(uttt_router_workspace_bytes(B, T, E, D)) +
-         uttt_row_id_map_workspace_bytes(B, T, E);
+         map_offsets_bytes(B, T, E);
 }
 
 extern "C" int uttt_route_tokens_map_src_rows(int T, int E) {
@@ -1370,7 +1376,7 @@ extern "C" int uttt_route_tokens_map(const void* x, int x_dtype, const float* ro
   const int blk_tokens = route_block_tokens(x, x_dtype, router_w, w_sb, B, T, D);
   Ws w = ws_layout(workspace, B, T, E, blk_tokens);
   const size_t rm_off = align256(w.bytes);
-  const size_t need = rm_off + uttt_row_id_map_workspace_bytes(B, T, E);
+  const size_t need = rm_off + map_offsets_bytes(B, T, E);
   UTTT_REQUIRE(workspace != nullptr && workspace_bytes >= need,
                "route_tokens_map: workspace %zu < %zu bytes", workspace_bytes, need);
   w.bal_sum = balance_sum;
