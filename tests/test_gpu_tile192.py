@@ -63,6 +63,7 @@ def test_chunked_weight_gradients(name):
     (2, 776, 392, torch.float32, 0), (3, 8, 1000, torch.bfloat16, 0),
     (1, 584, 584, torch.float32, 0), (2, 208, 416, torch.float32, 1),
     (2, 416, 208, torch.bfloat16, 1),
+    (1, 1544, 1608, torch.float32, 0),   # a second band of tiles, one matrix on every XCD
 ])
 def test_newton_schulz5_tiles(n, R, C, dtype, offset):
     """Against the same iteration in fp64: overall no further off than 1.5x the
@@ -92,3 +93,14 @@ def test_newton_schulz5_tiles(n, R, C, dtype, offset):
         if exact.shape[dim] >= 200:
             rms = exact.norm(dim=dim).pow(2).mean().sqrt()
             assert ((ours - exact).norm(dim=dim).max() / rms).item() <= 5e-2
+
+
+@pytest.mark.parametrize("n,R,C", [(9, 392, 584), (3, 1544, 1608)])
+def test_newton_schulz5_alone_or_stacked(n, R, C):
+    """A matrix's result does not depend on the matrices beside it: the tiles of
+    all are cut into one run per XCD, of which one alone fills parts (several
+    tiles per side; past eight a second band)."""
+    G = torch.randn(n, R, C, generator=torch.Generator().manual_seed(n)).to(DEV)
+    all_ = FWW.newton_schulz5(G)
+    for i in range(n):
+        assert torch.equal(FWW.newton_schulz5(G[i:i + 1].contiguous())[0], all_[i])

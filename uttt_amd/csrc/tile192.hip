@@ -31,6 +31,16 @@ __device__ __forceinline__ void unpack8_bf16(const uint4& u, float (&v)[8]) {
   }
 }
 
+// This workgroup's place among n when every XCD takes a contiguous eighth of
+// them (grid xcd_run_blocks(n)), or -1: neighbours share an XCD's L2, and few
+// large groups still reach every XCD.
+__device__ __forceinline__ int xcd_run(int n) {
+  const int each = (n + kXcds - 1) / kXcds;
+  const int i = blockIdx.x % kXcds * each + blockIdx.x / kXcds;
+  return i < n ? i : -1;
+}
+int64_t xcd_run_blocks(int64_t n) { return (n + kXcds - 1) / kXcds * kXcds; }
+
 // ======================================================= weight gradients ==
 // out[b, e][x][y] = sum_{n in seg(b, e)} P[n, y] Q[n, x] (two tasks per
 // launch), the segment of every expert cut into chunks of `chunk` tokens: one
@@ -263,7 +273,13 @@ __global__ __launch_bounds__(kTThreads, 2) void tn192_kernel(Tn192Args s) {
 // 288 matrices of 384 x 384 read and write 85 MB per operand and product,
 // which is what bounds them; 256 x 256 tiles (half padding there) took 180 / 134
 // / 136 us per product.
+// Every XCD takes a contiguous eighth of the tiles of all matrices: with a
+// matrix per XCD, few matrices left XCDs idle (one of 4096 x 4096 12.1 ms, now
+// 2.0; nine of 1536 x 3072 2.45 -> 1.82; the 256 x 256 tiles took 2.2 and 2.3).
+// Within a matrix the tiles run in bands of kNsBand rows, so that the 64 on an
+// XCD at once share eight rows' and eight columns' operands in its L2.
 enum NsProduct { kNsA = 0, kNsB = 1, kNsX = 2 };
+constexpr int kNsBand = 8;
 
 struct Ns192Args {
   const uint16_t* a;   // per matrix: [M, K] rows, or [K, M] (kNsX)
@@ -279,17 +295,20 @@ template <int P>
 __global__ __launch_bounds__(kTThreads, 2) void ns192_kernel(Ns192Args s) {
   constexpr int kAMaj = P == kNsX ? RMajor : KMajor;
   __shared__ __attribute__((aligned(16))) uint8_t ring[kTRing * kTStage];
-  // the tiles of one matrix run on one XCD and share its L2
   const int per = P == kNsA ? s.m_tiles * (s.m_tiles + 1) / 2 : s.m_tiles * s.r_tiles;
-  const int loc = blockIdx.x / kXcds;
-  const int mat = loc / per * kXcds + blockIdx.x % kXcds;
-  if (mat >= s.BE) return;
-  const int t = loc % per;
-  int mt = t % s.m_tiles, rt = t / s.m_tiles;
+  const int unit = xcd_run(s.BE * per);
+  if (unit < 0) return;
+  const int mat = unit / per, t = unit % per;
+  int mt, rt;
   if constexpr (P == kNsA) {  // tile t of the lower triangle, row rt holding rt + 1
     rt = 0;
     mt = t;
     while (mt > rt) mt -= ++rt;
+  } else {  // bands of kNsBand rows of tiles, column by column
+    const int band = t / (kNsBand * s.m_tiles) * kNsBand, p = t - band * s.m_tiles;
+    const int rows = min(kNsBand, s.r_tiles - band);
+    rt = band + p % rows;
+    mt = p / rows;
   }
   const int m0 = mt * kT, r0 = rt * kT;
   const int64_t om = (int64_t)mat * s.R * s.M;
@@ -435,7 +454,7 @@ template <int P>
 int launch_ns(const Ns192Args& s, hipStream_t st, const char* what) {
   const int64_t per = P == kNsA ? (int64_t)s.m_tiles * (s.m_tiles + 1) / 2
                                 : (int64_t)s.m_tiles * s.r_tiles;
-  const int64_t blocks = (int64_t)(s.BE + kXcds - 1) / kXcds * kXcds * per;
+  const int64_t blocks = xcd_run_blocks(s.BE * per);
   UTTT_REQUIRE(blocks <= 0x7fffffffLL, "%s: problem too large for one launch", what);
   hipLaunchKernelGGL((ns192_kernel<P>), dim3((unsigned)blocks), dim3(kTThreads), 0, st, s);
   return check_launch(what);
