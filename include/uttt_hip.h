@@ -313,9 +313,12 @@ int uttt_grouped_wgrad_pair(const void* dy0_dy2_tok, const void* k, const void* 
                             const void* v, const int32_t* group_sizes, int B, int E, int I,
                             int D, int N, void* dw0_w2, void* dw1, void* workspace,
                             size_t workspace_bytes, void* stream);
-/* Workspace of uttt_grouped_wgrad_pair: fp32 split-K partials when the
- * output tiles fill under half of the GPU (a single expert with small
- * weights, as uTTT-Dense), else 0 (workspace may then be NULL). */
+/* Workspace of uttt_grouped_wgrad_pair: fp32 partials of token segments cut
+ * into pieces, for small experts and short segments, else 0.  With several
+ * experts less than this, or NULL, is accepted too: every segment is then
+ * summed whole (slower, no partials).  Required only when the output tiles
+ * fill under half of the GPU (a single expert with small weights, as
+ * uTTT-Dense). */
 size_t uttt_grouped_wgrad_pair_workspace_bytes(int B, int E, int I, int D, int N);
 
 /* One weight-gradient product.  Replaces grouped_gemm_bwd_triton

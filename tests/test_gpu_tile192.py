@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from oracle import write as OW
+from uttt_amd import _lib as L
 from uttt_amd import fast_weight_write as FWW
 from uttt_amd.lact_moe_triton import _grouped as G
 
@@ -53,6 +54,34 @@ def test_chunked_weight_gradients(name):
                 ref = p64.T @ q64
                 bound = 2.0 ** -8 * ref.abs() + n * 2.0 ** -24 * (p64.abs().T @ q64.abs())
                 assert bool(((ours.double() - ref).abs() <= bound).all()), (b, e, n)
+
+
+@pytest.mark.parametrize("given", ["none", "short", "unaligned"])
+def test_weight_gradients_without_room_for_partials(given):
+    """48 experts of 192 x 192 with segments of several chunks: the workspace is
+    optional, and without it every segment is summed whole."""
+    B, E, D, I, N = 1, 48, 192, 192, 48 * 700
+    g = torch.Generator().manual_seed(1)
+    sizes = torch.randint(0, 1400, (B, E), generator=g, dtype=torch.int32)
+    gs = sizes.to(DEV)
+    dy, k, hid, v = (torch.randn(B, N, w, generator=g).to(torch.bfloat16).to(DEV)
+                     for w in (2 * I, D, I, D))
+    need = L.lib().uttt_grouped_wgrad_pair_workspace_bytes(B, E, I, D, N)
+    assert need > 0
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=DEV)
+    ptr, size = {"none": (None, 0), "short": (L.ptr(ws), need - 1),
+                 "unaligned": (L.ptr(ws) + 4, need)}[given]
+    dw02 = torch.empty(B, E, 2 * I, D, dtype=torch.bfloat16, device=DEV)
+    dw1 = torch.empty(B, E, D, I, dtype=torch.bfloat16, device=DEV)
+    L.call("uttt_grouped_wgrad_pair", L.ptr(dy), L.ptr(k), L.ptr(hid), L.ptr(v), L.ptr(gs), B, E,
+           I, D, N, L.ptr(dw02), L.ptr(dw1), ptr, size, L.stream_of(k))
+    ref = G.wgrad_pair(dy, k, hid, v, gs)
+    # one bf16 rounding each, and the fp32 sums in two orders of n products of
+    # mean magnitude 2 / pi: twice n 2^-24 times n of them
+    n = int(sizes.max())
+    for a, b in zip((dw02, dw1), ref):
+        a, b = a.double(), b.double()
+        assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + n * n * 2.0 ** -23).all())
 
 
 # (matrices, rows, columns, dtype, offset in elements): partial tiles on both

@@ -2032,13 +2032,11 @@ extern "C" int uttt_grouped_wgrad_pair(const void* dy0_dy2_tok, const void* k,
                "grouped_wgrad_pair: tensors must be 16-byte aligned");
   // dW0_W2 [2I][D] = DY^T K;  dW1 [D][I] = V^T Hid
   const Wg192Plan pl = wg192_plan(B, E, I, D, N);
-  if (pl.use) {
-    UTTT_REQUIRE(pl.bytes == 0 || (workspace && workspace_bytes >= pl.bytes && aligned16(workspace)),
-                 "grouped_wgrad_pair: workspace of %zu bytes needed (got %zu)", pl.bytes,
-                 workspace_bytes);
+  // without room for its partials: the 256-tile kernel, a segment per workgroup
+  if (pl.use &&
+      (pl.bytes == 0 || (workspace && workspace_bytes >= pl.bytes && aligned16(workspace))))
     return launch_wg192(pl, dy0_dy2_tok, k, hidden_tok, v, dw0_w2, dw1, group_sizes, B, E, I, D, N,
                         workspace, as_stream(stream), "grouped_wgrad_pair");
-  }
   const WgTask t0 = wg_task(k, dy0_dy2_tok, dw0_w2, 2 * I, D);
   const WgTask t1 = wg_task(hidden_tok, v, dw1, D, I);
   return launch_wg(t0, t1, group_sizes, B, E, N, wg_splits(t0, t1, B, E, N), workspace,
