@@ -428,8 +428,12 @@ int uttt_rows_preprocess_bwd(const void* in, int dtype, const void* grad_out, in
 /* Test hook (no reference counterpart): grids of the token-grouped GEMMs
  * with at least `min_tiles` workgroup tiles take the XCD super-tile order
  * (default 2048, one value per process; a negative value restores it).
- * Returns the previous value.  Results do not depend on it: tests lower it
- * to run small problems down the path the large ones take. */
+ * Any other value also takes every grouped product on the general 256x256
+ * tiles where the sizes would choose the 192-tile or narrow-expert kernels.
+ * Returns the previous value.  The tile order changes no result; against the
+ * other kernels the products agree bit for bit, the weight gradients and the
+ * UPDATE backward to the order of their fp32 sums.  Tests lower it to run
+ * small problems down the path the large ones take. */
 long long uttt_debug_set_supertile_min_tiles(long long min_tiles);
 
 /* Test hook: which kernel runs the weight-streaming APPLY products
@@ -447,7 +451,9 @@ int uttt_debug_set_apply_path(int path);
  * 1: eight waves (two per SIMD, 64x128 per wave; families whose eight-wave
  * kernel does not fit the register file keep four).  Both layouts
  * accumulate every output in the same k order with the same MFMA, so
- * results are identical.  Returns the previous value. */
+ * their results are identical.  A forced layout takes every grouped product
+ * on the 256x256 tiles, as uttt_debug_set_supertile_min_tiles does.  Returns
+ * the previous value. */
 int uttt_debug_set_gemm_layout(int na);
 
 /* Test hook (no reference counterpart): which path uttt_newton_schulz5 takes.

@@ -54,6 +54,16 @@ def test_wgrad_pair_split_rule():
     assert q(4, 1, 192, 96, 512) == 0            # 8 K steps per segment: one run
     assert q(1, 1, 64, 64, 64 * 8 * 40) == 32 * 3 * 64 * 64 * 4  # capped at 32 runs
     assert q(0, 1, I, D, 24576) == 0
+    # small experts: pieces of their segments, but not where the tests force
+    # the general tiles
+    hook = _lib.lib().uttt_debug_set_gemm_layout
+    assert q(1, 48, 192, 192, 196608) > 0
+    prev = hook(2)
+    try:
+        assert q(1, 48, 192, 192, 196608) == 0
+        assert q(2, 2, 64, 64, 4000) == 4 * 4 * 3 * 64 * 64 * 4  # four runs of 8 K steps
+    finally:
+        hook(prev)
 
 
 @pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")

@@ -7,9 +7,8 @@ both, each output element is one chain of v_mfma_f32_32x32x16_bf16 over the
 same k steps in the same order, so the layouts must agree bit for bit.  The
 hook uttt_debug_set_gemm_layout forces one layout process-wide; each case
 below runs the APPLY (general tiles), the UPDATE forward and its backward
-(from saved tensors and recomputing), the split-K weight gradients, the
-kernel-level compat pieces and Newton-Schulz under both layouts, on ragged
-groups, empty experts, K tails, two batches and the super-tile order, and
+(from saved tensors and recomputing), the split-K weight gradients and the
+kernel-level compat pieces under both layouts, on ragged groups, empty experts, K tails, two batches and the super-tile order, and
 compares every output with torch.equal.  The eight-wave kernels are also run
 through the oracle parity tests of the general path.
 """
@@ -142,6 +141,7 @@ def test_layouts_bit_identical_split_k(name):
 
 @pytest.mark.parametrize("n,R,C", [(3, 64, 128), (2, 256, 128), (1, 40, 200)])
 def test_layouts_bit_identical_newton_schulz(n, R, C):
+    """Newton-Schulz has tiles of its own, which the hook leaves alone."""
     from uttt_amd import fast_weight_write as FWW
 
     g = torch.Generator().manual_seed(n)

@@ -1,13 +1,12 @@
 """The XCD super-tile order of the token-grouped GEMMs against the oracle.
 
-Grids of 2048 workgroup tiles or more (the batched UPDATE at configs[4], the
-Newton-Schulz B X products of the 760M pool) map workgroups to tiles through
-the super-tile index math of tn_kernel; smaller grids keep the plain order.
+Grids of 2048 workgroup tiles or more (the 24-writer UPDATE of 32 experts of
+1536 x 3072) map workgroups to tiles through the super-tile index math of
+tn_kernel; smaller grids keep the plain order.
 Here the threshold is lowered to one tile (uttt_debug_set_supertile_min_tiles,
 a process-wide test hook), so every launch of the parity cases below -- APPLY
 forward and backward, UPDATE forward and backward with every pre-pass and
-chained product, the kernel-level compat pieces and Newton-Schulz -- takes
-that order, with super-tiles that overhang the grid on both axes, and is
+chained product, and the kernel-level compat pieces -- takes that order, with super-tiles that overhang the grid on both axes, and is
 checked in full against the same oracle bars as the plain order.
 """
 import pytest
@@ -69,5 +68,6 @@ def test_compat_pieces_supertile(name):
 
 @pytest.mark.parametrize("n,R,C", [(3, 64, 128), (2, 256, 128), (1, 40, 200)])
 def test_newton_schulz5_supertile(n, R, C):
+    """Newton-Schulz has tiles of its own, which the hook leaves alone."""
     import torch
     TM.test_newton_schulz5_matches_oracle(n, R, C, torch.float32, 1.0)

@@ -56,6 +56,33 @@ def test_chunked_weight_gradients(name):
                 assert bool(((ours.double() - ref).abs() <= bound).all()), (b, e, n)
 
 
+@pytest.mark.parametrize("name", list(WGRAD))
+def test_weight_gradients_equal_general_tiles(name):
+    """The forced 256 x 256 tiles (whole segments, or split K over few tiles):
+    the same products, an expert of several pieces added in another order."""
+    sizes, D, I, N = WGRAD[name]
+    gs = torch.tensor(sizes, dtype=torch.int32, device=DEV)
+    B, E = gs.shape
+    N = int(gs.sum(1).max()) if N is None else N
+    g = torch.Generator().manual_seed(N)
+    ins = [torch.randn(B, N, w, generator=g).to(torch.bfloat16).to(DEV) for w in (2 * I, D, I, D)]
+    ours = G.wgrad_pair(*ins, gs)
+    prev = L.lib().uttt_debug_set_gemm_layout(2)
+    try:
+        whole = L.lib().uttt_grouped_wgrad_pair_workspace_bytes(B, E, I, D, N) == 0
+        general = G.wgrad_pair(*ins, gs)
+    finally:
+        L.lib().uttt_debug_set_gemm_layout(prev)
+    for a, b in zip(ours, general):
+        for e in range(E):
+            n = int(gs[:, e].max())
+            x, y = a[:, e].double(), b[:, e].double()
+            if whole and n <= 512:   # one piece on either side: the same chain of products
+                assert torch.equal(x, y), e
+            else:                    # as above: one rounding each, sums in two orders
+                assert bool(((x - y).abs() <= 2.0 ** -7 * y.abs() + n * n * 2.0 ** -23).all()), e
+
+
 @pytest.mark.parametrize("given", ["none", "short", "unaligned"])
 def test_weight_gradients_without_room_for_partials(given):
     """48 experts of 192 x 192 with segments of several chunks: the workspace is

@@ -1659,8 +1659,15 @@ ApArgs apply_args(const void* w, const void* x, int K, int64_t a_group, int row_
   return a;
 }
 
-// Tests force a layout or tile order of the general tiles: everything takes them then.
+// Tests force a layout or tile order of the general tiles: every product with a
+// choice takes them then (Newton-Schulz has none).
 bool general_forced() { return g_gemm_na != 0 || g_xcd_map_min_tiles != kXcdMapMinTiles; }
+
+Wg192Plan wgrad_plan(int B, int E, int I, int D, int N) {
+  Wg192Plan p = wg192_plan(B, E, I, D, N);
+  p.use = p.use && !general_forced();
+  return p;
+}
 
 // bf16 products on 192 x 192 tiles with two workgroups per CU instead of 256 x
 // 256 with one (the same bits):
@@ -2010,7 +2017,7 @@ extern "C" size_t uttt_grouped_wgrad_pair_workspace_bytes(int B, int E, int I, i
   if (B <= 0 || E <= 0 || I <= 0 || D <= 0 || N <= 0) return 0;
   const WgTask t0 = wg_task(nullptr, nullptr, nullptr, 2 * I, D);
   const WgTask t1 = wg_task(nullptr, nullptr, nullptr, D, I);
-  const Wg192Plan pl = wg192_plan(B, E, I, D, N);
+  const Wg192Plan pl = wgrad_plan(B, E, I, D, N);
   if (pl.use) return pl.bytes;
   size_t off1;
   return wg_part_bytes(t0, t1, B, E, wg_splits(t0, t1, B, E, N), &off1);
@@ -2031,7 +2038,7 @@ extern "C" int uttt_grouped_wgrad_pair(const void* dy0_dy2_tok, const void* k,
                    aligned16(dw0_w2) && aligned16(dw1),
                "grouped_wgrad_pair: tensors must be 16-byte aligned");
   // dW0_W2 [2I][D] = DY^T K;  dW1 [D][I] = V^T Hid
-  const Wg192Plan pl = wg192_plan(B, E, I, D, N);
+  const Wg192Plan pl = wgrad_plan(B, E, I, D, N);
   // without room for its partials: the 256-tile kernel, a segment per workgroup
   if (pl.use &&
       (pl.bytes == 0 || (workspace && workspace_bytes >= pl.bytes && aligned16(workspace))))
@@ -2280,7 +2287,7 @@ extern "C" int uttt_grouped_update_bwd(
                                    "grouped_update_bwd(grad_V)"))
     return rc;
   // 7. grad_W0_W2 [2I][D] = grad_x0_x2^T K;  grad_W1 [D][I] = V^T grad_dh
-  const Wg192Plan pl = wg192_plan(B, E, I, D, N);
+  const Wg192Plan pl = wgrad_plan(B, E, I, D, N);
   if (pl.use && pl.bytes <= ws.gx)  // the partials over dhg, gy and dx, which nothing reads any more
     return launch_wg192(pl, gx, k, gdh, v, grad_w0_w2, grad_w1, group_sizes, B, E, I, D, N, wsb, st,
                         "grouped_update_bwd(weights)");
