@@ -83,6 +83,23 @@ def test_weight_gradients_equal_general_tiles(name):
                 assert bool(((x - y).abs() <= 2.0 ** -7 * y.abs() + n * n * 2.0 ** -23).all()), e
 
 
+def test_weight_gradients_of_many_batches():
+    """More than 65 535 (batch, expert) pairs, segments of two pieces among them."""
+    B, E, D, I, N = 1024, 65, 8, 8, 520
+    g = torch.Generator().manual_seed(2)
+    gs = torch.zeros(B, E, dtype=torch.int32)
+    gs[:, 0], gs[:, 64] = 3, 517          # the last expert's segment starts at 3
+    dy, k, hid, v = (torch.randint(-2, 3, (B, N, w), generator=g).to(torch.bfloat16).to(DEV)
+                     for w in (2 * I, D, I, D))
+    dw02, dw1 = G.wgrad_pair(dy, k, hid, v, gs.to(DEV))
+    for e, s in ((0, slice(0, 3)), (64, slice(3, 520))):   # small whole numbers: exact sums
+        for ours, p, q in ((dw02, dy, k), (dw1, v, hid)):
+            pt = p[:, s].float().transpose(1, 2).contiguous()
+            ref = torch.bmm(pt, q[:, s].float().contiguous())
+            assert torch.equal(ours[:, e].float(), ref.to(torch.bfloat16).float())
+    assert torch.count_nonzero(dw02[:, 1:64]) == 0 and torch.count_nonzero(dw1[:, 1:64]) == 0
+
+
 @pytest.mark.parametrize("given", ["none", "short", "unaligned"])
 def test_weight_gradients_without_room_for_partials(given):
     """48 experts of 192 x 192 with segments of several chunks: the workspace is

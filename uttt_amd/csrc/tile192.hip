@@ -162,9 +162,11 @@ __global__ __launch_bounds__(kTThreads, 2) void wg192_kernel(Wg192Args a) {
 }
 
 // The outputs of the experts with several chunks: bf16 of the partials' sum,
-// added in chunk order.  blockIdx.y = b * E + e.
-__global__ __launch_bounds__(256) void wg192_reduce_kernel(Wg192Args a) {
-  const int b = blockIdx.y / a.E, e = blockIdx.y % a.E;
+// added in chunk order.  `each` workgroups per (b, e), in one grid axis (the
+// others end at 65 535, which B * E need not).
+__global__ __launch_bounds__(256) void wg192_reduce_kernel(Wg192Args a, int each) {
+  const int be = blockIdx.x / each, blk = blockIdx.x % each;
+  const int b = be / a.E, e = be % a.E;
   const int lane = threadIdx.x & 63;
   const int32_t* gs_b = a.gs + (int64_t)b * a.E;
   int tok_base = 0, slot = 0, parts = 0;
@@ -187,8 +189,7 @@ __global__ __launch_bounds__(256) void wg192_reduce_kernel(Wg192Args a) {
   if (parts < 2) return;
   const int64_t n0 = (int64_t)a.t[0].X * a.t[0].Y;
   const float* src = a.part + ((int64_t)b * a.parts_ub + slot) * a.n_out;
-  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < a.n_out;
-       i += (int64_t)gridDim.x * 2048) {
+  for (int64_t i = ((int64_t)blk * 256 + threadIdx.x) * 8; i < a.n_out; i += (int64_t)each * 2048) {
     float v[8] = {};
 #pragma unroll 4
     for (int s = 0; s < parts; ++s) {
@@ -411,8 +412,9 @@ int launch_wg192(const Wg192Plan& pl, const void* dy, const void* k, const void*
   hipLaunchKernelGGL(wg192_kernel, dim3((unsigned)(units * pl.per)), dim3(kTThreads), 0, st, a);
   if (int rc = check_launch(what)) return rc;
   if (pl.parts_ub == 0) return UTTT_OK;  // no expert has a second chunk
-  const unsigned blocks = (unsigned)std::min<int64_t>((pl.n_out / 8 + 255) / 256, 64);
-  hipLaunchKernelGGL(wg192_reduce_kernel, dim3(blocks, (unsigned)(B * E)), dim3(256), 0, st, a);
+  const int each = (int)std::min<int64_t>((pl.n_out / 8 + 255) / 256, 64);
+  UTTT_REQUIRE((int64_t)B * E * each <= 0x7fffffffLL, "%s: problem too large for one launch", what);
+  hipLaunchKernelGGL(wg192_reduce_kernel, dim3((unsigned)(B * E * each)), dim3(256), 0, st, a, each);
   return check_launch(what);
 }
 
