@@ -67,6 +67,29 @@ def test_wgrad_pair_split_rule():
 
 
 @pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
+def test_wgrad_partials_fit_the_backward():
+    """The partials of chunked weight gradients take at most 12 B N I bytes, the
+    dead intermediates in which the UPDATE backward keeps them (a query that
+    the forced general tiles answer otherwise)."""
+    lib = _lib.lib()
+    q, hook = lib.uttt_grouped_wgrad_pair_workspace_bytes, lib.uttt_debug_set_gemm_layout
+    seen = 0
+    for B in (1, 12):
+        for E in (2, 33, 96):
+            for I in (8, 136, 192, 384, 512, 1536):
+                for D in (8, 192, 512, 768, 2056, 4096):
+                    for N in (100, 8400, 24576, 196608):
+                        prev = hook(2)
+                        general = q(B, E, I, D, N)
+                        hook(prev)
+                        n = q(B, E, I, D, N)
+                        if n != general:
+                            seen += 1
+                            assert n <= 12 * B * N * I, (B, E, I, D, N)
+    assert seen > 20
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
 def test_inverse_row_map_rule_matches_the_library():
     """routing.src_rows_supported restates uttt_route_tokens_map_src_rows in
     Python (so torch.compile traces the routed read); both are pure host

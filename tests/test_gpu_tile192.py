@@ -17,8 +17,9 @@ from uttt_amd.lact_moe_triton import _grouped as G
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
-# (group sizes per batch, D, I, N or None): chunks start at 512 tokens (at
-# least 2 D) for D, I <= 512; wider experts take them with short segments
+# (group sizes per batch, D, I, N or None): pieces start at 512 tokens (at
+# least 2 D) for D, I <= 512, else at 4096; some sizes take whole segments on
+# the 256 x 256 tiles (wg192_plan)
 WGRAD = {
     "chunk_edges": ([[512, 513, 0, 511, 1024, 1025, 31, 1]], 192, 192, None),
     "ragged_widths_two_batches": ([[700, 0, 1300], [1, 1999, 0]], 200, 104, None),
@@ -28,6 +29,12 @@ WGRAD = {
     "wide_short": ([[3, 200, 0, 129, 64, 33, 1, 250]], 520, 776, None),
     "all_empty": ([[0, 0, 0]], 192, 384, 64),
     "long": ([[9000, 2, 5000]], 64, 128, None),
+    "pieces_ragged_widths": ([[700, 0, 1300] + [0] * 5, [1, 1999, 0] + [0] * 5], 200, 104, None),
+    "pieces_slack_rows": ([[600, 40, 900, 0, 0]], 384, 384, 1700),
+    "pieces_over_count": ([[600, 900, 700, 0, 0, 0]], 96, 200, 1400),
+    "pieces_long": ([[9000, 2, 5000] + [0] * 53], 64, 128, None),
+    "pieces_deep": ([[8300, 0, 60] + [1] * 30], 2056, 8, None),   # pieces of 2 D or more tokens
+    "few_chunks": ([[0, 250]], 1544, 264, None),   # tiles of one dealt to the XCDs
 }
 
 

@@ -2288,9 +2288,11 @@ extern "C" int uttt_grouped_update_bwd(
     return rc;
   // 7. grad_W0_W2 [2I][D] = grad_x0_x2^T K;  grad_W1 [D][I] = V^T grad_dh
   const Wg192Plan pl = wgrad_plan(B, E, I, D, N);
-  if (pl.use && pl.bytes <= ws.gx)  // the partials over dhg, gy and dx, which nothing reads any more
+  if (pl.use) {  // the partials over dhg, gy and dx, which nothing reads any more (12 B N I bytes)
+    UTTT_REQUIRE(pl.bytes <= ws.gx, "grouped_update_bwd: %zu bytes of partials in %zu", pl.bytes, ws.gx);
     return launch_wg192(pl, gx, k, gdh, v, grad_w0_w2, grad_w1, group_sizes, B, E, I, D, N, wsb, st,
                         "grouped_update_bwd(weights)");
+  }
   const WgTask t0 = wg_task(k, gx, grad_w0_w2, 2 * I, D);
   const WgTask t1 = wg_task(gdh, v, grad_w1, D, I);
   return launch_wg(t0, t1, group_sizes, B, E, N, 1, nullptr, 0, st, "grouped_update_bwd(weights)");

@@ -71,6 +71,7 @@ struct Wg192Args {
   int64_t n_out;     // elements of both outputs of one expert
   int B, E, N, chunk;
   int slots, parts_ub;  // upper bounds of one batch's chunks and partial chunks
+  int run;              // tiles of one chunk that run on one XCD
 };
 
 // Chunk `slot` of a batch: its expert, first token, tokens, and its index
@@ -119,11 +120,12 @@ __global__ __launch_bounds__(kTThreads, 2) void wg192_kernel(Wg192Args a) {
   __shared__ __attribute__((aligned(16))) uint8_t ring[kTRing * kTStage];
   const int n0 = a.t[0].y_tiles * a.t[0].x_tiles;
   const int per = n0 + a.t[1].y_tiles * a.t[1].x_tiles;
-  // the tiles of one chunk run on one XCD: they read the same token rows
-  const int loc = blockIdx.x / kXcds;
-  const int unit = loc / per * kXcds + blockIdx.x % kXcds;
-  const int t = loc % per;
-  if (unit >= a.B * a.slots) return;
+  // the tiles of one chunk run on one XCD (they read the same token rows), or,
+  // of few chunks, in runs of a.run tiles dealt to the XCDs
+  const int loc = blockIdx.x / kXcds, runs = (per + a.run - 1) / a.run;
+  const int r = loc / a.run * kXcds + blockIdx.x % kXcds;
+  const int unit = r / runs, t = r % runs * a.run + loc % a.run;
+  if (unit >= a.B * a.slots || t >= per) return;
   const int b = unit / a.slots;
   const ChunkPos cp = find_chunk(a.gs + (int64_t)b * a.E, a.E, a.N, a.chunk, unit - b * a.slots);
   if (cp.e < 0) return;
@@ -367,19 +369,27 @@ int tiles_of(int n) { return (n + kT - 1) / kT; }
 }  // namespace
 
 // ------------------------------------------------------------------ host ----
+constexpr int kWgRuns = 64;  // runs of tiles that the weight gradients deal to the XCDs at least
 Wg192Plan wg192_plan(int B, int E, int I, int D, int N) {
   Wg192Plan p{};
   // dW0_W2 [2I][D] and dW1 [D][I]
   p.per = tiles_of(2 * I) * tiles_of(D) + tiles_of(D) * tiles_of(I);
-  const int64_t tiles256 =
-      (int64_t)B * E * (((2 * I + 255) / 256) * ((D + 255) / 256) + ((D + 255) / 256) * ((I + 255) / 256));
+  const auto tiles_256 = [](int n) { return (int64_t)(n + 255) / 256; };
+  const int64_t per256 = tiles_256(2 * I) * tiles_256(D) + tiles_256(D) * tiles_256(I);
+  const int64_t tiles256 = B * E * per256;
+  // tile area against that of the 256 x 256 tiles: at most 3/4, at most 1.05
+  const int64_t area192 = (int64_t)p.per * kT * kT, area256 = per256 * 65536;
+  const bool less = 4 * area192 <= 3 * area256, alike = 20 * area192 <= 21 * area256;
+  const int64_t mean = N / std::max(E, 1);
+  p.use = E > 1 && N > 0 &&
+          ((less && (tiles256 > 64 || mean <= 512)) ||
+           (mean <= 256 && tiles256 < 2048 &&
+            (tiles256 <= 64 || (alike && (tiles256 <= 128 || tiles256 > 256)))));
   const bool narrow = I <= 512 && D <= 512;
-  p.use = E > 1 && N > 0 && (narrow || (N <= 256 * (int64_t)E && tiles256 < 2048));
-  int chunk = 4096;
-  if (narrow) {
-    chunk = 512;
-    while (chunk < 4096 && (chunk < 2 * D || (int64_t)chunk * 256 < (int64_t)B * N * p.per)) chunk *= 2;
-  }
+  int chunk = narrow ? 512 : 4096;
+  while (chunk < 2 * D ||
+         (narrow && chunk < 4096 && (int64_t)chunk * 256 < (int64_t)B * N * p.per))
+    chunk *= 2;
   p.chunk = chunk;
   p.slots = (N + chunk - 1) / chunk + E;
   p.parts_ub = N > chunk ? (int)(2 * (int64_t)N / chunk) : 0;
@@ -391,8 +401,10 @@ Wg192Plan wg192_plan(int B, int E, int I, int D, int N) {
 int launch_wg192(const Wg192Plan& pl, const void* dy, const void* k, const void* hid,
                  const void* v, void* dw0_w2, void* dw1, const int32_t* gs, int B, int E, int I,
                  int D, int N, void* workspace, hipStream_t st, const char* what) {
-  const int64_t units = ((int64_t)B * pl.slots + kXcds - 1) / kXcds * kXcds;
-  UTTT_REQUIRE(units * pl.per <= 0x7fffffffLL, "%s: problem too large for one launch", what);
+  const int64_t units = (int64_t)B * pl.slots;
+  const int run = (int)std::max<int64_t>(1, std::min<int64_t>(pl.per, pl.per * units / kWgRuns));
+  const int64_t blocks = (units * ((pl.per + run - 1) / run) + kXcds - 1) / kXcds * kXcds * run;
+  UTTT_REQUIRE(blocks <= 0x7fffffffLL, "%s: problem too large for one launch", what);
   Wg192Args a{};
   auto task = [](const void* p, const void* q, void* out, int X, int Y) {
     return Wg192Task{static_cast<const uint16_t*>(p), static_cast<const uint16_t*>(q),
@@ -408,8 +420,9 @@ int launch_wg192(const Wg192Plan& pl, const void* dy, const void* k, const void*
   a.N = N;
   a.chunk = pl.chunk;
   a.slots = pl.slots;
+  a.run = run;
   a.parts_ub = pl.parts_ub;
-  hipLaunchKernelGGL(wg192_kernel, dim3((unsigned)(units * pl.per)), dim3(kTThreads), 0, st, a);
+  hipLaunchKernelGGL(wg192_kernel, dim3((unsigned)blocks), dim3(kTThreads), 0, st, a);
   if (int rc = check_launch(what)) return rc;
   if (pl.parts_ub == 0) return UTTT_OK;  // no expert has a second chunk
   const int each = (int)std::min<int64_t>((pl.n_out / 8 + 255) / 256, 64);

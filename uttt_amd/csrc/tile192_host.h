@@ -7,21 +7,27 @@ namespace uttt {
 
 // Chunked weight gradients of the grouped UPDATE on 192 x 192 tiles: `use`
 // where they are the faster ones, a pure function of the sizes (so the
-// workspace query and the launch agree):
-//   - narrow experts (I, D <= 512): the 256 x 256 tiles are half padding and
-//     one expert's few tiles are bound by its longest segment (48 experts of
-//     192 x 192 over 196 608 tokens: 285-459 -> 105 us; 96 of 384 x 384 over
-//     16 384: 70 -> 46, over 196 608: 374 -> 290);
-//   - short segments (at most 256 tokens per expert on average) on grids under
-//     eight rounds of 256-tile workgroups: 16 experts of 768 x 1536 over 3062
-//     tokens 71 -> 57 us; 32 of 1536 x 3072 over 4096 (27 rounds) 420 / 423.
-// Not for one expert per batch (uTTT-Dense heads), where the split-K 256 tiles
-// measure the same or faster (4 x [192 x 384] over 98 304 tokens 79 / 90 us).
-// Longer segments of wide experts keep the 256 tiles (16 of 768 x 1536 over
-// 49 152 tokens: 394 / 521 us).
+// workspace query and the launch agree), from 3000 sizes (2 to 128 experts, I
+// and D from 64 to 512 and wider with short segments, 64 to 196 608 tokens) timed on
+// both:
+//   - at most 3/4 of the 256 x 256 tiles' area (sides of 192, 320, 384): 48
+//     experts of 192 x 192 over 196 608 tokens 285-459 -> 105 us; 96 of 384 x
+//     384 over 16 384 70 -> 46, over 196 608 374 -> 290.  Not with few tiles and
+//     long segments, which the split-K 256 tiles cover (4 experts of 192 x 384
+//     over 4096 tokens 19 / 23 us);
+//   - means of at most 256 tokens, where a prologue and an epilogue per tile
+//     weigh most: with few tiles any width, else a like area (16 experts of 768
+//     x 1536 over 3062 tokens 71 -> 57 us), but not in place of one even round
+//     of 256 tiles on the 256 CUs (32 of 64 x 512 over 8192 27 / 32 us).
+// Sides of 256 and 512 pad by up to 1.9 times (8 experts of 512 x 256 over
+// 196 608 tokens 196 / 374 us).  One expert per batch (uTTT-Dense heads): the
+// split-K 256 tiles measure the same or faster (4 x [192 x 384] over 98 304
+// tokens 79 / 90 us).  Still up to 1.3 times slower: 8 to 32 experts with long
+// segments of one length (32 of 384 x 192 over 98 304: 83 / 109 us), where
+// unequal ones are up to twice faster.
 // Chunk length: about 256 (chunk, tile) workgroups on an even routing, 512 to
-// 4096 tokens, at least 2 D (a batch's partials then fit in the backward's
-// dead intermediates, 12 N I bytes).
+// 4096 tokens (4096 with a side above 512), at least 2 D: a batch's partials then
+// fit in the backward's dead intermediates, 12 N I bytes.
 struct Wg192Plan {
   bool use;
   int per;        // output tiles of one expert
