@@ -130,3 +130,22 @@ def test_short_segments_on_192_tiles_equal_general_tiles():
     n = int(gs.sum())
     for a, b in zip(ours, general):
         assert torch.equal(a[:, :n], b[:, :n])
+
+
+@pytest.mark.parametrize("M,K,sizes", [
+    (384, 16, [200000, 0, 3, 140001, 53333]),   # super-tiles that overhang the token tiles
+    (1736, 8, [97] * 640),                       # ten row tiles in super-tiles of eight
+])
+def test_super_tiles_of_192_equal_general_tiles(M, K, sizes):
+    """Grids of 4096 tiles and more."""
+    gs = torch.tensor([sizes], dtype=torch.int32, device=DEV)
+    E, N = len(sizes), sum(sizes)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)
+    W, Wt, X = rnd(1, E, K, M), rnd(1, E, M, K), rnd(1, N, K)
+    products = lambda: [G.gemm_tn(W, X, gs), G.gemm_nt(Wt, X, gs)]
+    ours = products()
+    with general_tiles():
+        general = products()
+    for a, b in zip(ours, general):
+        assert torch.equal(a, b)

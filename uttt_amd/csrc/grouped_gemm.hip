@@ -1670,20 +1670,33 @@ Wg192Plan wgrad_plan(int B, int E, int I, int D, int N) {
 }
 
 // bf16 products on 192 x 192 tiles with two workgroups per CU instead of 256 x
-// 256 with one (the same bits):
-//   - narrow experts (M <= 512 rows, K <= 1024), bound by the token rows: 48
-//     experts of 192 x 192 over 196 608 tokens 107 -> 88 us (grad_K) and 70 ->
-//     55 (grad_V); 96 of 384 x 384 over 16 384 evenly / unevenly routed ones 43
-//     -> 36 / 77 -> 49 and 26 -> 23 / 40 -> 32;
-//   - short segments (at most 256 tokens per expert on average) of experts up
-//     to 768 x 3072: 16 over 3062 tokens 120 -> 112 and 66 -> 60 us.
-// Larger experts re-read their weights per 192 tokens from beyond the L2: 32 of
-// 1536 x 3072 over 4096 unevenly routed tokens 358 / 401 us, over 98 304 3176 /
-// 3540; 16 of 768 x 1536 over 49 152 257 / 265 (grad_V).
-bool use_tn192(int M, int K, int N, int E) {
+// 256 with one (the same bits), for narrow experts (M <= 512 rows, K <= 1024),
+// bound by the token rows, and for short segments (at most 256 tokens per expert
+// on average) of experts of up to 4.5 MiB, about one XCD's L2 (larger ones
+// re-read their weights per 192 tokens: 32 of 1536 x 3072 over 4096 unevenly
+// routed tokens 358 / 401 us).  Within these by the rounds over the chip, from the
+// expected tiles: 256 of the one and 512 of the other run at once, a full round
+// of the latter taking 1.125 times as long (2 x 9/16 of the products per CU), and
+// up to 256 of them, one per CU, 0.6.  48 experts of 192 x 192: over 16 384 tokens
+// (T = 88 / 109 tiles) 24.9 -> 22.2 us (grad_K), over 49 152 (216 / 280) 30.5 / 39.6, so
+// 256 x 256, over 196 608 (792 / 1048) 127 -> 107; 8 of 512 x 256 over 16 384 30.7 / 38.
+// Row-major weights of segments of at most 32 tokens: the 256-tile kernel skips
+// the products of absent tokens (4 of 4096 x 288 over 32 104 / 146 us).  Of 16 000
+// timings (1 to 96 experts, widths 64 to 6144, 32 to 196 608 tokens) 55 on these
+// tiles are over 6 % slower than on the others, against 2571 by widths alone.
+bool use_tn192(bool a_kmajor, int M, int K, int N, int B, int E) {
   if (general_forced() || K <= 0) return false;
-  return (M <= 512 && K <= 1024) ||
-         (N <= 256 * (int64_t)E && (int64_t)M * K <= (int64_t)768 * 3072);
+  const bool narrow = M <= 512 && K <= 1024;
+  const bool small = N <= 256 * (int64_t)E && (int64_t)M * K <= (9 << 18);
+  if (!(narrow || small) || (a_kmajor && N <= 32 * (int64_t)E)) return false;
+  // a segment is cut about half a tile over its length, and takes one at least
+  const auto tiles = [&](int t) {
+    const int64_t tok = std::max<int64_t>(std::min(E, N), (N + t - 1) / t + E / 2);
+    return (M + t - 1) / t * tok * B;
+  };
+  const int64_t t256 = tiles(256), t192 = tiles(192);
+  const int64_t rounds256 = (t256 + 255) / 256, rounds192 = (t192 + 511) / 512;
+  return t192 <= 256 || 9 * rounds192 <= 8 * rounds256;
 }
 
 // Wide single product: y[b, n, m] = sum_k A(m, k) x[b, n, k] with M rows in
@@ -1693,7 +1706,7 @@ int launch_wide(const void* a, const void* x, int K, const void* a_2, const void
                 int M, int64_t lda, int64_t a_group, OutT* y, int B, int E, int N,
                 const int32_t* gs, hipStream_t st, const char* what) {
   if constexpr (std::is_same_v<OutT, uint16_t>) {
-    if (aligned16(y) && use_tn192(M, K, N, E))
+    if (aligned16(y) && use_tn192(AMAJ == KMajor, M, K, N, B, E))
       return launch_tn192(AMAJ == KMajor, a, x, K, a_2, x_2, K_2, M, y, B, E, N, gs, st, what);
   }
   TnArgs t = tn_args(a, a, x, K, lda, a_group, 0, kTileRows, M, M, 2 * kTileRows, M, B, E, N, gs);
