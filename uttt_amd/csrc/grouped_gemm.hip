@@ -1671,8 +1671,9 @@ Wg192Plan wgrad_plan(int B, int E, int I, int D, int N) {
 
 // bf16 products on 192 x 192 tiles with two workgroups per CU instead of 256 x
 // 256 with one (the same bits), for narrow experts (M <= 512 rows, K <= 1024),
-// bound by the token rows, and for short segments (at most 256 tokens per expert
-// on average) of experts of up to 4.5 MiB, about one XCD's L2 (larger ones
+// bound by the token rows, and for short segments (at most 192 tokens per expert
+// on average, one tile if even: 48 of 1024 x 1024 over 10 752 even ones, 224 each,
+// lost a quarter of the UPDATE backward) of experts of up to 4.5 MiB, about one XCD's L2 (larger ones
 // re-read their weights per 192 tokens: 32 of 1536 x 3072 over 4096 unevenly
 // routed tokens 358 / 401 us).  Within these by the rounds over the chip, from the
 // expected tiles: 256 of the one and 512 of the other run at once, a full round
@@ -1687,7 +1688,7 @@ Wg192Plan wgrad_plan(int B, int E, int I, int D, int N) {
 bool use_tn192(bool a_kmajor, int M, int K, int N, int B, int E) {
   if (general_forced() || K <= 0) return false;
   const bool narrow = M <= 512 && K <= 1024;
-  const bool small = N <= 256 * (int64_t)E && (int64_t)M * K <= (9 << 18);
+  const bool small = N <= 192 * (int64_t)E && (int64_t)M * K <= (9 << 18);
   if (!(narrow || small) || (a_kmajor && N <= 32 * (int64_t)E)) return false;
   // a segment is cut about half a tile over its length, and takes one at least
   const auto tiles = [&](int t) {
@@ -1997,7 +1998,7 @@ extern "C" int uttt_grouped_update_stage1(const void* w0_w2, const void* w1, con
   UTTT_REQUIRE(workspace_bytes >= need, "grouped_update_stage1: workspace %zu < %zu bytes",
                workspace_bytes, need);
   hipStream_t st = as_stream(stream);
-  if (token_major && narrow_stage1(I, D, N, E) && !general_forced())
+  if (token_major && narrow_stage1(I, D, N, B, E) && !general_forced())
     return launch_narrow_stage1(w0_w2, w1, k, v, lr0, lr1, lr2, lr_dtype, group_sizes, B, E, I, D, N,
                                 dy0_dy2, hidden, y0_y2_save, dh_save, st,
                                 "grouped_update_stage1");

@@ -7,11 +7,17 @@ namespace uttt {
 
 // Expert widths that narrow.hip's kernels take (any token counts).
 bool narrow_experts(int I, int D);
-// Sizes whose stage 1 it takes: also experts up to 768 x 1536 with at most 256
-// tokens on average, where half of the 256-token tiles is padding and the fp32
-// DH a round trip (16 over 3062 tokens: DH 34 + 64 us, here 69).  Their
-// backward gains nothing (GD 24 + 67 us, here 93 and twice the lr partials).
-bool narrow_stage1(int I, int D, int N, int E);
+// Sizes whose stage 1 it takes: also experts up to 768 x 1536 elements (the
+// product: 288 x 4096 and 4096 x 288 gain alike) with at most 256 tokens on
+// average, where half of the 256-token tiles is padding and the fp32 DH a round
+// trip (16 over 3062 tokens: DH 34 + 64 us, here 69).  Past 128 tokens only with
+// all weights within the 256 MB memory-side cache, since a second 128-token tile
+// then reads them again (128 experts of 768 x 1536 over 20 480: 333 / 405 us).
+// Their backward gains nothing (GD 24 + 67 us, here 93 and twice the lr
+// partials).  Of 3600 timings (1 to 128 experts, widths 8 to 8192) none is over
+// 6 % slower than the two launches, and of as many gate/up ones one (a few tokens
+// per expert, 9.6 / 10.5 us).
+bool narrow_stage1(int I, int D, int N, int B, int E);
 // Row blocks of its lr-gradient partials, lr_part[3][narrow_m_tiles][B][N].
 int narrow_m_tiles(int I);
 

@@ -20,8 +20,9 @@
 //   backward's second pass  302 us (two launches) -> 223 (830 MB, 3.7 TB/s)
 // 96 of 384 x 384 over 16 384 tokens, without saves: 89 -> 45 us; gate/up 42 ->
 // 31, of 48 x 192 x 192 17 -> 10.7 (against apply_kernel's 256 x 128 tiles).
-// Past 512 the products outweigh the rows and a token tile is read by more
-// than eight unit groups: the 256-token tiles' kernels (but see narrow_stage1).
+// Every I, D up to 512 measured gains (narrow_stage1's comment); past it long
+// segments were not timed, and a token tile is read by more than eight unit
+// groups: the 256-token tiles' kernels.
 #include "narrow.h"
 #include "tile192.h"
 
@@ -570,9 +571,11 @@ int narrow_args(NarrowArgs* a, const void* w0_w2, const void* w1, const void* k,
 
 // ------------------------------------------------------------------ host ----
 bool narrow_experts(int I, int D) { return I <= 512 && D <= 512 && D > kTK; }
-bool narrow_stage1(int I, int D, int N, int E) {
+bool narrow_stage1(int I, int D, int N, int B, int E) {
+  const int64_t weights = (int64_t)6 * B * E * I * D;  // bytes
   return narrow_experts(I, D) ||
-         (D > kTK && N <= 256 * (int64_t)E && (int64_t)I * D <= (int64_t)768 * 1536);
+         (D > kTK && (int64_t)I * D <= (int64_t)768 * 1536 &&
+          (N <= 128 * (int64_t)E || (N <= 256 * (int64_t)E && weights <= (256 << 20))));
 }
 int narrow_m_tiles(int I) { return (I + kHid - 1) / kHid; }
 
