@@ -48,6 +48,31 @@ def test_routes():
         assert _run(x)[1] == "_NoGraph"
 
 
+class _Address(torch.autograd.Function):
+    """Takes the storage's address, as every C call does."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x + (0 if x.data_ptr() else 1)
+
+    @staticmethod
+    def backward(ctx, g):
+        return g
+
+
+def test_a_tensor_that_outlived_its_transform():
+    kept = []
+
+    def loss(x):
+        kept.append(x * 2)
+        return kept[0].sum()
+
+    x = torch.randn(3)
+    torch.func.grad(loss)(x)
+    with torch.no_grad():
+        assert torch.equal(run_function(_Address, kept[0]), x * 2)
+
+
 def test_transforms_take_apply():
     with torch.no_grad():
         with pytest.raises(RuntimeError, match="setup_context|vmap"):

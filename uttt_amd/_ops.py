@@ -12,6 +12,7 @@ from __future__ import annotations
 import functools
 
 import torch
+from torch._functorch.utils import unwrap_dead_wrappers
 from torch.autograd import forward_ad
 
 
@@ -54,7 +55,9 @@ def run_function(fn, *args):
             or torch._C._are_functorch_transforms_active()
             or torch._C._get_tracing_state() is not None or forward_ad._current_level >= 0):
         return fn.apply(*args)
-    return fn.forward(_NoGraph(), *args)
+    # a tensor that outlived its functorch transform is a shell around the real
+    # one, which apply hands on
+    return fn.forward(_NoGraph(), *unwrap_dead_wrappers(args))
 
 
 def none_if_empty(t):
