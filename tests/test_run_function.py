@@ -48,6 +48,16 @@ def test_routes():
         assert _run(x)[1] == "_NoGraph"
 
 
+def test_an_input_handed_through_is_an_alias():
+    """As apply returns it: other metadata, the same storage."""
+    x, n = torch.randn(3), torch.zeros(1, dtype=torch.int32)
+    with torch.no_grad():
+        for out in (_Double.apply(x, n)[1], run_function(_Double, x, n)[1]):
+            assert out is not n and out.data_ptr() == n.data_ptr() and out._is_view()
+            out.unsqueeze_(0)
+            assert n.shape == (1,)
+
+
 class _Address(torch.autograd.Function):
     """Takes the storage's address, as every C call does."""
 

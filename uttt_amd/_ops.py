@@ -57,7 +57,12 @@ def run_function(fn, *args):
         return fn.apply(*args)
     # a tensor that outlived its functorch transform is a shell around the real
     # one, which apply hands on
-    return fn.forward(_NoGraph(), *unwrap_dead_wrappers(args))
+    args = unwrap_dead_wrappers(args)
+    out = fn.forward(_NoGraph(), *args)
+    if type(out) is tuple:  # an input that is handed through comes out as a tensor of its own
+        return tuple(o.view_as(o) if isinstance(o, torch.Tensor) and any(o is a for a in args) else o
+                     for o in out)
+    return out
 
 
 def none_if_empty(t):
