@@ -12,6 +12,7 @@ from __future__ import annotations
 import functools
 
 import torch
+from torch._C._functorch import is_dead_tensor_wrapper
 from torch._functorch.utils import unwrap_dead_wrappers
 from torch.autograd import forward_ad
 
@@ -55,13 +56,19 @@ def run_function(fn, *args):
             or torch._C._are_functorch_transforms_active()
             or torch._C._get_tracing_state() is not None or forward_ad._current_level >= 0):
         return fn.apply(*args)
-    # a tensor that outlived its functorch transform is a shell around the real
-    # one, which apply hands on
-    args = unwrap_dead_wrappers(args)
+    for a in args:
+        # a tensor that outlived its functorch transform is a shell around the
+        # real one, which apply hands on
+        if type(a) is torch.Tensor and is_dead_tensor_wrapper(a):
+            args = unwrap_dead_wrappers(args)
+            break
     out = fn.forward(_NoGraph(), *args)
-    if type(out) is tuple:  # an input that is handed through comes out as a tensor of its own
-        return tuple(o.view_as(o) if isinstance(o, torch.Tensor) and any(o is a for a in args) else o
-                     for o in out)
+    if type(out) is tuple:
+        ins = set(map(id, args))
+        for o in out:  # an input that is handed through comes out as a tensor of its own
+            if o is not None and id(o) in ins:
+                return tuple(t.view_as(t) if id(t) in ins and isinstance(t, torch.Tensor) else t
+                             for t in out)
     return out
 
 
