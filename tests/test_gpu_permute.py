@@ -266,8 +266,9 @@ def test_permute_roundtrip_full_size_property():
     torch.testing.assert_close(back.float(), x.float(), rtol=1e-2, atol=1e-2)
 
 
-@pytest.mark.parametrize("T,E", [(1, 25), (63, 64), (64, 65), (65, 128), (129, 33), (4112, 48),
-                                 (5000, 96), (70001, 27)])
+@pytest.mark.parametrize("T,E", [(1, 25), (9, 128), (63, 64), (64, 65), (65, 128), (129, 33),
+                                 (512, 65), (513, 65), (4112, 48), (5000, 96), (32904, 30),
+                                 (70001, 27)])
 @pytest.mark.parametrize("form", ["bool", "uint8_values", "int32", "token_major"])
 def test_row_map_from_64_token_tiles(T, E, form):
     """The general row map (E > 24, or too many tokens for one launch): every

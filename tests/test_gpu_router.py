@@ -279,6 +279,9 @@ def test_route_tokens_wide(B, T, D, E, k, rt):
     (1, 31, 768, 48, 1),       # one block per batch
     (3, 4100, 192, 48, 1),     # blocks of 64 tokens
     (1, 4128, 1536, 96, 3),    # more than 64 experts
+    (70, 9, 192, 100, 2),      # many short batches
+    (2, 255, 768, 65, 2),      # eight blocks of 32: one wave derives the offsets
+    (1, 33001, 8, 30, 1),      # more than 512 tiles
 ])
 def test_route_tokens_map_from_the_selection_counts(B, T, D, E, k):
     """Shapes off the one-launch row map: the map built from the selection's

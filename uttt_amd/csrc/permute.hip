@@ -5,8 +5,8 @@
 // permuted buffer is expert-major and token-ascending.  For E <= 24 two
 // launches (count per 256-token tile, then rowmap_scan_emit_kernel, which
 // derives each tile's offsets from the counts itself); else three over 64-token
-// tiles: rowmap_count64_kernel, rowmap_offsets_kernel (also group_sizes),
-// rowmap_emit64_kernel; after a router, whose selection leaves the counts, the
+// tiles: rowmap_count64_kernel, rowmap_offsets_kernel (or, of few tiles,
+// rowmap_offsets_few_kernel; also group_sizes), rowmap_emit64_kernel; after a router, whose selection leaves the counts, the
 // last two.  The packed per-token entry has the reference's format (rows and
 // experts in descending order, n_routed last, the reference's stale values in
 // columns [n, E)).
@@ -211,6 +211,7 @@ __device__ __forceinline__ void emit_tile(const uint32_t bits[kMaxExperts / 32],
 // per token wrote 4 bytes every 4 (2E + 1): 96 us at T = 196 608, E = 48, for 76 MB).
 constexpr int kTile64 = 64;
 constexpr int kExpertWords = kMaxExperts / kWave;  // experts per lane
+constexpr int kFewTiles = 8;  // tiles of a batch up to which one wave derives its offsets
 
 struct MaskView {
   const void* map;
@@ -363,6 +364,46 @@ __global__ __launch_bounds__(THREADS) void rowmap_offsets_kernel(
   }
 }
 
+// The same for few tiles: one wave per batch, whose lanes hold the experts and
+// walk the tiles.  A workgroup per (expert, batch) is E times as many, which at
+// short batches is most of the map's time (256 batches of 65 tokens, 128 experts:
+// the map 117 us, here 29).
+__global__ __launch_bounds__(kWave) void rowmap_offsets_few_kernel(
+    const int32_t* __restrict__ counts, int E, int ntiles, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ group_sizes, const float* __restrict__ part_bal, int nblk,
+    float* __restrict__ bal_sum) {
+  const int b = blockIdx.x, lane = lane_id();
+  const int32_t* tab = counts + (int64_t)b * ntiles * E;
+  int32_t* out = offsets + (int64_t)b * ntiles * E;
+  int before = 0;
+#pragma unroll
+  for (int q = 0; q < kExpertWords; ++q) {
+    const int e = lane + 64 * q;
+    const bool in = e < E;
+    int total = 0;
+    for (int t = 0; t < ntiles; ++t) total += in ? tab[t * E + e] : 0;
+    int incl = total;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int o = __shfl_up(incl, d, kWave);
+      if (lane >= d) incl += o;
+    }
+    int run = before + incl - total;
+    before += __shfl(incl, 63, kWave);
+    if (!in) continue;
+    for (int t = 0; t < ntiles; ++t) {
+      out[t * E + e] = run;
+      run += tab[t * E + e];
+    }
+    if (group_sizes != nullptr) group_sizes[(int64_t)b * E + e] = total;
+    if (part_bal != nullptr) {
+      float f = 0.0f;
+      for (int k = 0; k < nblk; ++k) f += part_bal[((int64_t)b * nblk + k) * E + e];
+      bal_sum[(int64_t)b * E + e] = f;
+    }
+  }
+}
+
 // The map of one 64-token tile per workgroup, TPW tokens per wave (offsets in
 // tiles of `tt` = 32 or 64 tokens).  Per token, the lanes' routed flags are one
 // ballot per 64 experts: n and the experts come from it, the rows from the
@@ -373,13 +414,32 @@ __global__ __launch_bounds__(kTile64 / TPW * kWave) void rowmap_emit64_kernel(Ma
                                                               const int32_t* __restrict__ offsets,
                                                               int32_t* __restrict__ row_id_map) {
   constexpr int kPasses = (2 * kMaxExperts + 1 + kWave - 1) / kWave;
+  __shared__ uint64_t words[kMaxExperts];
   const int b = blockIdx.y, t0 = blockIdx.x * kTile64;
   const int w = threadIdx.x / kWave, lane = lane_id();
   const int first = TPW * w;                      // this wave's first token in the tile
-  if (t0 + first >= T) return;
   const int W = 2 * E + 1;
   uint64_t bits[kExpertWords];
-  tile_bits<MB>(m, b, t0, T, E, bits);
+  if (MB == 1 && m.fast && t0 + kTile64 <= T) {
+    tile_bits<MB>(m, b, t0, T, E, bits);
+  } else {  // the waves share the experts' ballots
+    const int t = min(t0 + lane, T - 1);
+    const int64_t base = (int64_t)b * m.s_b + (int64_t)t * m.s_t;
+    for (int e0 = 8 * w; e0 < E; e0 += 8 * (int)(blockDim.x / kWave)) {
+      bool on[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) on[i] = mask_bit<MB>(m.map, base + (int64_t)min(e0 + i, E - 1) * m.s_e);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint64_t bal = __ballot(on[i] && t0 + lane < T);
+        if (lane == 0 && e0 + i < E) words[e0 + i] = bal;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kExpertWords; ++q) bits[q] = lane + 64 * q < E ? words[lane + 64 * q] : 0;
+  }
+  if (t0 + first >= T) return;
   const int nt = (T + tt - 1) / tt;
   const int toff = first / tt * tt;               // its offset tile's first token in the tile
   int next[kExpertWords];
@@ -1683,7 +1743,10 @@ void launch_offsets_emit(const MaskView& m, int B, int T, int E, const int32_t* 
                          int32_t* offsets, int32_t* group_sizes, const float* part_bal, int nblk,
                          float* bal_sum, int32_t* row_id_map, hipStream_t st) {
   const int nt = (T + tt - 1) / tt;
-  if ((int64_t)nt * E > 4096)
+  if (nt <= kFewTiles)
+    hipLaunchKernelGGL(rowmap_offsets_few_kernel, dim3(B), dim3(kWave), 0, st, counts, E, nt,
+                       offsets, group_sizes, part_bal, nblk, bal_sum);
+  else if ((int64_t)nt * E > 4096)
     hipLaunchKernelGGL(rowmap_offsets_kernel<1024>, dim3(E, B), dim3(1024), 0, st, counts, E, nt,
                        offsets, group_sizes, part_bal, nblk, bal_sum);
   else
@@ -1691,14 +1754,15 @@ void launch_offsets_emit(const MaskView& m, int B, int T, int E, const int32_t* 
                        offsets, group_sizes, part_bal, nblk, bal_sum);
   // few tiles: 4 tokens per wave (a token's entry is a serial chain: T = 517,
   // E = 16 9.2 -> 7.9 us); many: 16, which read the tile's mask four times
-  // less often
+  // less often.  As many waves as a (shorter) batch has tokens for.
   const int tiles = (T + kTile64 - 1) / kTile64;
+  const int tokens = T < kTile64 ? T : kTile64;
   if ((int64_t)tiles * B <= 512)
-    hipLaunchKernelGGL((rowmap_emit64_kernel<MB, 4>), dim3(tiles, B), dim3(1024), 0, st, m, T, E, tt,
-                       offsets, row_id_map);
+    hipLaunchKernelGGL((rowmap_emit64_kernel<MB, 4>), dim3(tiles, B), dim3((tokens + 3) / 4 * kWave),
+                       0, st, m, T, E, tt, offsets, row_id_map);
   else
-    hipLaunchKernelGGL((rowmap_emit64_kernel<MB, 16>), dim3(tiles, B), dim3(256), 0, st, m, T, E, tt,
-                       offsets, row_id_map);
+    hipLaunchKernelGGL((rowmap_emit64_kernel<MB, 16>), dim3(tiles, B),
+                       dim3((tokens + 15) / 16 * kWave), 0, st, m, T, E, tt, offsets, row_id_map);
 }
 }  // namespace
 
