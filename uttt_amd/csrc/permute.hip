@@ -1752,12 +1752,12 @@ void launch_offsets_emit(const MaskView& m, int B, int T, int E, const int32_t* 
   else
     hipLaunchKernelGGL(rowmap_offsets_kernel<256>, dim3(E, B), dim3(256), 0, st, counts, E, nt,
                        offsets, group_sizes, part_bal, nblk, bal_sum);
-  // few tiles: 4 tokens per wave (a token's entry is a serial chain: T = 517,
+  // few tiles or short batches: 4 tokens per wave (a token's entry is a serial chain: T = 517,
   // E = 16 9.2 -> 7.9 us); many: 16, which read the tile's mask four times
   // less often.  As many waves as a (shorter) batch has tokens for.
   const int tiles = (T + kTile64 - 1) / kTile64;
   const int tokens = T < kTile64 ? T : kTile64;
-  if ((int64_t)tiles * B <= 512)
+  if ((int64_t)tiles * B <= 512 || T <= 32)
     hipLaunchKernelGGL((rowmap_emit64_kernel<MB, 4>), dim3(tiles, B), dim3((tokens + 3) / 4 * kWave),
                        0, st, m, T, E, tt, offsets, row_id_map);
   else
