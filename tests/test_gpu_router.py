@@ -234,9 +234,11 @@ def test_route_tokens_map_src_rows_refused_where_the_row_map_takes_more_launches
 
 
 @pytest.mark.parametrize("B,T,D,E,k", [
-    (2, 9, 192, 48, 1),        # the smallest batch off the few-token path
+    (2, 9, 192, 48, 1),        # a short batch, on the other kernel
+    (2, 33, 192, 48, 1),       # the shortest on this one
     (1, 65, 40, 5, 3),         # one token past a block, a tail of 8 features
-    (3, 130, 256, 128, 4),     # every expert block, the widest of the narrow rows
+    (3, 130, 160, 128, 4),     # every expert block
+    (1, 70, 256, 80, 2),       # the widest of the narrow rows
     (2, 100, 8, 33, 33),       # one chunk of one lane group, all experts selected
     (1, 12289, 264, 17, 2),    # many tokens of wider rows: three groups of features
 ])

@@ -1208,16 +1208,23 @@ bool route_vec(const void* x, const float* router_w, int64_t w_sb, int D) {
 
 // Tokens per block of the fused logits + selection launch: 32
 // (router_mfma_kernel, whose waves share a token block's features) or
-// router_wide_kernel's.  The latter for bf16 rows of at most 256 features (E =
-// 48, D = 192: 800 tokens 11.8 -> 10.8 us, 16 384 tokens 22.7 -> 12.2, 196 608
-// tokens 232 -> 59), whose few steps a wave runs by itself, and from 12 288
-// tokens on, where its waves fill the chip: 16 384 tokens of 384 features and 96
-// experts 30.7 -> 24.4 us (6000: 19.7 / 22.0), 24 576 of 768 and 16 24.5 ->
-// 17.0 (2048: 11.8 / 14.0), 49 152 of 1536 and 32 76 -> 51 (2048: 15.4 / 27).
+// router_wide_kernel's.  The latter
+//   - for bf16 rows of at most 256 features and 20 480 weights (E = 48, D = 192: 800
+//     tokens 11.8 -> 10.8 us, 16 384 tokens 22.7 -> 12.2, 196 608 tokens 232 -> 59),
+//     whose few steps a wave runs by itself (96 experts of 256: 100 tokens 17 / 19);
+//   - from 12 288 tokens, and 16 per feature, on, where its waves fill the chip:
+//     16 384 tokens of 384 features and 96 experts 30.7 -> 24.4 us (6000: 19.7 /
+//     22.0), 24 576 of 768 and 16 24.5 -> 17.0 (2048: 11.8 / 14.0), 49 152 of 1536
+//     and 32 76 -> 51 (12 288 and 8: 24 / 28);
+//   - in batches of more than 32 tokens: shorter ones leave most of a 64-token block
+//     empty (2048 batches of 9 tokens, 256 features and 128 experts 112 / 167 us; 1024
+//     of 33 tokens 413 -> 245).
 int route_block_tokens(const void* x, int x_dtype, const float* router_w, int64_t w_sb, int B,
-                       int T, int D) {
-  const bool wide = x_dtype == UTTT_BF16 && T > kSmallT && route_vec(x, router_w, w_sb, D) &&
-                    (D <= 256 || (int64_t)B * T >= 12288);
+                       int T, int D, int E) {
+  const int64_t all = (int64_t)B * T;
+  const bool wide = x_dtype == UTTT_BF16 && T > 32 && route_vec(x, router_w, w_sb, D) &&
+                    ((D <= 256 && (int64_t)D * E <= 20480) ||
+                     (all >= 12288 && all >= 16 * (int64_t)D));
   return wide ? kWideWaves * 16 * kWideBlocks : 32;
 }
 
@@ -1322,7 +1329,7 @@ extern "C" int uttt_route_tokens(const void* x, int x_dtype, const float* router
   if (B == 0 || T == 0) return UTTT_OK;
   UTTT_REQUIRE(x && router_w && mask && combine && balance, "route_tokens: null pointer");
   // the workspace query assumes blocks of 32 tokens: larger ones need less
-  const int blk_tokens = route_block_tokens(x, x_dtype, router_w, w_sb, B, T, D);
+  const int blk_tokens = route_block_tokens(x, x_dtype, router_w, w_sb, B, T, D, E);
   Ws w = ws_layout(workspace, B, T, E, blk_tokens);
   UTTT_REQUIRE(workspace != nullptr && workspace_bytes >= w.bytes,
                "route_tokens: workspace %zu < %zu bytes", workspace_bytes, w.bytes);
@@ -1373,7 +1380,7 @@ extern "C" int uttt_route_tokens_map(const void* x, int x_dtype, const float* ro
   UTTT_REQUIRE(x && router_w && mask && combine && balance && group_sizes && balance_sum &&
                    row_id_map,
                "route_tokens_map: null pointer");
-  const int blk_tokens = route_block_tokens(x, x_dtype, router_w, w_sb, B, T, D);
+  const int blk_tokens = route_block_tokens(x, x_dtype, router_w, w_sb, B, T, D, E);
   Ws w = ws_layout(workspace, B, T, E, blk_tokens);
   const size_t rm_off = align256(w.bytes);
   const size_t need = rm_off + map_offsets_bytes(B, T, E);
