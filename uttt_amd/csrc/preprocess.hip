@@ -224,9 +224,13 @@ __global__ __launch_bounds__(kPrepThreads) void rows_prep_bwd_kernel(
     const int ch = lane + G * c;
     const bool ok = ch < chunks;
     if constexpr (ROPE) {
-      rope8(g[c], a, table, 8 * (ok ? ch : chunks - 1), true);
+      // the longest rows a chunk at a time (uniform branches; all chunks' rotations
+      // interleaved hold too many registers: 16 384 rows of 4096 191 / 249 us)
+      if (NI < kMaxChunksPerLane || G * c < chunks) {
+        rope8(g[c], a, table, 8 * (ok ? ch : chunks - 1), true);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) g[c][u] = rnd<TI>(rnd<BF16T>(g[c][u]));
+        for (int u = 0; u < 8; ++u) g[c][u] = rnd<TI>(rnd<BF16T>(g[c][u]));
+      }
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
