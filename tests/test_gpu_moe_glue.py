@@ -267,10 +267,14 @@ def test_routed_read_without_gradient_equals_the_permuted_path():
 @pytest.mark.parametrize("D,rope_dim", [(8, 0), (64, 64), (192, 64), (256, 256), (384, 128), (520, 0),
                                         (768, 16), (1032, 0), (1536, 64), (2048, 256), (4096, 32)])
 @pytest.mark.parametrize("norm", [None, "l2", "rms"])
-def test_rows_preprocess_row_widths(D, rope_dim, norm):
-    """Every lane-group width and chunk count of the row kernels, a row count
-    that does not fill the last workgroup, forward and backward."""
-    B, Lx = 1, 37
+@pytest.mark.parametrize("Lx", [37, 4101])
+def test_rows_preprocess_row_widths(D, rope_dim, norm, Lx):
+    """Every lane-group width and chunk count of the row kernels (few rows take
+    more lanes), a row count that does not fill the last workgroup, forward and
+    backward."""
+    if Lx > 37 and D > 768:
+        pytest.skip("64 lanes per row at either count")
+    B = 1
     g = torch.Generator().manual_seed(D)
     x = torch.randn(B, Lx, D, generator=g).to(torch.bfloat16)
     gy = torch.randn(B, Lx, D, generator=g).to(torch.bfloat16)
@@ -280,7 +284,16 @@ def test_rows_preprocess_row_widths(D, rope_dim, norm):
         rp, orp = moe.Rope(cos.to(DEV), sin.to(DEV), 5), (cos, sin, 5)
     xd = x.to(DEV).requires_grad_()
     y = moe.rows_preprocess(xd, silu=True, norm=norm, rows_of=D, rope=rp)
-    _close(y, MU.preprocess_rows(x, silu=True, norm=norm, rows_of=D, rope=orp), 8e-3, "forward")
+    fwd = MU.preprocess_rows(x, silu=True, norm=norm, rows_of=D, rope=orp)
     y.backward(gy.to(DEV))
     ref = MU.preprocess_rows_bwd(x, gy, silu=True, norm=norm, rows_of=D, rope=orp)
-    _close(xd.grad, ref, 2e-2, "backward")
+    if Lx == 37:
+        _close(y, fwd, 8e-3, "forward")
+        _close(xd.grad, ref, 2e-2, "backward")
+        return
+    # among many elements some rotate or project to nearly zero, so by rows: at most
+    # four bf16 roundings (2^-8 each) of values no longer than the row; one wrong
+    # element of up to 768 would be 1 / sqrt(768)
+    for ours, r in ((y, fwd), (xd.grad, ref)):
+        d = (ours.detach().double().cpu() - r.double()).norm(dim=-1)
+        assert bool((d <= 2.0 ** -6 * r.double().norm(dim=-1)).all())
