@@ -8,9 +8,10 @@ from uttt_amd import fast_weight_write as fww
 pytestmark = pytest.mark.gpu
 
 
-# one vector, a partial and a whole workgroup tile of 4096, one vector past it,
+# one vector, around half a workgroup tile of 4096 (below it the scalar kernel), a
+# whole tile, one vector past it,
 # several tiles, and counts that are no whole vectors
-@pytest.mark.parametrize("n", [4, 1020, 4096, 4100, 3 * 4096 + 12, 1, 4099])
+@pytest.mark.parametrize("n", [4, 2044, 2048, 2052, 4096, 4100, 3 * 4096 + 12, 1, 4099])
 @pytest.mark.parametrize("B", [1, 3])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("offset", [0, 1])

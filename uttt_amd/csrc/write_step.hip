@@ -404,10 +404,11 @@ extern "C" int uttt_momentum_add(const void* raw, int raw_dtype, const float* mo
   const int64_t blocks = (total + 255) / 256;
   UTTT_REQUIRE(blocks <= 0x7fffffffLL, "momentum_add: too many elements for one launch");
   hipStream_t st = as_stream(stream);
-  // whole, aligned vectors in every batch: 16-byte accesses (113 -> 68 us at 42.5 M
-  // elements); anything else an element per thread
+  // whole, aligned vectors in every batch, at least half a workgroup's: 16-byte
+  // accesses (113 -> 68 us at 42.5 M elements); anything else an element per thread
+  // (65 535 batches of 64: 11 us, in mostly idle workgroups of their own 60)
   const int64_t tiles = (per_batch + kMomTile - 1) / kMomTile;
-  if (per_batch % 4 == 0 && B <= 65535 && tiles < (1 << 24) && aligned(mom, 16) &&
+  if (per_batch % 4 == 0 && per_batch >= kMomTile / 2 && B <= 65535 && tiles < (1 << 24) && aligned(mom, 16) &&
       aligned(out, 16) && aligned(raw, dtype_bytes(raw_dtype) * 4)) {
     UTTT_DTYPE_SWITCH_LR(raw_dtype, TT, {
       hipLaunchKernelGGL((momentum_add4_kernel<TT>), dim3((unsigned)tiles, B), dim3(256), 0, st,
