@@ -1683,23 +1683,23 @@ template <class F>
 void grp_dispatch(int H, int T, int B, F&& f) {
   const int g = grp_lanes(H), ni = (H / 8 + g - 1) / g;
   const bool many = (int64_t)B * ((T + 63) / 64) >= 512;
-  auto with = [&](auto G) {
-    auto tok = [&](auto NI) {
-      if (many) f(G, NI, std::integral_constant<int, 64>{});
-      else f(G, NI, std::integral_constant<int, 16>{});
-    };
-    switch (ni) {
-      case 1: tok(std::integral_constant<int, 1>{}); break;
-      case 2: tok(std::integral_constant<int, 2>{}); break;
-      case 3: tok(std::integral_constant<int, 3>{}); break;
-      default: tok(std::integral_constant<int, 4>{}); break;
-    }
+  auto tok = [&](auto G, auto NI) {
+    if (many) f(G, NI, std::integral_constant<int, 64>{});
+    else f(G, NI, std::integral_constant<int, 16>{});
+  };
+  auto wide = [&](auto G) {  // grp_lanes takes more than 8 lanes for three or four chunks each
+    if (ni <= 3) tok(G, std::integral_constant<int, 3>{});
+    else tok(G, std::integral_constant<int, 4>{});
   };
   switch (g) {
-    case 8: with(std::integral_constant<int, 8>{}); break;
-    case 16: with(std::integral_constant<int, 16>{}); break;
-    case 32: with(std::integral_constant<int, 32>{}); break;
-    default: with(std::integral_constant<int, 64>{}); break;
+    case 8:
+      if (ni <= 1) tok(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
+      else if (ni <= 2) tok(std::integral_constant<int, 8>{}, std::integral_constant<int, 2>{});
+      else wide(std::integral_constant<int, 8>{});
+      break;
+    case 16: wide(std::integral_constant<int, 16>{}); break;
+    case 32: wide(std::integral_constant<int, 32>{}); break;
+    default: wide(std::integral_constant<int, 64>{}); break;
   }
 }
 // The launch of grouped-lane kernel K<types..., G, NI, TOK> over T tokens per batch.
