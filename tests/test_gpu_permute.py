@@ -297,9 +297,15 @@ def test_row_map_from_64_token_tiles(T, E, form):
     assert torch.equal(gs.cpu(), mask.sum(-1).to(torch.int32))
 
 
-@pytest.mark.parametrize("H", [8, 24, 192, 200, 384, 520, 768, 2048, 2056])
-@pytest.mark.parametrize("B,T,E,k", [(1, 1, 1, 1), (2, 65, 128, 4), (1, 700, 16, 2)])
-def test_grouped_lane_kernels_of_16_bit_rows(H, B, T, E, k):
+LANE_SIZES = [(B, T, E, k, H) for H in (8, 24, 192, 200, 384, 520, 768, 2048, 2056)
+              for B, T, E, k in ((1, 1, 1, 1), (2, 65, 128, 4), (1, 700, 16, 2))] + [
+    # token counts past which the lane groups take narrow rows, more slots and wide rows
+    (1, 2049, 16, 2, 24), (2, 1030, 16, 2, 1024), (1, 4100, 48, 4, 264), (1, 8200, 9, 3, 136),
+    (1, 16400, 9, 2, 1536), (1, 32775, 6, 2, 1032)]
+
+
+@pytest.mark.parametrize("B,T,E,k,H", LANE_SIZES)
+def test_grouped_lane_kernels_of_16_bit_rows(B, T, E, k, H):
     """The 16-bit backward kernels and the k / v / lr permute at the edges of
     their lane groups (and past them: H = 2056), tokens with none to k + 1
     experts, gates of zero, rows past num_out.  k / v / lr outputs bit-exact.

@@ -1307,7 +1307,8 @@ int pick_ve(int H, std::initializer_list<const void*> ptrs) {
 // forward 127 -> 62; unpermute / permute backward of 65 536 x 768, top-2 116 -> 85
 // and 89 -> 55 us (with non-temporal stores 100 and 63, with plain loads 101 and
 // 72).  For 16-bit payloads of 16-byte rows (H a multiple of 8, H <= 2048, aligned
-// pointers), E <= 128 and num_out >= 1; the kernels above take the rest.
+// pointers), E <= 128 and num_out >= 1, where they gain (grp_pays); the kernels above
+// take the rest.
 // Workgroups of TOK tokens (64, or 16 where those would leave CUs idle) and at
 // most 512 threads.
 constexpr int grp_threads(int g, int tok) { return g * tok < 512 ? g * tok : 512; }
@@ -1672,10 +1673,31 @@ inline int grp_lanes(int H) {
   while (g < 64 && 4 * g < CH) g *= 2;
   return g;
 }
+// Where the lane groups measure faster, from 3565 timings (H 8 to 2048, 8 to 65 536
+// tokens, 1 to 8 slots).  A row past 1024 fills a wave by itself, so that only
+// many tokens gain; few tokens are latency, a wave each; without prob gradients
+// the permute's backward has no scattered stores to save; from the third slot on
+// the slots' rows are read one after the other (1000 tokens of 1536 with 8: k / v
+// permute 17.7 / 28.7 us, permute backward 17.3 / 26.9).  Six timings within these
+// lines are still over 6 % slower, by up to 1.17.
+enum GrpKind { kGrpPermuteBwd, kGrpPermuteBwdNoProbs, kGrpUnpermuteBwd, kGrpKvFwd, kGrpKvBwd };
+bool grp_pays(GrpKind kind, int H, int B, int T, int num_out) {
+  const int64_t tokens = (int64_t)B * T;
+  const bool few_slots = num_out <= 2 * (int64_t)T;
+  switch (kind) {
+    case kGrpPermuteBwd: return H <= 1024 ? tokens > (few_slots ? 2048 : 4096) : tokens >= 32768;
+    case kGrpPermuteBwdNoProbs: return H <= 256 && tokens > (few_slots ? 2048 : 8192);
+    case kGrpUnpermuteBwd: return H <= 1024 || tokens >= 16384;
+    case kGrpKvFwd: return H <= 1024 ? few_slots || tokens > 4096 : tokens >= 16384;
+    case kGrpKvBwd: return H <= 1024 || tokens > 2048;
+  }
+  return false;
+}
 template <class TT>
-bool grp_fits(int H, int E, int num_out, std::initializer_list<const void*> ptrs) {
+bool grp_fits(GrpKind kind, int H, int B, int T, int E, int num_out,
+              std::initializer_list<const void*> ptrs) {
   if (sizeof(typename TT::S) != 2 || H < 8 || H > 2048 || E > 128 || num_out < 1) return false;
-  return pick_ve<TT>(H, ptrs) == 8;
+  return grp_pays(kind, H, B, T, num_out) && pick_ve<TT>(H, ptrs) == 8;
 }
 // f(G, NI, TOK) with compile-time lanes per token, chunks per lane and tokens
 // per workgroup
@@ -1952,7 +1974,8 @@ extern "C" int uttt_permute_bwd(const void* grad_out, int dtype, int B, int T, i
   UTTT_DTYPE_SWITCH(dtype, TT, {
     using S = typename TT::S;
     if constexpr (sizeof(S) == 2) {
-      if (grp_fits<TT>(H, E, num_out, {grad_out, grad_inp})) {
+      if (grp_fits<TT>(grad_probs ? kGrpPermuteBwd : kGrpPermuteBwdNoProbs, H, B, T, E, num_out,
+                       {grad_out, grad_inp})) {
         UTTT_GRP_LAUNCH(E, hipLaunchKernelGGL((permute_bwd_grp_kernel<TT, G, NI, TOK>), grid, block, lds, st,
                              reinterpret_cast<const S*>(grad_out), H, T, row_id_map, E, num_out,
                              grad_permuted_probs, reinterpret_cast<S*>(grad_inp), grad_probs));
@@ -2010,7 +2033,7 @@ extern "C" int uttt_unpermute_bwd(const void* grad_out, const void* fwd_inp, int
   UTTT_DTYPE_SWITCH(dtype, TT, {
     using S = typename TT::S;
     if constexpr (sizeof(S) == 2) {
-      if (grp_fits<TT>(H, E, num_out, {grad_out, fwd_inp, grad_inp})) {
+      if (grp_fits<TT>(kGrpUnpermuteBwd, H, B, T, E, num_out, {grad_out, fwd_inp, grad_inp})) {
         UTTT_GRP_LAUNCH(E, hipLaunchKernelGGL((unpermute_bwd_grp_kernel<TT, G, NI, TOK>), grid, block, lds, st,
                              reinterpret_cast<const S*>(grad_out),
                              reinterpret_cast<const S*>(fwd_inp), H, T, row_id_map, E, num_out,
@@ -2039,7 +2062,7 @@ int launch_permute_kv_fwd(const void* k, const void* v, const void* lr0, const v
                           int64_t p_se, int64_t p_st, void* k_out, void* v_out, void* lr0_out,
                           void* lr1_out, void* lr2_out, int num_out, hipStream_t st) {
   if constexpr (sizeof(typename KT::S) == 2 && sizeof(typename VT::S) == 2) {
-    if (grp_fits<KT>(H, 1, num_out, {k, v, k_out, v_out})) {
+    if (grp_fits<KT>(kGrpKvFwd, H, B, T, 1, num_out, {k, v, k_out, v_out})) {
       UTTT_GRP_LAUNCH(0, hipLaunchKernelGGL((permute_kv_fwd_grp_kernel<KT, VT, G, NI, TOK>), grid, block, lds, st,
                            reinterpret_cast<const uint16_t*>(k), reinterpret_cast<const uint16_t*>(v),
                            reinterpret_cast<const uint8_t*>(lr0), reinterpret_cast<const uint8_t*>(lr1),
@@ -2077,7 +2100,7 @@ int launch_permute_kv_bwd(const void* gk, const void* gv, const void* glr0, cons
                           void* grad_v, void* grad_lr0, void* grad_lr1, void* grad_lr2,
                           float* grad_probs, hipStream_t st) {
   if constexpr (sizeof(typename KT::S) == 2 && sizeof(typename VT::S) == 2) {
-    if (grp_fits<KT>(H, E, num_out, {gk, gv, grad_k, v, grad_v})) {
+    if (grp_fits<KT>(kGrpKvBwd, H, B, T, E, num_out, {gk, gv, grad_k, v, grad_v})) {
       using SL = typename LT::S;
       UTTT_GRP_LAUNCH(E, hipLaunchKernelGGL((permute_kv_bwd_grp_kernel<KT, VT, LT, G, NI, TOK>), grid, block, lds, st,
                            reinterpret_cast<const uint16_t*>(gk), reinterpret_cast<const uint16_t*>(gv),
