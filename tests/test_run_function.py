@@ -48,14 +48,20 @@ def test_routes():
         assert _run(x)[1] == "_NoGraph"
 
 
-def test_an_input_handed_through_is_an_alias():
-    """As apply returns it: other metadata, the same storage."""
-    x, n = torch.randn(3), torch.zeros(1, dtype=torch.int32)
-    with torch.no_grad():
-        for out in (_Double.apply(x, n)[1], run_function(_Double, x, n)[1]):
-            assert out is not n and out.data_ptr() == n.data_ptr() and out._is_view()
-            out.unsqueeze_(0)
-            assert n.shape == (1,)
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_given_row_map_comes_out_as_an_alias(grad, monkeypatch):
+    """As Function.apply returns it: metadata of its own, the same storage."""
+    from uttt_amd.lact_moe_triton import triton_permute as tp
+
+    monkeypatch.setattr(tp, "triton_permute_with_mask_map",
+                        lambda x, *a: (x.repeat(1, 2, 1), None))
+    x, mask = torch.randn(1, 4, 8, requires_grad=True), torch.ones(1, 2, 4, dtype=torch.bool)
+    rm = torch.zeros(1, 4, 5, dtype=torch.int32)
+    with torch.set_grad_enabled(grad):
+        out = tp.permute_with_expert_mask(x, mask, None, 2, rm)[2]
+    assert out is not rm and out.data_ptr() == rm.data_ptr()
+    out.unsqueeze_(0)
+    assert rm.shape == (1, 4, 5)
 
 
 class _Address(torch.autograd.Function):

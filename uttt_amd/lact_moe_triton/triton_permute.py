@@ -338,7 +338,11 @@ def permute_with_expert_mask(
     row_id_map: torch.Tensor = None,
 ):
     """(out [B, topk*T, H], permuted_probs [B, topk*T] or None, row_id_map) (P:1241-1248)."""
-    return run_function(PermuteWithMaskMap, inp, expert_mask, probs, topk, row_id_map)
+    out, permuted_probs, row_map = run_function(PermuteWithMaskMap, inp, expert_mask, probs, topk,
+                                                row_id_map)
+    if row_map is row_id_map:  # a given map comes out as an alias, with or without gradients
+        row_map = row_map.view_as(row_map)
+    return out, permuted_probs, row_map
 
 
 class UnPermuteWithMaskMap(torch.autograd.Function):
