@@ -40,7 +40,7 @@ from ._ops import run_function
 from .lact_moe_triton import _grouped
 from .lact_moe_triton.lact_fw_grad import grouped_lact_swiglu_ffn_fast_weight_grads
 from .lact_moe_triton.lact_swiglu_ffn import grouped_swiglu_ffn_fwd
-from .lact_moe_triton.triton_permute import (permute_kv_and_lrs, permute_with_expert_mask,
+from .lact_moe_triton.triton_permute import (permute_kv_and_lrs, permute_rows,
                                              unpermute_and_merge_with_probs)
 from .routing import route_tokens, route_tokens_map, src_rows_supported
 
@@ -147,7 +147,7 @@ def apply_moe_fast_weights_grouped(x, w0, w1, w2, router_proj_weights, cfg: Rout
                                          routed[6], group_sizes)
         y_perm = _grouped.gemm_nt(w1c, hidden, group_sizes)
     else:
-        x_perm, _, row_id_map = permute_with_expert_mask(
+        x_perm, _, row_id_map = permute_rows(
             xt.to(w0_w2.dtype).contiguous(), expert_mask, router_probs, cfg.topk, row_id_map)
         y_perm = grouped_swiglu_ffn_fwd(w0_w2, w1.contiguous(), x_perm, group_sizes)
     out = unpermute_and_merge_with_probs(y_perm, row_id_map, router_probs)
