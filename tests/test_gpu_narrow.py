@@ -149,3 +149,51 @@ def test_super_tiles_of_192_equal_general_tiles(M, K, sizes):
         general = products()
     for a, b in zip(ours, general):
         assert torch.equal(a, b)
+
+
+def _same(a, b):
+    return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("D,I", [(192, 192), (200, 104), (512, 512)])
+def test_infinities_and_nan_stay_with_their_tokens_and_experts(D, I):
+    """An infinity in one token's rows, at the end of its expert's segment (the
+    row that partial tiles repeat), and a NaN in another expert's weights: what
+    has no part in them keeps its bits, the rest is the general tiles'."""
+    sizes = [130, 65, 200, 31]
+    gs = torch.tensor([sizes], dtype=torch.int32, device=DEV)
+    E, N = len(sizes), sum(sizes)
+    g = torch.Generator().manual_seed(D)
+    rnd = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).to(torch.bfloat16).to(DEV)
+    W02, gW02 = (rnd(1, E, 2 * I, D, scale=D ** -0.5) for _ in range(2))
+    W1, gW1 = (rnd(1, E, D, I, scale=I ** -0.5) for _ in range(2))
+    K, V, H, Y = rnd(1, N, D), rnd(1, N, D), rnd(1, N, I), rnd(1, N, 2 * I)
+    lrs = [torch.rand(1, N, generator=g).to(DEV) for _ in range(3)]
+
+    def run():
+        s1 = G.update_stage1(W02, W1, K, V, *lrs, gs, True, save=True)
+        bwd = UB._backward(W02, W1, K, V, *lrs, gs, gW02, gW1, *s1[2:])
+        tok = [G.gate_up(W02, K, gs, token_major=True), G.gemm_nt(W1, H, gs), G.gemm_tn(W02, Y, gs),
+               *s1, *bwd[2:]]
+        return tok, [*G.wgrad_pair(Y, K, H, V, gs), *bwd[:2]]
+
+    clean = run()
+    bad_tok, bad_e = sizes[0] + sizes[1] - 1, 2
+    for t in (K, V, H, Y):
+        t[0, bad_tok] = float("inf")
+    W02[0, bad_e, 5, 7] = W1[0, bad_e, 3, 2] = float("nan")
+    ours = run()
+    with general_tiles():
+        general = run()
+    e_of = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes)).to(DEV)
+    ok_rows = (e_of != bad_e) & (torch.arange(N, device=DEV) != bad_tok)
+    for a, c in zip(ours[0], clean[0], strict=True):
+        assert torch.equal(a[0, ok_rows], c[0, ok_rows])
+    for a, b in zip(ours[0][:7], general[0][:7]):     # all but the backward: bit for bit
+        assert _same(a, b)
+    for a, b in zip(ours[0][7:], general[0][7:]):
+        assert torch.equal(a.isfinite(), b.isfinite())
+    clean_e = [0, 3]
+    for a, c, b in zip(ours[1], clean[1], general[1], strict=True):
+        assert torch.equal(a[0, clean_e], c[0, clean_e])
+        assert torch.equal(a.isfinite(), b.isfinite())

@@ -367,3 +367,45 @@ def test_grouped_lane_kernels_of_16_bit_rows(B, T, E, k, H):
     ref = torch.zeros(B, E, T)
     ref[b_, e_, t_] = gpp[b_, r_]
     assert torch.equal(gp.cpu(), ref)
+
+
+@pytest.mark.parametrize("H", [24, 384])
+def test_grouped_lane_kernels_keep_infinities_apart(H):
+    """An infinity or NaN in one row reaches its token's sums and its own prob
+    gradient only, also in the chunks that lanes past the row repeat."""
+    B, T, E, k = 1, 2100, 16, 2
+    g = torch.Generator().manual_seed(H)
+    mask = torch.rand(B, E, T, generator=g).argsort(1).argsort(1) < k
+    probs = (torch.rand(B, E, T, generator=g) * mask).to(DEV)
+    rm = TP.make_row_id_map(mask.to(DEV), B, T, E)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    x, v, go, y, gk, gv = bf(B, T, H), bf(B, T, H), bf(B, T, H), bf(B, k * T, H), bf(B, k * T, H), bf(B, k * T, H)
+    lr = [torch.rand(B, T, generator=g).to(DEV) for _ in range(3)]
+    gl = [torch.rand(B, k * T, generator=g).to(DEV) for _ in range(3)]
+    gpp = torch.rand(B, k * T, generator=g).to(DEV)
+
+    def run():
+        kv = TP._kv_fwd(x, v, *lr, rm, probs, k * T)
+        kvb = TP._kv_bwd(gk, gv, *gl, v, probs, rm, T)
+        pb = TP._permute_bwd(gk, rm, gpp, B, T, E, H)
+        ub = TP._unpermute_bwd(go, rm, y, probs, B, T, E, k * T, H)
+        return [kvb[0], kvb[1], pb[0]], [kvb[5], pb[1], ub[1]], [kv[0], kv[1], ub[0]]
+
+    clean = run()
+    t = T - 1
+    rows = rm[0, t, :k].long()
+    for a in (x, v, go):
+        a[0, t, H - 1] = float("inf")
+    for a in (y, gk, gv):
+        a[0, rows[1], H - 1] = float("nan")
+    bad = run()
+    tok = torch.arange(T, device=DEV) != t
+    out = torch.ones(k * T, dtype=torch.bool, device=DEV)
+    out[rows] = False
+    for a, c in zip(bad[0], clean[0]):
+        assert torch.equal(a[0, tok], c[0, tok]) and bool(a[0, t, H - 1].isnan())
+        assert bool(a[0, t, : H - 1].isfinite().all())
+    for a, c in zip(bad[1], clean[1]):
+        assert torch.equal(a[0, :, tok], c[0, :, tok])
+    for a, c in zip(bad[2], clean[2]):
+        assert torch.equal(a[0, out], c[0, out])

@@ -301,3 +301,22 @@ def test_route_tokens_map_from_the_selection_counts(B, T, D, E, k):
     torch.testing.assert_close(bsum.cpu(), bal.cpu().double().sum(-1).float(), rtol=1e-5, atol=1e-5)
     m2, gs2, comb2, bal2 = RT.route_tokens(x, Rw, k, combine_mode="topk_renorm")
     assert torch.equal(mask, m2) and torch.equal(gs, gs2) and torch.equal(comb, comb2)
+
+
+def test_route_tokens_wide_infinities_and_nan():
+    """All scores -inf: the first k experts, as with equal scores.  A NaN token
+    leaves the others' masks, gates and balances alone."""
+    B, T, D, E, k = 1, 200, 192, 48, 2
+    g = torch.Generator().manual_seed(4)
+    x = torch.randn(B, T, D, generator=g).to(torch.bfloat16).to(DEV)
+    Rw = torch.randn(E, D, generator=g).to(DEV)
+    bias = torch.full((1, E, 1), -float("inf"), device=DEV)
+    mask = RT.route_tokens(x, Rw, k, routing_bias=bias)[0]
+    assert bool(mask[:, :k].all()) and int(mask.sum()) == B * T * k
+    clean = RT.route_tokens(x, Rw, k)
+    x[0, 77] = float("nan")
+    bad = RT.route_tokens(x, Rw, k)
+    rest = torch.arange(T, device=DEV) != 77
+    for a, c in zip((bad[0], bad[2], bad[3]), (clean[0], clean[2], clean[3])):
+        assert torch.equal(a[..., rest], c[..., rest])
+    assert bool(bad[3][..., 77].isnan().all())
