@@ -1683,7 +1683,7 @@ Wg192Plan wgrad_plan(int B, int E, int I, int D, int N) {
 // 256 x 256, over 196 608 (792 / 1048) 127 -> 107; 8 of 512 x 256 over 16 384 30.7 / 38.
 // Row-major weights of segments of at most 32 tokens: the 256-tile kernel skips
 // the products of absent tokens (4 of 4096 x 288 over 32 104 / 146 us).  Of 16 000
-// timings (1 to 96 experts, widths 64 to 6144, 32 to 196 608 tokens) 55 on these
+// timings (1 to 96 experts, widths 64 to 6144, 32 to 196 608 tokens) about 70 on these
 // tiles are over 6 % slower than on the others, against 2571 by widths alone.
 bool use_tn192(bool a_kmajor, int M, int K, int N, int B, int E) {
   if (general_forced() || K <= 0) return false;
@@ -1697,7 +1697,11 @@ bool use_tn192(bool a_kmajor, int M, int K, int N, int B, int E) {
   };
   const int64_t t256 = tiles(256), t192 = tiles(192);
   const int64_t rounds256 = (t256 + 255) / 256, rounds192 = (t192 + 511) / 512;
-  return t192 <= 256 || 9 * rounds192 <= 8 * rounds256;
+  // 256-token tiles expected to just fill one round, of segments shorter than a
+  // tile, often take a second: 96 experts of 384 x 384 over 16 384 tokens (224 / 268),
+  // grad_K even 43.8 -> 38.6 us, of three routings 80 -> 54, 78 -> 53 and 50 / 52
+  const bool near_full = narrow && N < 256 * (int64_t)E && t256 > 216 && t192 <= 320;
+  return t192 <= 256 || near_full || 9 * rounds192 <= 8 * rounds256;
 }
 
 // Wide single product: y[b, n, m] = sum_k A(m, k) x[b, n, k] with M rows in
