@@ -264,16 +264,17 @@ def test_routed_read_without_gradient_equals_the_permuted_path():
         assert torch.equal(lb[1], lb2[1])
 
 
-@pytest.mark.parametrize("D,rope_dim", [(8, 0), (64, 64), (192, 64), (256, 256), (384, 128), (520, 0),
-                                        (768, 16), (1032, 0), (1536, 64), (2048, 256), (4096, 32)])
+ROW_WIDTHS = [(8, 0), (64, 64), (192, 64), (256, 256), (384, 128), (520, 0), (768, 16), (1032, 0),
+              (1536, 64), (2048, 256), (4096, 32)]
+
+
+@pytest.mark.parametrize("D,rope_dim,Lx", [(*w, 37) for w in ROW_WIDTHS] +
+                         [(*w, 4101) for w in ROW_WIDTHS if w[0] <= 768])  # wider: 64 lanes either way
 @pytest.mark.parametrize("norm", [None, "l2", "rms"])
-@pytest.mark.parametrize("Lx", [37, 4101])
 def test_rows_preprocess_row_widths(D, rope_dim, norm, Lx):
     """Every lane-group width and chunk count of the row kernels (few rows take
     more lanes), a row count that does not fill the last workgroup, forward and
     backward."""
-    if Lx > 37 and D > 768:
-        pytest.skip("64 lanes per row at either count")
     B = 1
     g = torch.Generator().manual_seed(D)
     x = torch.randn(B, Lx, D, generator=g).to(torch.bfloat16)

@@ -35,9 +35,9 @@ COMMON_FLAGS = [
 
 
 # Sources whose kernels must not use scratch memory: the grouped GEMMs, the
-# 192-tile products and the staged uTTT-Dense stage 1 issue their LDS fragment reads as inline asm with
-# explicit waits, so a register spill between a read and its wait would save
-# the value from before the read;
+# 192-tile and narrow-expert products and the staged uTTT-Dense stage 1 issue
+# their LDS fragment reads as inline asm with explicit waits, so a register
+# spill between a read and its wait would save the value from before the read;
 # the one-launch Newton-Schulz holds its accumulators and the products it
 # writes back across barriers, where a spill would cost more than the work.
 NO_SCRATCH = {"grouped_gemm.hip", "tile192.hip", "narrow.hip", "ns_small.hip", "dense_update.hip"}

@@ -264,7 +264,7 @@ __global__ __launch_bounds__(kTThreads, 2) void tn192_kernel(Tn192Args s) {
 
 // ========================================================= Newton-Schulz ==
 // The three products of a step over BE matrices, with the rounding of the
-// reference's bf16 tensor arithmetic (grouped_gemm.hip's EpiLinComb):
+// reference's bf16 tensor arithmetic, a rounding after every operation:
 //   kNsA  A = bf16(X X^T).  Symmetric bit for bit: only the tiles on or below
 //         the diagonal run, and one below it also stores its transpose.
 //   kNsB  B = bf16(bf16(b A) + bf16((c A) A)): A's rows are both operands, the
