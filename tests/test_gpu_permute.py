@@ -301,7 +301,10 @@ LANE_SIZES = [(B, T, E, k, H) for H in (8, 24, 192, 200, 384, 520, 768, 2048, 20
               for B, T, E, k in ((1, 1, 1, 1), (2, 65, 128, 4), (1, 700, 16, 2))] + [
     # token counts past which the lane groups take narrow rows, more slots and wide rows
     (1, 2049, 16, 2, 24), (2, 1030, 16, 2, 1024), (1, 4100, 48, 4, 264), (1, 8200, 9, 3, 136),
-    (1, 16400, 9, 2, 1536), (1, 32775, 6, 2, 1032)]
+    (1, 16400, 9, 2, 1536), (1, 32775, 6, 2, 1032),
+    # many short batches: waves past the end, full and nearly full 64s, 17 to 19 tokens
+    (600, 9, 8, 6, 192), (300, 17, 6, 4, 520), (300, 17, 6, 4, 264), (300, 20, 6, 4, 1024),
+    (512, 60, 8, 3, 24), (514, 51, 3, 3, 136)]
 
 
 @pytest.mark.parametrize("B,T,E,k,H", LANE_SIZES)

@@ -1320,6 +1320,12 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// Whether this wave's first token (this lane's is t) is past the end: no lane has work.
+template <int G>
+__device__ __forceinline__ bool wave_past(int t, int T) {
+  return t - (int)(threadIdx.x % kWave) / G >= T;
+}
+
 // A token's first two slots (the rest is read when used), from its row of the
 // map; rows outside [0, num_out) count as absent but keep their slot.
 struct GrpSlots {
@@ -1408,6 +1414,7 @@ __global__ __launch_bounds__(grp_threads(G, TOK)) void permute_bwd_grp_kernel(
   const uint16_t* gb = gout + (int64_t)b * num_out * H;
   for (int tl = threadIdx.x / G; tl < TOK; tl += kThr / G) {
     const int t = t0 + tl;
+    if (wave_past<G>(t, T)) break;
     const int64_t bt = (int64_t)b * T + min(t, T - 1);
     const int32_t* rm = rmap + bt * (2 * E + 1);
     GrpSlots s;
@@ -1465,6 +1472,7 @@ __global__ __launch_bounds__(grp_threads(G, TOK)) void unpermute_bwd_grp_kernel(
   uint16_t* gb = ginp + (int64_t)b * num_out * H;
   for (int tl = threadIdx.x / G; tl < TOK; tl += kThr / G) {
     const int t = t0 + tl;
+    if (wave_past<G>(t, T)) break;
     const int tc = min(t, T - 1);
     const int64_t bt = (int64_t)b * T + tc;
     const int32_t* rm = rmap + bt * (2 * E + 1);
@@ -1532,6 +1540,7 @@ __global__ __launch_bounds__(grp_threads(G, TOK)) void permute_kv_fwd_grp_kernel
   const int cl = threadIdx.x % G, CH = H / 8;
   for (int tl = threadIdx.x / G; tl < TOK; tl += kThr / G) {
     const int t = t0 + tl;
+    if (wave_past<G>(t, T)) break;
     const int tc = min(t, T - 1);
     const int64_t bt = (int64_t)b * T + tc;
     const int32_t* rm = rmap + bt * (2 * E + 1);
@@ -1604,6 +1613,7 @@ __global__ __launch_bounds__(grp_threads(G, TOK)) void permute_kv_bwd_grp_kernel
   SL* go = (cl == 0 ? grad_lr0 : cl == 1 ? grad_lr1 : grad_lr2);
   for (int tl = threadIdx.x / G; tl < TOK; tl += kThr / G) {
     const int t = t0 + tl;
+    if (wave_past<G>(t, T)) break;
     const int tc = min(t, T - 1);
     const int64_t bt = (int64_t)b * T + tc;
     const int32_t* rm = rmap + bt * (2 * E + 1);
@@ -1678,12 +1688,16 @@ inline int grp_lanes(int H) {
 // many tokens gain; few tokens are latency, a wave each; without prob gradients
 // the permute's backward has no scattered stores to save; from the third slot on
 // the slots' rows are read one after the other (1000 tokens of 1536 with 8: k / v
-// permute 17.7 / 28.7 us, permute backward 17.3 / 26.9).  Six timings within these
-// lines are still over 6 % slower, by up to 1.17.
+// permute 17.7 / 28.7 us, permute backward 17.3 / 26.9).  Many batches of 17 to 19
+// tokens leave most of each one's second 16 absent (300 of 17 x 1024, top-2: permute
+// backward 8.0 / 10.7 us, k / v permute 13.9 / 18.9).  Six of the timings within these
+// lines are over 6 % slower, by up to 1.17, and of 760 more, batches of 9 to 100
+// tokens, 22, by up to 1.2 (2048 batches of 20 x 1024, top-2).
 enum GrpKind { kGrpPermuteBwd, kGrpPermuteBwdNoProbs, kGrpUnpermuteBwd, kGrpKvFwd, kGrpKvBwd };
 bool grp_pays(GrpKind kind, int H, int B, int T, int num_out) {
   const int64_t tokens = (int64_t)B * T;
   const bool few_slots = num_out <= 2 * (int64_t)T;
+  if (H >= 384 && T > 16 && T < 20 && tokens > 2048) return false;
   switch (kind) {
     case kGrpPermuteBwd: return H <= 1024 ? tokens > (few_slots ? 2048 : 4096) : tokens >= 32768;
     case kGrpPermuteBwdNoProbs: return H <= 256 && tokens > (few_slots ? 2048 : 8192);
@@ -1704,7 +1718,10 @@ bool grp_fits(GrpKind kind, int H, int B, int T, int E, int num_out,
 template <class F>
 void grp_dispatch(int H, int T, int B, F&& f) {
   const int g = grp_lanes(H), ni = (H / 8 + g - 1) / g;
-  const bool many = (int64_t)B * ((T + 63) / 64) >= 512;
+  // not where the last (or only) 64 tokens of a batch would be mostly absent (512
+  // batches of 65 tokens of 1024: permute backward 37 / 57 us)
+  const int blocks = (T + 63) / 64;
+  const bool many = (int64_t)B * blocks >= 512 && 4 * (int64_t)blocks * 64 <= 5 * (int64_t)T;
   auto tok = [&](auto G, auto NI) {
     if (many) f(G, NI, std::integral_constant<int, 64>{});
     else f(G, NI, std::integral_constant<int, 16>{});
