@@ -28,6 +28,9 @@ CASES = {
     "slack_rows": ([[60, 40]], 384, 384, 160),
     "over_count": ([[60, 90, 70]], 96, 200, 140),
     "all_empty": ([[0, 0, 0]], 192, 64, 32),
+    # from the tokens where the widest backward takes the general tiles, and one less
+    "widest_many_tokens": ([[49111, 41]], 448, 512, None),
+    "widest_one_token_less": ([[49110, 41]], 448, 512, None),
     "short_segments_wide": ([[200, 0, 193, 1, 300, 192]], 520, 776, None),
 }
 

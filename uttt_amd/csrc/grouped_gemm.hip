@@ -2197,7 +2197,7 @@ extern "C" int uttt_grouped_update_bwd(
   const int64_t g02 = (int64_t)2 * I * D, g1 = (int64_t)D * I;
   const int m_tiles = (I + kTileRows - 1) / kTileRows;
 
-  if (y0_y2_saved != nullptr && narrow_experts(I, D) && !general_forced()) {
+  if (y0_y2_saved != nullptr && narrow_bwd(I, D, N, B) && !general_forced()) {
     if (int rc = launch_narrow_bwd(grad_dw0_w2, grad_dw1, k, v, lr0, lr1, lr2, lr_dtype, group_sizes,
                                    B, E, I, D, N, y0_y2_saved, dh_saved, gdh, gx, dx, hlr, part, st,
                                    "grouped_update_bwd(second order)"))

@@ -18,6 +18,12 @@ bool narrow_experts(int I, int D);
 // 6 % slower than the two launches, and of as many gate/up ones one (a few tokens
 // per expert, 9.6 / 10.5 us).
 bool narrow_stage1(int I, int D, int N, int B, int E);
+// Whose backward it takes: those widths, but not many tokens of experts that fill
+// both of the general tiles' 256s, which reuse a token's row for twice the units
+// (timings of 7 widths from 384 x 512; 16 experts of 480 x 512 over 131 072 tokens:
+// 1288 / 1167 us here / there; 448 x 512 over 65 536 alike; 512 x 384 over 196 608
+// 1604 / 1631; 512 x 512 over 16 384: 208 / 219).
+bool narrow_bwd(int I, int D, int N, int B);
 // Row blocks of its lr-gradient partials, lr_part[3][narrow_m_tiles][B][N].
 int narrow_m_tiles(int I);
 

@@ -20,9 +20,10 @@
 //   backward's second pass  302 us (two launches) -> 223 (830 MB, 3.7 TB/s)
 // 96 of 384 x 384 over 16 384 tokens, without saves: 89 -> 45 us; gate/up 42 ->
 // 31, of 48 x 192 x 192 17 -> 10.7 (against apply_kernel's 256 x 128 tiles).
-// Every I, D up to 512 measured gains (narrow_stage1's comment); past it long
-// segments were not timed, and a token tile is read by more than eight unit
-// groups: the 256-token tiles' kernels.
+// Stage 1 of every I, D up to 512 measured gains, the backward but for the widest
+// of many tokens (narrow_stage1, narrow_bwd); past 512 long segments were not
+// timed, and a token tile is read by more than eight unit groups: the 256-token
+// tiles' kernels.
 #include "narrow.h"
 #include "tile192.h"
 
@@ -576,6 +577,9 @@ bool narrow_stage1(int I, int D, int N, int B, int E) {
   return narrow_experts(I, D) ||
          (D > kTK && (int64_t)I * D <= (int64_t)768 * 1536 &&
           (N <= 128 * (int64_t)E || (N <= 256 * (int64_t)E && weights <= (256 << 20))));
+}
+bool narrow_bwd(int I, int D, int N, int B) {
+  return narrow_experts(I, D) && !(I * D >= 448 * 512 && (int64_t)B * N >= 49152);
 }
 int narrow_m_tiles(int I) { return (I + kHid - 1) / kHid; }
 
