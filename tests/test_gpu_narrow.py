@@ -31,6 +31,9 @@ CASES = {
     # from the tokens where the widest backward takes the general tiles, and one less
     "widest_many_tokens": ([[49111, 41]], 448, 512, None),
     "widest_one_token_less": ([[49110, 41]], 448, 512, None),
+    # absent tiles between the batches': 256 tiles, and 192 where both may take a second round
+    "many_batches_256": ([[256, 0, 255, 300]] * 16, 256, 256, 1024),
+    "many_batches_192": ([[16, 0, 30, 18]] * 64, 192, 384, 64),
     "short_segments_wide": ([[200, 0, 193, 1, 300, 192]], 520, 776, None),
 }
 

@@ -1701,7 +1701,13 @@ bool use_tn192(bool a_kmajor, int M, int K, int N, int B, int E) {
   // tile, often take a second: 96 experts of 384 x 384 over 16 384 tokens (224 / 268),
   // grad_K even 43.8 -> 38.6 us, of three routings 80 -> 54, 78 -> 53 and 50 / 52
   const bool near_full = narrow && N < 256 * (int64_t)E && t256 > 216 && t192 <= 320;
-  return t192 <= 256 || near_full || 9 * rounds192 <= 8 * rounds256;
+  // Several batches' launches have their absent tiles between the others: where these
+  // may take a second tile of 192 to a CU but not one of 256, one each does not hold
+  // (16 batches of 4 experts of 384 x 384 over 1024 tokens, grad_V 25.8 / 35.7 us; 64 of
+  // 4 of 384 x 192 over 64, up to 320 of either: grad_K 74 -> 42)
+  const auto upto = [&](int t) { return (M + t - 1) / t * ((N + t - 1) / t + (int64_t)E) * B; };
+  const bool one_each = t192 <= 256 && (B == 1 || upto(192) <= 256 || upto(256) > 256);
+  return one_each || near_full || 9 * rounds192 <= 8 * rounds256;
 }
 
 // Wide single product: y[b, n, m] = sum_k A(m, k) x[b, n, k] with M rows in

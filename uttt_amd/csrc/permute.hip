@@ -1719,7 +1719,7 @@ template <class F>
 void grp_dispatch(int H, int T, int B, F&& f) {
   const int g = grp_lanes(H), ni = (H / 8 + g - 1) / g;
   // not where the last (or only) 64 tokens of a batch would be mostly absent (512
-  // batches of 65 tokens of 1024: permute backward 37 / 57 us)
+  // batches of 65 tokens of 1024, top-2: permute backward 38 / 57 us)
   const int blocks = (T + 63) / 64;
   const bool many = (int64_t)B * blocks >= 512 && 4 * (int64_t)blocks * 64 <= 5 * (int64_t)T;
   auto tok = [&](auto G, auto NI) {
