@@ -279,8 +279,11 @@ int uttt_grouped_gemm_nt(const void* w, const void* x, const int32_t* group_size
 int uttt_grouped_gemm_tn(const void* w, const void* x, const int32_t* group_sizes, int B, int E,
                          int M, int K, int N, void* y, void* stream);
 
-/* Scratch bytes for uttt_grouped_update_stage1 at (B, I, N). */
+/* Scratch bytes for uttt_grouped_update_stage1: enough at (B, I, N) for any
+ * experts, widths and layout, and exactly what one call uses, 0 where one kernel
+ * keeps DH in registers (token-major outputs of small experts). */
 size_t uttt_update_stage1_workspace_bytes(int B, int I, int N);
+size_t uttt_update_stage1_scratch_bytes(int B, int E, int I, int D, int N, int token_major);
 
 /* UPDATE, stage 1.  Replaces swiglu_backward_three_bmm_grouped_with_lr_triton
  * (L/triton_grouped_swiglu_bwd_with_lr_kernels.py:255-353; kernel :49-252).
@@ -296,7 +299,8 @@ size_t uttt_update_stage1_workspace_bytes(int B, int I, int N);
  * L/triton_grouped_swiglu_bwd_kernels.py:49-320, with v = grad_out).
  * y0_y2_save [B,N,2I] and dh_save [B,N,I] (optional, both or neither):
  * bf16(Y0 | Y2) and bf16(DH), token-major, for uttt_grouped_update_bwd.
- * workspace: uttt_update_stage1_workspace_bytes(B, I, N) bytes (DH). */
+ * workspace: uttt_update_stage1_scratch_bytes(...) bytes (DH) or more; may be
+ * NULL where that is 0. */
 int uttt_grouped_update_stage1(const void* w0_w2, const void* w1, const void* k, const void* v,
                                const void* lr0, const void* lr1, const void* lr2, int lr_dtype,
                                const int32_t* group_sizes, int B, int E, int I, int D, int N,

@@ -67,6 +67,25 @@ def test_wgrad_pair_split_rule():
 
 
 @pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
+def test_stage1_scratch_only_where_dh_goes_through_memory():
+    """The one-launch stage 1 uses no workspace: its query answers 0 there, and
+    the (B, I, N) bound for the reference layout, wide experts and forced
+    general tiles."""
+    lib = _lib.lib()
+    q, hook = lib.uttt_update_stage1_scratch_bytes, lib.uttt_debug_set_gemm_layout
+    full = lib.uttt_update_stage1_workspace_bytes(2, 192, 5000)
+    assert full >= 2 * 192 * 5000 * 4
+    assert q(2, 48, 192, 192, 5000, 1) == 0
+    assert q(2, 48, 192, 192, 5000, 0) == full
+    assert q(2, 48, 192, 4096, 50000, 1) == lib.uttt_update_stage1_workspace_bytes(2, 192, 50000)
+    prev = hook(2)
+    try:
+        assert q(2, 48, 192, 192, 5000, 1) == full
+    finally:
+        hook(prev)
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="library not built")
 def test_wgrad_partials_fit_the_backward():
     """The partials of chunked weight gradients take at most 12 B N I bytes, the
     dead intermediates in which the UPDATE backward keeps them (a query that

@@ -81,6 +81,21 @@ def test_narrow_update_equals_general_tiles(name, lr_dtype):
         assert bool(((a - b).abs() <= ulp * b.abs() + I * 2.0 ** -23 * scale).all())
 
 
+def test_one_launch_stage1_allocates_its_outputs_alone():
+    """No fp32 DH [B, N, I] beside them: the peak over the call is the outputs
+    (and what the allocator rounds up, under 2 MiB for each of four tensors)."""
+    B, E, I, D, N = 1, 4, 512, 512, 32768
+    rnd = lambda *s: torch.randn(*s, device=DEV).to(torch.bfloat16)
+    gs = torch.full((B, E), N // E, dtype=torch.int32, device=DEV)
+    args = (rnd(B, E, 2 * I, D), rnd(B, E, D, I), rnd(B, N, D), rnd(B, N, D), None, None, None, gs)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    outs = G.update_stage1(*args, True)
+    peak = torch.cuda.max_memory_allocated() - before
+    assert peak < B * N * 3 * I * 2 + 4 * (2 << 20), (peak, [tuple(o.shape) for o in outs])
+
+
 @contextlib.contextmanager
 def general_tiles():
     """The 256-token tiles: a forced wave layout takes every product there."""

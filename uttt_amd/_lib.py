@@ -74,6 +74,7 @@ SIGNATURES = {
         c_int, [c_p, c_p, c_p, c_int, c_int, c_int, c_int, c_int, c_p, c_p],
     ),
     "uttt_update_stage1_workspace_bytes": (c_sz, [c_int, c_int, c_int]),
+    "uttt_update_stage1_scratch_bytes": (c_sz, [c_int] * 6),
     "uttt_grouped_update_stage1": (
         c_int,
         [c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_int, c_p, c_int, c_int, c_int, c_int, c_int,

@@ -1983,6 +1983,19 @@ extern "C" size_t uttt_update_stage1_workspace_bytes(int B, int I, int N) {
   return up256((size_t)B * N * I * sizeof(float));
 }
 
+namespace {
+bool stage1_one_launch(int B, int E, int I, int D, int N, int token_major) {
+  return token_major && narrow_stage1(I, D, N, B, E) && !general_forced();
+}
+}  // namespace
+
+extern "C" size_t uttt_update_stage1_scratch_bytes(int B, int E, int I, int D, int N,
+                                                   int token_major) {
+  return stage1_one_launch(B, E, I, D, N, token_major)
+             ? 0
+             : uttt_update_stage1_workspace_bytes(B, I, N);
+}
+
 extern "C" int uttt_grouped_update_stage1(const void* w0_w2, const void* w1, const void* k,
                                           const void* v, const void* lr0, const void* lr1,
                                           const void* lr2, int lr_dtype,
@@ -1994,7 +2007,9 @@ extern "C" int uttt_grouped_update_stage1(const void* w0_w2, const void* w1, con
   UTTT_REQUIRE(I % 8 == 0 && D % 8 == 0,
                "grouped_update_stage1: I=%d and D=%d must be multiples of 8", I, D);
   if (B == 0 || N == 0 || I == 0) return UTTT_OK;
-  UTTT_REQUIRE(w0_w2 && w1 && k && v && group_sizes && dy0_dy2 && hidden && workspace,
+  const size_t need = uttt_update_stage1_scratch_bytes(B, E, I, D, N, token_major);
+  UTTT_REQUIRE(w0_w2 && w1 && k && v && group_sizes && dy0_dy2 && hidden &&
+                   (need == 0 || workspace),
                "grouped_update_stage1: null pointer");
   UTTT_REQUIRE((lr0 == nullptr) == (lr1 == nullptr) && (lr1 == nullptr) == (lr2 == nullptr),
                "grouped_update_stage1: pass all three lr vectors or none");
@@ -2004,11 +2019,10 @@ extern "C" int uttt_grouped_update_stage1(const void* w0_w2, const void* w1, con
                    aligned16(dy0_dy2) && aligned16(hidden) && aligned16(workspace) &&
                    (y0_y2_save == nullptr || (aligned16(y0_y2_save) && aligned16(dh_save))),
                "grouped_update_stage1: tensors must be 16-byte aligned");
-  const size_t need = uttt_update_stage1_workspace_bytes(B, I, N);
   UTTT_REQUIRE(workspace_bytes >= need, "grouped_update_stage1: workspace %zu < %zu bytes",
                workspace_bytes, need);
   hipStream_t st = as_stream(stream);
-  if (token_major && narrow_stage1(I, D, N, B, E) && !general_forced())
+  if (stage1_one_launch(B, E, I, D, N, token_major))
     return launch_narrow_stage1(w0_w2, w1, k, v, lr0, lr1, lr2, lr_dtype, group_sizes, B, E, I, D, N,
                                 dy0_dy2, hidden, y0_y2_save, dh_save, st,
                                 "grouped_update_stage1");

@@ -193,7 +193,7 @@ def _update_stage1(W0_W2: Tensor, W1: Tensor, K: Tensor, V: Tensor, lr0: Optiona
     else:
         Ys = torch.empty((0,), dtype=torch.bfloat16, device=dev)
         DHs = torch.empty((0,), dtype=torch.bfloat16, device=dev)
-    ws_bytes = L.lib().uttt_update_stage1_workspace_bytes(B, I, N)
+    ws_bytes = L.lib().uttt_update_stage1_scratch_bytes(B, E, I, D, N, int(token_major))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     L.call("uttt_grouped_update_stage1", L.ptr(W0_W2), L.ptr(W1), L.ptr(K), L.ptr(V),
            L.ptr(lrs[0]), L.ptr(lrs[1]), L.ptr(lrs[2]), lr_code, L.ptr(gs),
