@@ -661,7 +661,7 @@ int uttt_dense_gather_heads(const void* const* k_layers, const void* const* v_la
  * it out.  The weight gradients split K once per layer (L runs; fp32
  * partials in the workspace, uttt_dense_wgrad_pair_layers_workspace_bytes,
  * summed in layer order), so they are bit-identical to the gathered path
- * wherever its split count is L (configs[1]: 12 layers, 12 runs).  dy, hid
+ * wherever its split count is L (dense 124M: 12 layers, 12 runs).  dy, hid
  * as uttt_dense_update_stage1's outputs [b*H, L*l, 2I] / [b*H, L*l, I].
  * l must be a multiple of 64 (of 32 for stage 1), L <= 64, pointer arrays
  * on the host, every tensor 16-byte aligned.  No reference counterpart: the

@@ -43,7 +43,7 @@ def _run(path, W02, W1, X, gs, B, E, I, D, N):
 
 
 @pytest.mark.parametrize("B,E,I,D,N,empty", [
-    (1, 32, 3072, 1536, 4096, (5, 9)),    # the configs[4] chunk shape
+    (1, 32, 3072, 1536, 4096, (5, 9)),    # the 760M MoE chunk shape
     (2, 8, 384, 200, 700, (3,)),          # K tails (200, 384 % 64 = 0 / 200 % 64 = 8)
     (1, 70, 136, 96, 900, (1, 68)),       # > 64 experts, partial row tiles
     (1, 4, 256, 128, 1500, ()),           # many tokens per expert (4 token tiles each)
@@ -67,8 +67,8 @@ def test_apply_paths_identical(B, E, I, D, N, empty):
 
 
 @pytest.mark.parametrize("B,E,I,D,T,k,empty", [
-    (1, 32, 3072, 1536, 2048, 2, (5, 9)),   # the configs[4] routed read
-    (1, 16, 1536, 768, 2048, 2, ()),        # the configs[3] routed read
+    (1, 32, 3072, 1536, 2048, 2, (5, 9)),   # the 760M MoE routed read
+    (1, 16, 1536, 768, 2048, 2, ()),        # the 124M MoE routed read
     (2, 8, 384, 200, 350, 2, (3,)),         # K tails, two batches
     (1, 70, 136, 96, 300, 3, (1, 68)),      # > 64 experts, partial row tiles
 ])

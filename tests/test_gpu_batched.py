@@ -1,4 +1,4 @@
-"""GPU parity at the shapes bench.py times for configs[4] (uTTT-MoE 760M:
+"""GPU parity at the shapes bench.py times for the 760M MoE pool (uTTT-MoE 760M:
 E=32, top-2, D=1536, I=3072, Zipf(1.1) routing prior), against the oracle.
 
 The UPDATE runs through the product API, uttt_amd.moe.aggregate_moe_update_grads:

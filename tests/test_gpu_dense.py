@@ -1,6 +1,6 @@
 """GPU parity of the uTTT-Dense path (uttt_amd.dense) against oracle/dense.py
-on the same seeded inputs at the configs[0] head shape (H = 4, d = 96,
-d_h = 192, chunks of 512) and the configs[1] shape (d = 192, d_h = 384).
+on the same seeded inputs at the small dense head (H = 4, d = 96,
+d_h = 192, chunks of 512) and the dense 124M one (d = 192, d_h = 384).
 
 Bar: bf16 outputs and weights within rtol 2e-2 (tests.helpers.assert_bf16_close)
 of the oracle run with the reference's bf16 storage points; raw updates
@@ -64,7 +64,7 @@ def test_dense_read_few_tokens(H, d, r, l):
 
 
 @pytest.mark.parametrize("L,S,chunk,H,d,r,master_renorm", [
-    (1, 4096, 512, 4, 96, 2, False),     # configs[0]: one layer, 8 chunks
+    (1, 4096, 512, 4, 96, 2, False),     # the small dense layer: one layer, 8 chunks
     (3, 1536, 512, 4, 96, 2, True),      # aggregate over layers, master renorm
 ])
 def test_dense_sweep(L, S, chunk, H, d, r, master_renorm):
@@ -151,8 +151,8 @@ def test_fused_dense_read(b, H, d, dh, l):
 
 
 @pytest.mark.parametrize("b,H,d,dh,l", [
-    (1, 4, 96, 192, 512),     # configs[0]
-    (1, 4, 192, 384, 2048),   # configs[1]
+    (1, 4, 96, 192, 512),     # the small dense layer
+    (1, 4, 192, 384, 2048),   # dense 124M
     (2, 3, 128, 96, 77),
     (1, 2, 256, 512, 64),
     (3, 1, 64, 32, 9),
@@ -191,8 +191,8 @@ def test_packed_dense_read_is_bit_identical(b, H, d, dh, l):
 
 
 @pytest.mark.parametrize("BH,N,d,dh,with_lr", [
-    (4, 3000, 192, 384, True),   # configs[1] head, ragged token tiles
-    (4, 1024, 96, 192, True),    # configs[0] head
+    (4, 3000, 192, 384, True),   # a dense 124M head, ragged token tiles
+    (4, 1024, 96, 192, True),    # the small dense head
     (2, 77, 128, 96, True),      # one partial tile
     (3, 128, 64, 32, False),     # one hidden block, lr = 1
     (1, 513, 256, 512, True),    # the largest head
@@ -222,7 +222,7 @@ def test_fused_dense_update_stage1(BH, N, d, dh, with_lr):
     assert_bf16_close(dy.cpu(), ref_dy.cpu(), name="DY0_DY2")
     assert_bf16_close(hl.cpu(), ref_hl.cpu(), name="Hid")
     # same products in the same k order on the same MFMA, same epilogue: the
-    # two routes agree bit for bit (measured at the configs[0] and [1] heads)
+    # two routes agree bit for bit (measured at heads of 96 and 192)
     if (d, dh) in ((192, 384), (96, 192)):
         assert torch.equal(dy.view(torch.int16), ref_dy.view(torch.int16))
         assert torch.equal(hl.view(torch.int16), ref_hl.view(torch.int16))
@@ -233,8 +233,8 @@ def test_fused_dense_update_stage1(BH, N, d, dh, with_lr):
 
 
 @pytest.mark.parametrize("BH,N,d,dh", [
-    (4, 3000, 192, 384),   # configs[1] head, ragged token tiles
-    (4, 1024, 96, 192),    # configs[0] head
+    (4, 3000, 192, 384),   # a dense 124M head, ragged token tiles
+    (4, 1024, 96, 192),    # the small dense head
     (2, 77, 128, 96),      # one partial tile, odd block count (3 blocks: a lone last block)
     (3, 128, 64, 32),      # one hidden block
 ])
@@ -323,9 +323,9 @@ def test_bank_owns_its_weights():
 
 
 @pytest.mark.parametrize("b,H,d,r,L,l,lr_kind", [
-    (1, 4, 192, 2, 12, 2048, "shared_f32"),   # the configs[1] write: 12 layers, 12 K runs
+    (1, 4, 192, 2, 12, 2048, "shared_f32"),   # the dense 124M write: 12 layers, 12 K runs
     (2, 2, 64, 2, 3, 512, "per_head_bf16"),
-    (1, 4, 96, 2, 1, 512, "none"),            # one layer (configs[0]'s shape)
+    (1, 4, 96, 2, 1, 512, "none"),            # one layer (the small dense layer)
 ])
 def test_layered_update_equals_gathered_heads(b, H, d, r, L, l, lr_kind):
     """The aggregate write's UPDATE read from every layer's own k, v, lr

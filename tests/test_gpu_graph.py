@@ -17,7 +17,7 @@ DEV = "cuda"
 
 CASES = [
     # T, E, D, I, topk
-    (2048, 16, 768, 1536, 2),   # the configs[3] chunk
+    (2048, 16, 768, 1536, 2),   # the 124M MoE chunk
     (300, 8, 256, 512, 3),
 ]
 

@@ -4,7 +4,7 @@ seeded bf16 inputs.
 
 Bar: rtol 2e-2 in bf16 (tests.helpers.assert_bf16_close: |ours - ref| <=
 2e-2*|ref| + 2e-2*rms(ref)), compared on the token columns / experts the
-reference writes.  At the 760M shape the oracle is too slow on
+reference writes.  At the 760M MoE shape the oracle is too slow on
 the CPU, so those outputs are checked expert by expert against torch fp32
 matmuls of the same bf16 operands on the GPU.
 """
@@ -46,8 +46,8 @@ def routed_sizes(T, E, k, seed, zipf=None):
 CASES = {
     "ragged": (1, 4, 64, 96, [[37, 0, 130, 5]], None),
     "slack": (2, 3, 128, 256, [[300, 1, 64], [0, 0, 365]], 400),   # unwritten tail columns
-    "one_expert": (1, 1, 96, 192, [[517]], None),                 # dense (E=1) shape of configs[0]
-    "c3_chunk": (1, 16, 768, 1536, None, None),                   # configs[3], one chunk
+    "one_expert": (1, 1, 96, 192, [[517]], None),                 # dense (E=1), the small head
+    "c3_chunk": (1, 16, 768, 1536, None, None),                   # 124M MoE, one chunk
 }
 
 
@@ -219,7 +219,7 @@ def _expert_fp32(c, b, e):
 
 @pytest.mark.parametrize("zipf", [None, 1.1])
 def test_760m_shape_against_torch_fp32(zipf):
-    """configs[4] chunk: E=32, top-2, D=1536, I=3072, N=4096 (Zipf(1.1) prior)."""
+    """760M MoE chunk: E=32, top-2, D=1536, I=3072, N=4096 (Zipf(1.1) prior)."""
     gs = routed_sizes(2048, 32, 2, seed=1, zipf=zipf)
     c = make_case(1, 32, 1536, 3072, gs, seed=1)
     W02, W1, K, V, gsd = dev(c, "W02", "W1", "K", "V", "gs")

@@ -101,7 +101,7 @@ def test_prenorm_lact_loop_matches_oracle(kv_repeat, use_muon, with_mom):
     # amplifies bf16-level differences along small singular directions: the
     # trajectories of two correct roundings part after a few writes, so the
     # Muon cases check one write (two chunks) stage by stage
-    b, dh, d, c = 2, 192, 96, 256                  # the configs[0] head shape
+    b, dh, d, c = 2, 192, 96, 256                  # the small dense head
     seq = 2 * c if use_muon else 1024
     w0, w1, w2, q, k, v, lrs, mom = _case(b=b, dh=dh, d=d, seq=seq, kv_repeat=kv_repeat,
                                           seed=kv_repeat + 2 * use_muon + 4 * with_mom)

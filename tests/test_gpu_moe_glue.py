@@ -2,7 +2,7 @@
 oracle's compositions:
   - the routed prefill read (route -> row map -> permute -> grouped APPLY ->
     gate-weighted unpermute, modeling_recurrent_lact.py:296-349) at the
-    configs[4] chunk (T = 2048, E = 32, D = 1536, I = 3072) and with four
+    760M MoE chunk (T = 2048, E = 32, D = 1536, I = 3072) and with four
     fast-weight heads, against oracle/moe_read.apply_moe_grouped on the
     router's own mask and gates;
   - one writer's gradients (M:453-518) and the aggregate of several writers
@@ -116,7 +116,7 @@ def test_read_query_path():
 
 
 @pytest.mark.parametrize("T,E,D,I,heads,topk,combine", [
-    (2048, 32, 1536, 3072, 1, 2, "topk_renorm"),   # the configs[4] chunk read
+    (2048, 32, 1536, 3072, 1, 2, "topk_renorm"),   # the 760M MoE chunk read
     (256, 16, 4 * 96, 192, 4, 2, "selected_prob"),  # four fast-weight heads
 ])
 def test_routed_read_matches_oracle(T, E, D, I, heads, topk, combine):
@@ -242,8 +242,8 @@ def test_compiled_read_and_update_equal_eager():
 def test_routed_read_without_gradient_equals_the_permuted_path():
     """The routed read under no_grad reads its token rows through the inverse
     row map (no permuted copy); with a gradient to track it permutes as the
-    reference does.  Both give the same output bit for bit (configs[3] and
-    configs[4] chunks)."""
+    reference does.  Both give the same output bit for bit (124M MoE and
+    760M MoE chunks)."""
     for E, D, I in ((16, 768, 1536), (32, 1536, 3072)):
         g = torch.Generator(device=DEV).manual_seed(E)
         W02 = (torch.randn(1, E, 2 * I, D, generator=g, device=DEV) * D ** -0.5).to(torch.bfloat16)

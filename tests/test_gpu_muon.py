@@ -87,7 +87,7 @@ def _ns5_kernels(run):
 @pytest.mark.parametrize("n,R,C,dtype,scale", [
     (16, 192, 192, torch.float32, 1.0),    # the uTTT-Dense 124M w0 / w2 slices
     (8, 192, 192, torch.bfloat16, 0.5),
-    (4, 96, 96, torch.float32, 1.0),       # configs[0]'s d = 96 slices
+    (4, 96, 96, torch.float32, 1.0),       # slices of d = 96
     (3, 64, 128, torch.float32, 1.0),      # wide
     (3, 192, 96, torch.float32, 0.7),      # tall: X = G^T
     (2, 32, 192, torch.bfloat16, 1.0),     # one row block

@@ -61,7 +61,7 @@ def test_moe_write_matches_oracle(B, E, I, D, grad_dtype, mom):
 
 @pytest.mark.parametrize("master_renorm,mom", [(False, False), (True, False), (False, True)])
 def test_dense_write_matches_oracle(master_renorm, mom):
-    b, h, d, r = 1, 4, 96, 2   # configs[0] head shape: d = 96, d_h = 192
+    b, h, d, r = 1, 4, 96, 2   # the small dense head: d = 96, d_h = 192
     shapes = [(b, h, r * d, d), (b, h, d, r * d), (b, h, r * d, d)]
     masters = [_rand(s, i) / d ** 0.5 for i, s in enumerate(shapes)]
     # fast weights 3-6% off their masters, row by row: a write that took the

@@ -400,8 +400,8 @@ void launch_update_s1(int BH, int N, int I, hipStream_t st, const uint16_t* k, c
                       const float* a, const float* b, const float* c, const uint16_t* p,
                       uint16_t* o, uint16_t* h, const S1Layers& ly = S1Layers{}) {
   const dim3 grid((unsigned)((N + kUpdTok - 1) / kUpdTok), (unsigned)BH);
-  // the staged kernel where the grid fills the chip (configs[1]'s write:
-  // 768 workgroups, 100 -> 89 us); on small grids (configs[0]: 16) its
+  // the staged kernel where the grid fills the chip (the dense 124M write:
+  // 768 workgroups, 100 -> 89 us); on small grids (the small dense layer: 16) its
   // per-pair load wait and barrier cost more than the shared loads save
   // (50.5 -> 56.7 us), and the four-wave kernel with register prefetch runs
   if constexpr (D <= 192) {

@@ -1593,8 +1593,8 @@ bool g_apply_down_two = false;  // down products on 256-row tiles (default 128: 
 constexpr int kCUs = 256;       // MI355X compute units
 
 // Gate/up (256-row weight tiles either way): the skinny 128-token tiles when
-// the experts average at most 256 routed rows (configs[3]: 129 -> 100 us per
-// apply with the down projection below; configs[4] gate/up 188 -> 184 us).
+// the experts average at most 256 routed rows (124M MoE: 129 -> 100 us per
+// apply with the down projection below; 760M MoE gate/up 188 -> 184 us).
 bool use_apply_kernel(int64_t N, int E) {
   return g_apply_path == 1 || g_apply_path == 2 ||
          (g_apply_path < 0 && N <= (int64_t)kBRows * E);
@@ -1608,7 +1608,7 @@ bool use_narrow_gate_up(int I, int D) {
 // The down projection (and every uttt_grouped_gemm_nt): the skinny tiles
 // (128 weight rows x 128 tokens) when the general 256x256 tiles would not
 // fill the chip once even at their upper-bound count, else the general tiles.
-// configs[3] (3 x 32 tiles of 256): 38.9 -> 21.5 us; configs[4] (6 x 48):
+// 124M MoE (3 x 32 tiles of 256): 38.9 -> 21.5 us; 760M MoE (6 x 48):
 // the general tiles, 101 us against 110 us on the skinny ones.
 bool use_apply_kernel_nt(int64_t N, int E, int B, int M) {
   if (g_apply_path >= 0) return g_apply_path > 0;

@@ -22,9 +22,9 @@ namespace uttt {
 // Sides of 256 and 512 pad by up to 1.9 times (8 experts of 512 x 256 over
 // 196 608 tokens 196 / 374 us).  One expert per batch (uTTT-Dense heads): the
 // split-K 256 tiles measure the same or faster (4 x [192 x 384] over 98 304
-// tokens 79 / 90 us).  Still up to 1.3 times slower: 8 to 32 experts with long
-// segments of one length (32 of 384 x 192 over 98 304: 83 / 109 us), where
-// unequal ones are up to twice faster.
+// tokens 79 / 90 us).  Still up to 1.3 times slower: 8 to 32 experts, or 16 batches
+// of 4, with long segments of one length (32 of 384 x 192 over 98 304: 83 / 109 us),
+// where unequal ones are up to twice faster.
 // Chunk length: about 256 (chunk, tile) workgroups on an even routing, 512 to
 // 4096 tokens (4096 with a side above 512), at least 2 D: a batch's partials then
 // fit in the backward's dead intermediates, 12 N I bytes.
